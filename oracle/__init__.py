@@ -50,7 +50,7 @@ def build(force: bool = False, ref: bool = True) -> None:
     """Compile the checkers with oracle/Makefile (the reference library only
     when its sources are present)."""
     targets = ["all"]
-    if ref and os.path.isdir(REF_SRC):
+    if ref and os.path.exists(os.path.join(REF_SRC, "core", "src", "core.cpp")):
         targets.append("ref")
     cmd = ["make", "-s", "-C", HERE] + (["-B"] if force else []) + targets
     subprocess.run(cmd, check=True)
