@@ -20,7 +20,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libfluid_hip.so")
-SOURCES = ["pbf_kernels.hip", "pbf_tiles.hip", "pbf_adjoint.hip", "pbf_capi.hip"]
+SOURCES = ["pbf_kernels.hip", "pbf_gather.hip", "pbf_tiles.hip", "pbf_adjoint.hip", "pbf_capi.hip"]
 ARCH = os.environ.get("FLUID_HIP_ARCH", "gfx950")
 
 HIPCC_FLAGS = [

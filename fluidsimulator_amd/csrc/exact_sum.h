@@ -111,6 +111,7 @@ constexpr int kAddInPlace = 64;
 // add_repeat for hot loops, with the in-place cut-over.
 __host__ __device__ inline float add_k(float x, float w, int k) {
   if (k <= kAddInPlace) {
+#pragma unroll 4
     for (int i = 0; i < k; ++i) x += w;
     return x;
   }

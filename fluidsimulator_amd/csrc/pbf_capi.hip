@@ -189,11 +189,8 @@ void compute_consts_of(Ctx& c, const fluid_hip_params* params, int n_scenes) {
   k.vort_norm_eps = p.vort_norm_eps;
   k.record_diag = c.record_diag ? 1 : 0;
   k.xcd_remap = c.xcd_remap;
-  k.coop = c.wave_mode >= 2 ? 1 : 0;
-  k.coop_bulk = c.wave_mode == 2 ? 1 : 0;
   k.runs = (c.wave_mode == 2 && !c.record_diag) ? 1 : 0;
-  k.full_lists = c.record_diag ? 1 : 0;
-  k.count_only = 0;
+  k.full_lists = (c.record_diag || c.wave_mode == 1) ? 1 : 0;
   // tile mode 0 (default) tiles from kTileAutoMinParticles particles: below
   // that a substep is bound by launches, to which the tile kernels add
   const bool tile_mode = c.tile_gather == 1 || (c.tile_gather == 0 && c.n >= fluidhip::kTileAutoMinParticles);
@@ -270,12 +267,11 @@ void free_all(Ctx& c) {
   for (int** p : {&c.key, &c.sort_k[0], &c.sort_k[1], &c.sort_v[0], &c.sort_v[1],
                   &c.radix_hist, &c.radix_off, &c.radix_len, &c.count, &c.start, &c.bbox,
                   &c.total_cells, &c.scan_partial, &c.slot_key, &c.nbr, &c.seg, &c.nwords,
-                  &c.ncount, &c.tile_bbox, &c.run_no, &c.run_excl, &c.rep_list, &c.run_end,
-                  &c.n_dev, &c.cell_no, &c.cell_excl, &c.cell_first, &c.lanes1, &c.lanes2,
-                  &c.off1, &c.off2,
-                  &c.lane_rep, &c.lane_info,
+                  &c.ncount, &c.tile_bbox, &c.run_no, &c.rep_list, &c.info,
                   &c.steps_started})
     dfree(*p);
+  dfree(c.units);
+  dfree(c.dense);
   dfree(c.slot_cell);
   dfree(c.grid);
   dfree(c.in_tile);
@@ -682,23 +678,13 @@ bool noalloc_layout(Ctx& c, unsigned char* base, size_t bytes) {
   take(c.bbox, 6);
   take(c.tile_bbox, 6 * (n / 64 + 1));
   take(c.run_no, n);
-  take(c.run_excl, n + 1);
-  take(c.rep_list, n);
-  take(c.run_end, n);
-  take(c.cell_no, n);
-  take(c.cell_excl, n + 1);
-  take(c.cell_first, n + 1);
-  take(c.lanes1, n + 1);
-  take(c.lanes2, n + 1);
-  take(c.off1, n + 1);
-  take(c.off2, n + 1);
-  c.lane_cap = 3ll * c.n + 64;
-  take(c.lane_rep, static_cast<size_t>(c.lane_cap));
-  take(c.lane_info, 3);
-  take(c.n_dev, 1);
+  take(c.rep_list, n + 1);
+  take(c.units, n);
+  take(c.dense, n);
+  take(c.info, 4);
   take(c.grid, 1);
   take(c.total_cells, 1);
-  take(c.scan_partial, 2 * static_cast<size_t>(c.scan_blocks) + 2);
+  take(c.scan_partial, 3 * static_cast<size_t>(c.scan_blocks) + 2);
   take(c.nbr_total, 1);
   take(c.need_cells, 1);
   take(c.pair_total, 1);
@@ -735,13 +721,12 @@ bool noalloc_layout(Ctx& c, unsigned char* base, size_t bytes) {
 // flags and bounding box, and the cell histogram (kernel stores, so the
 // sequence holds no memset node if a caller captures it).
 __global__ void k_noalloc_init(int n, int radix_len, fluidhip::ScenePlanes sp, int* seg,
-                               fluidhip::ScenePlanes* planes, int* n_dev, int* rlen, int* bbox,
+                               fluidhip::ScenePlanes* planes, int* rlen, int* bbox,
                                unsigned* flags, int* steps_started) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     seg[0] = 0;
     seg[1] = n;
     *planes = sp;
-    *n_dev = n;
     *rlen = radix_len;
     bbox[0] = bbox[1] = bbox[2] = INT_MAX;
     bbox[3] = bbox[4] = bbox[5] = INT_MIN;
@@ -879,27 +864,16 @@ int fluid_hip_create(fluid_hip_ctx** out, int32_t n_scenes, const int64_t* scene
   ALLOC(c.bbox, 6 * static_cast<size_t>(n_scenes));
   ALLOC(c.tile_bbox, 6 * (n / 64 + 1));
   ALLOC(c.run_no, n);
-  ALLOC(c.run_excl, static_cast<size_t>(n) + 1);
-  ALLOC(c.rep_list, n);
-  ALLOC(c.run_end, n);
-  ALLOC(c.cell_no, n);
-  ALLOC(c.cell_excl, static_cast<size_t>(n) + 1);
-  ALLOC(c.cell_first, static_cast<size_t>(n) + 1);
-  ALLOC(c.lanes1, static_cast<size_t>(n) + 1);
-  ALLOC(c.lanes2, static_cast<size_t>(n) + 1);
-  ALLOC(c.off1, static_cast<size_t>(n) + 1);
-  ALLOC(c.off2, static_cast<size_t>(n) + 1);
-  // every dense cell (>= 32 slots) pads its runs by at most 63 lanes
-  // (n lanes always hold the packed layout; more than 3n + 64 is never used)
+  ALLOC(c.rep_list, n + 1);
+  ALLOC(c.units, n);
+  ALLOC(c.dense, n);
+  ALLOC(c.info, 4);
   c.lane_cap = 3ll * n + 64;
   if (cfg.lane_capacity > 0)
     c.lane_cap = std::min<long long>(c.lane_cap, std::max<long long>(cfg.lane_capacity, n));
-  ALLOC(c.lane_rep, static_cast<size_t>(c.lane_cap));
-  ALLOC(c.lane_info, 3);
-  ALLOC(c.n_dev, 1);
   ALLOC(c.grid, static_cast<size_t>(n_scenes));
   ALLOC(c.total_cells, 1);
-  ALLOC(c.scan_partial, 2 * static_cast<size_t>(c.scan_blocks) + 2);
+  ALLOC(c.scan_partial, 3 * static_cast<size_t>(c.scan_blocks) + 2);
   ALLOC(c.nbr_total, 1);
   ALLOC(c.need_cells, 1);
   ALLOC(c.pair_total, 1);
@@ -921,8 +895,6 @@ int fluid_hip_create(fluid_hip_ctx** out, int32_t n_scenes, const int64_t* scene
   ALLOC(c.tile_list, static_cast<size_t>(c.tile_list_cap / 8) * n);
   ALLOC(c.tile_cnt, n);
 #undef ALLOC
-  e = hipMemcpy(c.n_dev, &c.n, sizeof(int), hipMemcpyHostToDevice);
-  if (e != hipSuccess) return bail(hip_fail(e, "hipMemcpy(particle count)"));
   {
     const int len = 256 * c.radix_blocks;
     e = hipMemcpy(c.radix_len, &len, sizeof(int), hipMemcpyHostToDevice);
@@ -1178,8 +1150,8 @@ int fluid_hip_get_diag(fluid_hip_ctx* ctx, int32_t* cell, int32_t* sorted_ids,
   }
   if (nbr_count) {
     if (c.lists_partial) {
-      // particles of dense cells and non-head slots of runs kept no count:
-      // a counting walk of the last grid writes every slot's
+      // dense heads and the other slots of runs kept no count: a counting
+      // walk of the last grid writes every slot's
       HIP_TRY(fluidhip::enqueue_count_pairs(c), "count pairs");
       HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
     }
@@ -1190,20 +1162,7 @@ int fluid_hip_get_diag(fluid_hip_ctx* ctx, int32_t* cell, int32_t* sorted_ids,
   if (rho) {
     std::vector<float> r(n);
     HIP_TRY(hipMemcpy(r.data(), c.rho, sizeof(float) * n, hipMemcpyDeviceToHost), "read rho");
-    // with runs only each run's first slot wrote rho; the others equal it
-    std::vector<int> run_no, rep;
-    if (c.last_runs) {
-      run_no.resize(n);
-      rep.resize(n);
-      HIP_TRY(hipMemcpy(run_no.data(), c.run_no, sizeof(int) * n, hipMemcpyDeviceToHost),
-              "read runs");
-      HIP_TRY(hipMemcpy(rep.data(), c.rep_list, sizeof(int) * n, hipMemcpyDeviceToHost),
-              "read runs");
-    }
-    for (size_t s = 0; s < n; ++s) {
-      const size_t src = c.last_runs ? static_cast<size_t>(rep[run_no[s]]) : s;
-      rho[ids[s]] = c.iterations > 0 ? r[src] : 0.0f;
-    }
+    for (size_t s = 0; s < n; ++s) rho[ids[s]] = c.iterations > 0 ? r[s] : 0.0f;
   }
   if (lambda) {
     if (c.iterations > 0) {
@@ -1229,42 +1188,70 @@ int fluid_hip_get_neighbors(fluid_hip_ctx* ctx, int32_t* out, int64_t cap, int64
   std::vector<long long> off(n);
   std::vector<int> nw(n);
   HIP_TRY(hipMemcpy(pos.data(), c.posA, sizeof(float4) * n, hipMemcpyDeviceToHost), "read pos");
-  HIP_TRY(hipMemcpy(off.data(), c.noff, sizeof(long long) * n, hipMemcpyDeviceToHost), "read offsets");
   HIP_TRY(hipMemcpy(nw.data(), c.nwords, sizeof(int) * n, hipMemcpyDeviceToHost), "read lengths");
-  // particles of LDS tiles keep a candidate mask instead of a list: decode it
-  // with the tile's halo layout (the candidates are the 27 cells in (dz, dy,
-  // dx) order, 9 contiguous runs of three cells of the halo, as in
-  // pbf_tiles.hip)
+  // particles of LDS tiles keep LDS records of the tile's halo: decode them
+  // with its layout; list heads keep slots in their row, and a step that
+  // stores no words leaves lists too long for a row to this call
   const bool tiled = c.consts.tiles && c.last_runs && c.in_tile != nullptr;
-  std::vector<int> in_tile, tseg, tsrc, tcnt;
+  std::vector<int> in_tile, tseg, tsrc, tcnt, ncnt;
   std::vector<uint16_t> tlist;
   if (tiled) {
     in_tile.resize(n);
     HIP_TRY(hipMemcpy(in_tile.data(), c.in_tile, sizeof(int) * n, hipMemcpyDeviceToHost),
             "read tiles");
   }
-  bool any_tile = false;
+  bool any_tile = false, any_row = false, any_long = false;
   for (size_t s = 0; s < n; ++s) {
     if (nw[s] >= 0) continue;
-    if (!tiled || in_tile[s] <= 0)
+    if (nw[s] == fluidhip::kRowList)
+      any_row = true;
+    else if (nw[s] == fluidhip::kLongList)
+      any_long = true;
+    else if (tiled && in_tile[s] > 0)
+      any_tile = true;
+    else
       return fail(FLUID_HIP_ESTATE,
                   "the last step stored no list for some particles; create the context "
                   "with record_diag for complete lists");
-    any_tile = true;
+  }
+  if (any_long) {
+    // the words buffer holds nothing else then
+    for (int attempt = 0; attempt < 2; ++attempt) {
+      HIP_TRY(fluidhip::enqueue_long_lists(c), "long lists");
+      unsigned long long need = 0;
+      HIP_TRY(hipMemcpyAsync(&need, c.nbr_total, sizeof(need), hipMemcpyDeviceToHost, c.stream),
+              "read total");
+      HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+      if (need <= static_cast<unsigned long long>(c.nbr_cap)) break;
+      drop_graph(c);
+      if ((rc = alloc_neighbors(c, static_cast<long long>(need)))) return rc;
+      HIP_TRY(hipMemcpy(c.nwords, nw.data(), sizeof(int) * n, hipMemcpyHostToDevice),
+              "restore lengths");
+    }
+    HIP_TRY(hipMemcpy(nw.data(), c.nwords, sizeof(int) * n, hipMemcpyDeviceToHost),
+            "read lengths");
+  }
+  HIP_TRY(hipMemcpy(off.data(), c.noff, sizeof(long long) * n, hipMemcpyDeviceToHost), "read offsets");
+  if (any_tile || any_row) {
+    tlist.resize(static_cast<size_t>(c.tile_list_cap) * n);
+    HIP_TRY(hipMemcpy(tlist.data(), c.tile_list, sizeof(uint16_t) * tlist.size(),
+                      hipMemcpyDeviceToHost),
+            "read lists");
+  }
+  if (any_row) {
+    ncnt.resize(n);
+    HIP_TRY(hipMemcpy(ncnt.data(), c.ncount, sizeof(int) * n, hipMemcpyDeviceToHost),
+            "read counts");
   }
   if (any_tile) {
     const size_t cap = static_cast<size_t>(c.tile_cap);
     tseg.resize(cap * 217);
     tsrc.resize(cap * 216);
-    tlist.resize(static_cast<size_t>(c.tile_list_cap) * n);
     tcnt.resize(n);
     HIP_TRY(hipMemcpy(tseg.data(), c.tile_seg, sizeof(int) * tseg.size(), hipMemcpyDeviceToHost),
             "read tiles");
     HIP_TRY(hipMemcpy(tsrc.data(), c.tile_src, sizeof(int) * tsrc.size(), hipMemcpyDeviceToHost),
             "read tiles");
-    HIP_TRY(hipMemcpy(tlist.data(), c.tile_list, sizeof(uint16_t) * tlist.size(),
-                      hipMemcpyDeviceToHost),
-            "read tile lists");
     HIP_TRY(hipMemcpy(tcnt.data(), c.tile_cnt, sizeof(int) * n, hipMemcpyDeviceToHost),
             "read tile lists");
   }
@@ -1301,7 +1288,16 @@ int fluid_hip_get_neighbors(fluid_hip_ctx* ctx, int32_t* out, int64_t cap, int64
     const int s = slot_of[id];
     if (nw[s] < 0) {
       tn.clear();
-      tile_neighbors(static_cast<size_t>(s), tn);
+      if (nw[s] == fluidhip::kRowList) {
+        // chunk q of slot s: entries 4 q .. 4 q + 3, 32 bits each
+        for (int k = 0; k < ncnt[s]; ++k) {
+          int t;
+          std::memcpy(&t, &tlist[(static_cast<size_t>(k >> 2) * n + s) * 8 + 2 * (k & 3)], sizeof(t));
+          tn.push_back(t);
+        }
+      } else {
+        tile_neighbors(static_cast<size_t>(s), tn);
+      }
       for (int t : tn) {
         if (out && k < cap) out[k] = ids[t];
         ++k;
@@ -1355,7 +1351,7 @@ int fluid_hip_get_stats(fluid_hip_ctx* ctx, int64_t* out, int32_t n) {
                    c.adj ? c.adj->recomputed : 0, 0, 0};
   if (c.stepped && c.n > 0) {
     if (c.lists_partial) {
-      // cooperative particles stored no list: count their pairs again
+      // dense heads stored no list: count their pairs again
       HIP_TRY(fluidhip::enqueue_count_pairs(c), "count pairs");
       unsigned long long pairs = 0;
       HIP_TRY(hipMemcpyAsync(&pairs, c.pair_total, sizeof(pairs), hipMemcpyDeviceToHost,
@@ -1756,7 +1752,7 @@ int fluid_hip_step_noalloc(const fluid_hip_params* params, int64_t n, float* pos
     return fail(FLUID_HIP_ECAPACITY, "buffers do not fit the scratch array");
 
   k_noalloc_init<<<1, 64, 0, c.stream>>>(c.n, 256 * c.radix_blocks, scene_table(*params), c.seg,
-                                         c.planes, c.n_dev, c.radix_len, c.bbox, c.flags,
+                                         c.planes, c.radix_len, c.bbox, c.flags,
                                          c.steps_started);
   HIP_TRY(hipGetLastError(), "scratch set-up");
   k_zero_ints<<<1024, 256, 0, c.stream>>>(c.count, c.cell_cap);

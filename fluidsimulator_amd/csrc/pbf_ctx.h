@@ -47,6 +47,25 @@ struct TileArgs {
   const int* tile_cnt;     // n: neighbors of a tile particle
 };
 
+// What the gather passes over the heads (pbf_gather.hip) read besides their
+// pass's arrays.
+struct GatherView {
+  const int* info;         // runs, list heads, dense units, heads per unit (device)
+  const int4* units;       // list heads: {slot, neighbors or -1, slots of the run, scene}
+  const int2* dense;       // dense units: {first head's slot, scene | kSingle}
+  const int* run_no;       // per slot
+  const int* rep;          // per run: first slot; [runs] = n
+  const int4* rows;        // chunk q of slot s at q * n + s: neighbors 4 q .. 4 q + 3
+  int row_cap;             // neighbors of a row
+  const uint64_t* slot_cell;
+  const int* slot_key;
+  const GridDesc* grid;
+  const int* start;
+  const int* seg;
+  const float4* p0;        // predicted positions p^0 (xyz) of the lists
+  int dense_blocks;        // workgroups of a pass that take the dense units
+};
+
 struct Prof {
   struct Pending {
     const char* name;
@@ -119,27 +138,16 @@ struct Ctx {
   int* tile_bbox = nullptr;  // 6 per particle tile (workgroup)
   GridDesc* grid = nullptr;
   int* total_cells = nullptr;
-  int* scan_partial = nullptr;  // 2 scan_blocks + 2: range sums of one or two scanned arrays
+  int* scan_partial = nullptr;  // 3 scan_blocks + 2: range sums of up to three scanned arrays
   uint64_t* slot_cell = nullptr;  // packed cell of pred0 per sorted slot
   int* slot_key = nullptr;  // table key of each sorted slot's cell
-  // runs of identical consecutive slots (one lane computes each run)
-  int* run_no = nullptr;     // per slot: head flag, then the slot's run number
-  int* run_excl = nullptr;   // n + 1: exclusive scan of the head flags; [n] = runs
-  int* rep_list = nullptr;   // per run: its first slot
-  int* run_end = nullptr;    // per slot: one past the last slot of its run
-  int* n_dev = nullptr;      // the particle count, on the device (scan length)
-  // lanes of the passes: runs of sparse cells packed, then each dense cell's
-  // runs from a wave boundary (one cell per wave)
-  int* cell_no = nullptr;    // per slot: cell head flag, then the slot's non-empty cell number
-  int* cell_excl = nullptr;  // n + 1: exclusive scan of the cell head flags; [n] = cells
-  int* cell_first = nullptr; // per non-empty cell: its first slot
-  int* lanes1 = nullptr;     // per non-empty cell: packed lanes
-  int* lanes2 = nullptr;     // per non-empty cell: aligned lanes (whole waves)
-  int* off1 = nullptr;       // n + 1: exclusive scan of lanes1; [cells] = total
-  int* off2 = nullptr;       // n + 1: exclusive scan of lanes2; [cells] = total
-  int* lane_rep = nullptr;   // lane_cap: the run head slot of each lane, -1 for padding
-  int* lane_info = nullptr;  // 3: packed lanes, first aligned lane, end of aligned lanes
-  long long lane_cap = 0;    // lanes the passes launch with runs: 3n + 64
+  // runs of identical consecutive slots, and the heads the passes compute
+  int* run_no = nullptr;       // per slot: its class, then its run's number
+  int* rep_list = nullptr;     // n + 1: per run its first slot; [runs] = n
+  int4* units = nullptr;       // per list head: {slot, neighbors or -1, slots of its run, scene}
+  int2* dense = nullptr;       // groups of heads without a row: {first slot, scene | kSingle}
+  int* info = nullptr;         // 4: runs, list heads, dense units, heads per unit
+  long long lane_cap = 0;      // reported by the tuner; no layout depends on it
 
   // brick tiles (sparse bricks whose passes run through LDS)
   int* in_tile = nullptr;      // per slot: 1 + its tile's index this substep, 0 outside tiles
@@ -174,11 +182,11 @@ struct Ctx {
   bool uploaded = false;
   bool stepped = false;
   long long grow_events = 0;  // capacity growths (each replays the failed substep)
-  // the last substep stored no lists for cooperative particles (their
-  // neighbor counts need a counting walk), and its p^0 is in pred[0]
+  // the last substep stored no words of any list (counts of dense heads need
+  // a counting walk), and its p^0 is in pred[0]
   bool lists_partial = false;
-  // the last substep computed one lane per run of identical slots (the
-  // run's other slots copied its outputs; rho was written by the heads only)
+  // the last substep computed each run of identical slots once (it was not
+  // recorded and kept no diagnostics)
   bool last_runs = false;
 
   // staging for transfers
@@ -277,10 +285,32 @@ hipError_t enqueue_tape_copy(Ctx& c, SubTape& t, unsigned long long* need);
 hipError_t enqueue_upload(Ctx& c, const float* d_pos, const float* d_vel);
 hipError_t enqueue_download(Ctx& c, float* d_pos, float* d_vel);
 hipError_t enqueue_reset_flags(Ctx& c);
-// Counts the neighbor pairs of the last substep's grid (lists of
-// cooperative particles are not stored) into c.pair_total.
-hipError_t enqueue_count_pairs(Ctx& c);
 hipError_t enqueue_init_grid(Ctx& c);
+
+// Entries (slots) of a head's neighbor row: a row is the slot's part of the
+// tile lists, whose entries are 16 bits.
+inline int row_capacity(const Ctx& c) { return c.tile_list_cap / 2; }
+
+// The passes over the heads (pbf_gather.hip).
+GatherView gather_view(const Ctx& c, const float4* p0);
+hipError_t enqueue_heads(Ctx& c, const StepConsts& k);
+hipError_t enqueue_neighbors(Ctx& c, const StepConsts& k, const GatherView& gv);
+hipError_t enqueue_lambda(Ctx& c, const StepConsts& k, const GatherView& gv, float4* P, bool last,
+                          float4* sq);
+hipError_t enqueue_delta(Ctx& c, const StepConsts& k, const GatherView& gv, const float4* P,
+                         float4* Pn, bool last, bool rest, float4* vout, unsigned* pm,
+                         unsigned* rm);
+hipError_t enqueue_commit(Ctx& c, const StepConsts& k, const float4* P, bool rest, float4* vout);
+hipError_t enqueue_xsph(Ctx& c, const StepConsts& k, const GatherView& gv, bool rest,
+                        unsigned* rm);
+hipError_t enqueue_vort_omega(Ctx& c, const StepConsts& k, const GatherView& gv);
+hipError_t enqueue_vort_apply(Ctx& c, const StepConsts& k, const GatherView& gv, bool rest);
+// After a substep that stored no words: counts every particle's neighbors
+// into c.ncount and their sum into c.pair_total.
+hipError_t enqueue_count_pairs(Ctx& c);
+// ... or stores the lists too long for a row (nwords kLongList) in c.nbr;
+// *c.nbr_total is what they need, and a list that does not fit is left out.
+hipError_t enqueue_long_lists(Ctx& c);
 
 // The tile kernels (pbf_tiles.hip).
 hipError_t enqueue_tile_classify(Ctx& c, const StepConsts& k);

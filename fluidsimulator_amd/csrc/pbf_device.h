@@ -7,6 +7,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stdint.h>
 
 namespace fluidhip {
@@ -55,12 +56,9 @@ struct StepConsts {
   float vort_norm_eps;
   int record_diag;
   int xcd_remap;
-  int coop;         // 1: wavefronts sharing a cell use shared candidate tiles
-  int coop_bulk;    // 1: ... and whole coincident tiles in one step
-  int runs;         // 1: one lane per run of identical consecutive slots
-  int full_lists;   // 1: cooperative particles get stored lists too (otherwise
-                    //    their passes retest the list's distance predicate)
-  int count_only;   // 1: the neighbor walk only counts pairs (statistics)
+  int runs;         // 1: a run of identical consecutive slots is computed once
+  int full_lists;   // 1: every particle's list is stored (the adjoint and the
+                    //    diagnostics read them)
   int tiles;        // 1: sparse 4x4x4-cell bricks run the LDS-tiled passes
 };
 
@@ -146,9 +144,8 @@ __device__ __forceinline__ float pair_spiky(float r2, const StepConsts& c) {
 
 // The neighbor predicate: candidate q is a neighbor of a particle at p when
 // |p - q|^2 < h^2, both at their predicted positions p^0 (core.cpp:140-142
-// and 222-245).  Lists and neighbor masks are built with it, and cooperative
-// walks retest it instead of reading stored lists, so all must use this one
-// expression.
+// and 222-245).  Lists are built with it, and walks without a list retest
+// it, so all must use this one expression.
 __device__ __forceinline__ bool near0(const float3& p, const float3& q, const StepConsts& c) {
   const float ex = p.x - q.x;
   const float ey = p.y - q.y;
@@ -156,19 +153,23 @@ __device__ __forceinline__ bool near0(const float3& p, const float3& q, const St
   return ex * ex + ey * ey + ez * ez < c.h2;
 }
 
-// Lanes whose own cell holds at least this many particles are served by
-// wavefront-cooperative walks (one per distinct dense cell in the
-// wavefront); the others walk alone.
+// Particles of cells of at least this many walk the 27 cells in every pass
+// instead of storing a list.
 constexpr int kDenseCell = 32;
-// ... and so are lanes with at least this many neighbors (or, while the
-// lists are built, candidates).
-constexpr int kHeavyList = 256;
 
-// Z-order of a cell inside its brick: the low `bits` bits of x, y, z
-// interleaved as x0 y0 z0 x1 y1 z1 ...
-__device__ __forceinline__ int morton_in_brick(int x, int y, int z, int bits) {
+// A dense unit of one head only (in the scene's sign bit).
+constexpr int kSingle = INT_MIN;
+
+// nwords of a slot without words: none stored, neighbors in the slot's row,
+// or too many for a row.
+constexpr int kRowList = -2, kLongList = -3;
+
+// Z-order of a cell inside its brick of up to 8 cells an edge: the low bits
+// of x, y, z interleaved as x0 y0 z0 x1 y1 z1 x2 y2 z2.
+__device__ __forceinline__ int morton_in_brick(int x, int y, int z) {
   int m = 0;
-  for (int b = 0; b < bits; ++b)
+#pragma unroll
+  for (int b = 0; b < 3; ++b)
     m |= (((x >> b) & 1) << (3 * b)) | (((y >> b) & 1) << (3 * b + 1)) |
          (((z >> b) & 1) << (3 * b + 2));
   return m;
@@ -183,7 +184,7 @@ __device__ __forceinline__ int cell_key(int rx, int ry, int rz, const GridDesc& 
   const int s = g.bshift;
   const int m = (1 << s) - 1;
   const int b = ((rz >> s) * g.nby + (ry >> s)) * g.nbx + (rx >> s);
-  return g.cell_off + (b << (3 * s)) + morton_in_brick(rx & m, ry & m, rz & m, s);
+  return g.cell_off + (b << (3 * s)) + morton_in_brick(rx & m, ry & m, rz & m);
 }
 
 __device__ __forceinline__ int floor_cell(float v, float inv_h, bool& bad) {
@@ -300,33 +301,5 @@ struct NbrView {
   const int* __restrict__ list;
   const int* __restrict__ count;
 };
-
-// Calls f(t, load(t)) for each neighbor slot t of slot s, in list order.
-// Runs are walked four slots at a time with the four loads issued before
-// any use, which keeps several memory requests in flight per lane; the
-// callbacks still run strictly in list order, so every sum accumulates in
-// the reference's order.
-template <typename Load, typename F>
-__device__ __forceinline__ void for_each_neighbor(const NbrView& v, int s, Load&& load, F&& f) {
-  const int* __restrict__ L = v.list + v.off[s];
-  const int nw = v.nw[s];
-  for (int w = 0; w < nw;) {
-    const int e = L[w++];
-    int t = e & 0x7fffffff;
-    int end = t + 1;
-    if (e < 0) end = t + L[w++];
-    for (; t + 4 <= end; t += 4) {
-      const auto a = load(t);
-      const auto b = load(t + 1);
-      const auto c = load(t + 2);
-      const auto d = load(t + 3);
-      f(t, a);
-      f(t + 1, b);
-      f(t + 2, c);
-      f(t + 3, d);
-    }
-    for (; t < end; ++t) f(t, load(t));
-  }
-}
 
 }  // namespace fluidhip
