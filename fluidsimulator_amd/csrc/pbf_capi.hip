@@ -247,6 +247,176 @@ void dfree(T*& p) {
   p = nullptr;
 }
 
+// Device memory and streams of destroyed contexts, kept for the next ones:
+// a program that steps through the stateless call creates and destroys a
+// context for every substep, and hipMalloc and hipFree of its buffers took 0.9
+// to 2.5 ms of each call (of the 1,728-particle call's 2.0 ms in all, and up to
+// 3.9 ms), hipFree of the two 64 MiB cell arrays alone 0.5 ms.  Bounded:
+// at most kKeepBytes over all devices (more is freed, oldest first) and
+// kKeepStreams stream sets; given back when an allocation fails.  A block is
+// kept only once the work that used it has finished, and belongs to nobody
+// until it is handed out again, so any thread may take it.
+constexpr size_t kKeepBytes = static_cast<size_t>(256) << 20;
+constexpr size_t kKeepStreams = 4;
+
+struct Kept {
+  struct Block {
+    int device;
+    void* p;
+    size_t bytes;
+  };
+  struct Streams {
+    int device;
+    hipStream_t main, side;
+    hipEvent_t fork, join;
+  };
+  std::mutex mu;
+  std::vector<Block> blocks;  // oldest first
+  size_t bytes = 0;
+  std::vector<Streams> streams;
+};
+Kept& kept() {
+  static Kept* k = new Kept();  // never destroyed: contexts may outlive statics
+  return *k;
+}
+
+// The current device's memory of at least `bytes` (at most twice as much, so
+// that a small context does not hold a large one's); *got is its size.
+hipError_t take_block(int device, size_t bytes, void** p, size_t* got) {
+  *p = nullptr;
+  *got = bytes;
+  Kept& k = kept();
+  {
+    std::lock_guard<std::mutex> lock(k.mu);
+    size_t best = k.blocks.size();
+    for (size_t i = 0; i < k.blocks.size(); ++i) {
+      const Kept::Block& b = k.blocks[i];
+      if (b.device == device && b.bytes >= bytes && b.bytes / 2 <= bytes &&
+          (best == k.blocks.size() || b.bytes < k.blocks[best].bytes))
+        best = i;
+    }
+    if (best < k.blocks.size()) {
+      *p = k.blocks[best].p;
+      *got = k.blocks[best].bytes;
+      k.bytes -= *got;
+      k.blocks.erase(k.blocks.begin() + static_cast<long>(best));
+      return hipSuccess;
+    }
+  }
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  std::vector<Kept::Block> out;
+  {
+    std::lock_guard<std::mutex> lock(k.mu);
+    out.swap(k.blocks);
+    k.bytes = 0;
+  }
+  for (auto& b : out) (void)hipFree(b.p);
+  return hipMalloc(p, bytes);
+}
+
+// Gives back a block whose work has finished.
+void give_block(int device, void* p, size_t bytes) {
+  if (!p) return;
+  Kept& k = kept();
+  std::vector<Kept::Block> out;
+  {
+    std::lock_guard<std::mutex> lock(k.mu);
+    k.blocks.push_back({device, p, bytes});
+    k.bytes += bytes;
+    size_t n = 0;
+    while (k.bytes > kKeepBytes) k.bytes -= k.blocks[n++].bytes;
+    out.assign(k.blocks.begin(), k.blocks.begin() + static_cast<long>(n));
+    k.blocks.erase(k.blocks.begin(), k.blocks.begin() + static_cast<long>(n));
+  }
+  for (auto& b : out) (void)hipFree(b.p);
+}
+
+template <typename T>
+hipError_t take_array(int device, size_t count, T** p, size_t* got) {
+  void* q = nullptr;
+  const hipError_t e = take_block(device, std::max<size_t>(count, 1) * sizeof(T), &q, got);
+  *p = static_cast<T*>(q);
+  return e;
+}
+
+// Lays arrays out one after another in [base, base + bytes), or with a null
+// base only counts what they need.
+struct Carver {
+  unsigned char* base;
+  size_t bytes;
+  size_t off = 0;
+  bool ok = true;
+  template <typename T>
+  void take(T*& p, size_t count) {
+    off = (off + 255) & ~static_cast<size_t>(255);
+    const size_t need = std::max<size_t>(count, 1) * sizeof(T);
+    p = nullptr;
+    if (base && off + need > bytes) ok = false;
+    if (base && ok) p = reinterpret_cast<T*>(base + off);
+    off += need;
+  }
+};
+
+// Entries of a tile particle's neighbor list for a batch of n particles.
+int tile_list_cap_for(long long n) {
+  return n < fluidhip::kForkMinParticles ? fluidhip::kTileListSmall : fluidhip::kTileList;
+}
+
+// Every array of a context but for the cell table, the neighbor lists and the
+// transfers' staging.
+void carve_arrays(Ctx& c, Carver& a, bool omega) {
+  const size_t n = static_cast<size_t>(c.n), ns = static_cast<size_t>(c.n_scenes);
+  for (float4** q : {&c.posA, &c.velA, &c.posB, &c.velB, &c.pred[0], &c.pred[1], &c.pred[2]})
+    a.take(*q, n);
+  if (omega) a.take(c.omega, n);
+  a.take(c.rho, n);
+  a.take(c.cellc, n);
+  a.take(c.key, n);
+  for (int q = 0; q < 2; ++q) {
+    a.take(c.sort_k[q], n);
+    a.take(c.sort_v[q], n);
+  }
+  c.radix_blocks = static_cast<int>((n + fluidhip::kRadixTile - 1) / fluidhip::kRadixTile);
+  a.take(c.radix_hist, 256 * static_cast<size_t>(c.radix_blocks));
+  a.take(c.radix_off, 256 * static_cast<size_t>(c.radix_blocks) + 1);
+  a.take(c.radix_len, 1);
+  a.take(c.slot_cell, n);
+  a.take(c.slot_key, n);
+  a.take(c.noff, n);
+  a.take(c.nwords, n);
+  a.take(c.ncount, n);
+  a.take(c.bbox, 6 * ns);
+  a.take(c.tile_bbox, 6 * (n / 64 + 1));
+  a.take(c.run_no, n);
+  a.take(c.rep_list, n + 1);
+  a.take(c.units, n);
+  a.take(c.dense, n);
+  a.take(c.info, 4);
+  a.take(c.grid, ns);
+  a.take(c.total_cells, 1);
+  a.take(c.scan_partial, 3 * static_cast<size_t>(c.scan_blocks) + 2);
+  a.take(c.nbr_total, 1);
+  a.take(c.need_cells, 1);
+  a.take(c.pair_total, 1);
+  a.take(c.seg, ns + 1);
+  a.take(c.planes, ns);
+  a.take(c.flags, 1);
+  a.take(c.steps_started, 1);
+  // brick tiles: beyond this capacity bricks take the other passes
+  c.tile_cap = static_cast<long long>(n / 32 + 256);
+  a.take(c.in_tile, n);
+  a.take(c.tile_count, 2);
+  a.take(c.tile_cand, static_cast<size_t>(c.tile_cap));
+  a.take(c.tile_rec, 2 * static_cast<size_t>(c.tile_cap));
+  a.take(c.tile_seg, static_cast<size_t>(c.tile_cap) * 217);
+  a.take(c.tile_src, static_cast<size_t>(c.tile_cap) * 216);
+  c.tile_list_cap = tile_list_cap_for(c.n);
+  a.take(c.tile_list, static_cast<size_t>(c.tile_list_cap / 8) * n);
+  a.take(c.tile_cnt, n);
+}
+
 void drop_graph(Ctx& c) {
   if (c.graph_exec) hipGraphExecDestroy(c.graph_exec);
   if (c.graph) hipGraphDestroy(c.graph);
@@ -259,38 +429,12 @@ void free_adj(Ctx& c);
 void free_all(Ctx& c) {
   drop_graph(c);
   free_adj(c);
-  for (float4** p : {&c.posA, &c.velA, &c.posB, &c.velB, &c.pred[0], &c.pred[1], &c.pred[2],
-                    &c.omega})
-    dfree(*p);
-  dfree(c.rho);
-  dfree(c.cellc);
-  for (int** p : {&c.key, &c.sort_k[0], &c.sort_k[1], &c.sort_v[0], &c.sort_v[1],
-                  &c.radix_hist, &c.radix_off, &c.radix_len, &c.count, &c.start, &c.bbox,
-                  &c.total_cells, &c.scan_partial, &c.slot_key, &c.nbr, &c.seg, &c.nwords,
-                  &c.ncount, &c.tile_bbox, &c.run_no, &c.rep_list, &c.info,
-                  &c.steps_started})
-    dfree(*p);
-  dfree(c.units);
-  dfree(c.dense);
-  dfree(c.slot_cell);
-  dfree(c.grid);
-  dfree(c.in_tile);
-  dfree(c.tile_count);
-  dfree(c.tile_cand);
-  dfree(c.tile_rec);
-  dfree(c.tile_seg);
-  dfree(c.tile_src);
-  dfree(c.tile_list);
-  dfree(c.tile_cnt);
-  dfree(c.noff);
-  dfree(c.nwords);
-  dfree(c.ncount);
-  dfree(c.nbr_total);
-  dfree(c.need_cells);
-  dfree(c.pair_total);
-  dfree(c.planes);
-  dfree(c.flags);
-  dfree(c.stage);
+  give_block(c.device, c.arena, c.arena_bytes);
+  give_block(c.device, c.count, c.count_bytes);
+  give_block(c.device, c.start, c.start_bytes);
+  give_block(c.device, c.nbr, c.nbr_bytes);
+  c.arena = nullptr;
+  c.count = c.start = c.nbr = nullptr;
   for (auto& q : c.prof.pending) {
     hipEventDestroy(q.a);
     hipEventDestroy(q.b);
@@ -303,18 +447,23 @@ void free_all(Ctx& c) {
 }
 
 int alloc_cells(Ctx& c, long long cap) {
-  dfree(c.count);
-  dfree(c.start);
-  HIP_TRY(dalloc(&c.count, cap), "hipMalloc(cell counts)");
-  HIP_TRY(dalloc(&c.start, cap + 1), "hipMalloc(cell starts)");
+  give_block(c.device, c.count, c.count_bytes);
+  give_block(c.device, c.start, c.start_bytes);
+  c.count = c.start = nullptr;
+  HIP_TRY(take_array(c.device, static_cast<size_t>(cap), &c.count, &c.count_bytes),
+          "hipMalloc(cell counts)");
+  HIP_TRY(take_array(c.device, static_cast<size_t>(cap) + 1, &c.start, &c.start_bytes),
+          "hipMalloc(cell starts)");
   HIP_TRY(hipMemsetAsync(c.count, 0, sizeof(int) * cap, c.stream), "hipMemset(cell counts)");
   c.cell_cap = cap;
   return FLUID_HIP_OK;
 }
 
 int alloc_neighbors(Ctx& c, long long cap) {
-  dfree(c.nbr);
-  HIP_TRY(dalloc(&c.nbr, cap), "hipMalloc(neighbor list)");
+  give_block(c.device, c.nbr, c.nbr_bytes);
+  c.nbr = nullptr;
+  HIP_TRY(take_array(c.device, static_cast<size_t>(cap), &c.nbr, &c.nbr_bytes),
+          "hipMalloc(neighbor list)");
   c.nbr_cap = cap;
   return FLUID_HIP_OK;
 }
@@ -450,12 +599,7 @@ using fluidhip::AdjRecord;
 using fluidhip::SubTape;
 
 void free_tape(SubTape& t) {
-  for (float4** p : {&t.X, &t.PI, &t.VC, &t.P, &t.SQ}) dfree(*p);
-  dfree(t.M);
-  dfree(t.RM);
-  dfree(t.noff);
-  dfree(t.nwords);
-  dfree(t.ncount);
+  dfree(t.block);
   dfree(t.nbr);
   t.nbr_cap = 0;
   t.Pk.clear();
@@ -488,16 +632,20 @@ void invalidate_record(Ctx& c) {
 int alloc_tape(Ctx& c, SubTape& t) {
   const size_t n = static_cast<size_t>(std::max(c.n, 1));
   const size_t I = static_cast<size_t>(c.iterations);
-  HIP_TRY(dalloc(&t.X, n), "hipMalloc(tape)");
-  HIP_TRY(dalloc(&t.PI, n), "hipMalloc(tape)");
-  HIP_TRY(dalloc(&t.VC, n), "hipMalloc(tape)");
-  HIP_TRY(dalloc(&t.P, I * n), "hipMalloc(tape iterates)");
-  HIP_TRY(dalloc(&t.SQ, I * n), "hipMalloc(tape sums)");
-  HIP_TRY(dalloc(&t.M, I * n), "hipMalloc(tape masks)");
-  HIP_TRY(dalloc(&t.RM, n), "hipMalloc(tape masks)");
-  HIP_TRY(dalloc(&t.noff, n), "hipMalloc(tape lists)");
-  HIP_TRY(dalloc(&t.nwords, n), "hipMalloc(tape lists)");
-  HIP_TRY(dalloc(&t.ncount, n), "hipMalloc(tape lists)");
+  auto carve = [&](Carver a) {
+    for (float4** p : {&t.X, &t.PI, &t.VC}) a.take(*p, n);
+    a.take(t.P, I * n);
+    a.take(t.SQ, I * n);
+    a.take(t.M, I * n);
+    a.take(t.RM, n);
+    a.take(t.noff, n);
+    a.take(t.nwords, n);
+    a.take(t.ncount, n);
+    return a.off;
+  };
+  const size_t bytes = carve(Carver{nullptr, 0});
+  HIP_TRY(dalloc(&t.block, bytes), "hipMalloc(tape)");
+  (void)carve(Carver{t.block, bytes});
   t.Pk.resize(I);
   t.SQk.resize(I);
   t.Mk.resize(I);
@@ -619,14 +767,45 @@ int noalloc_scratch(int dev, unsigned char** out) {
   return FLUID_HIP_OK;
 }
 
-// Entries of a tile particle's neighbor list for a batch of n particles.
-int tile_list_cap_for(long long n) {
-  return n < fluidhip::kForkMinParticles ? fluidhip::kTileListSmall : fluidhip::kTileList;
+// The context's streams and events: kept ones, or new ones.
+hipError_t make_streams(Ctx& c) {
+  Kept& k = kept();
+  {
+    std::lock_guard<std::mutex> lock(k.mu);
+    for (size_t i = 0; i < k.streams.size(); ++i)
+      if (k.streams[i].device == c.device) {
+        const Kept::Streams s = k.streams[i];
+        k.streams.erase(k.streams.begin() + static_cast<long>(i));
+        c.stream = s.main;
+        c.own_stream = true;
+        c.side = s.side;
+        c.ev_fork = s.fork;
+        c.ev_join = s.join;
+        return hipSuccess;
+      }
+  }
+  hipError_t e = hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking);
+  if (e != hipSuccess) return e;
+  c.own_stream = true;
+  // the side stream of the LDS-tile kernels and its fork/join events
+  e = hipStreamCreateWithFlags(&c.side, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&c.ev_fork, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&c.ev_join, hipEventDisableTiming);
+  return e;
 }
 
-// The context's own streams and events (the main stream only when it is not
-// the caller's).
+// Gives back the context's own streams and events (the main stream only when
+// it is not the caller's); their work has finished.
 void destroy_streams(Ctx& c) {
+  if (c.own_stream && c.stream && c.side && c.ev_fork && c.ev_join) {
+    Kept& k = kept();
+    std::lock_guard<std::mutex> lock(k.mu);
+    if (k.streams.size() < kKeepStreams) {
+      k.streams.push_back({c.device, c.stream, c.side, c.ev_fork, c.ev_join});
+      c.stream = c.side = nullptr;
+      c.ev_fork = c.ev_join = nullptr;
+    }
+  }
   if (c.ev_fork) hipEventDestroy(c.ev_fork);
   if (c.ev_join) hipEventDestroy(c.ev_join);
   if (c.side) hipStreamDestroy(c.side);
@@ -641,80 +820,22 @@ void destroy_streams(Ctx& c) {
 // between the neighbor lists (5/8) and the cell table (3/8).  Returns false
 // when they do not fit.
 bool noalloc_layout(Ctx& c, unsigned char* base, size_t bytes) {
-  size_t off = 0;
-  bool ok = true;
-  auto take = [&](auto*& p, size_t count) {
-    using T = std::remove_reference_t<decltype(*p)>;
-    off = (off + 255) & ~static_cast<size_t>(255);
-    const size_t need = std::max<size_t>(count, 1) * sizeof(T);
-    if (off + need > bytes) {
-      ok = false;
-      p = nullptr;
-      return;
-    }
-    p = reinterpret_cast<T*>(base + off);
-    off += need;
-  };
-  const size_t n = static_cast<size_t>(c.n);
-  for (float4** q : {&c.posA, &c.velA, &c.posB, &c.velB, &c.pred[0], &c.pred[1], &c.pred[2]})
-    take(*q, n);
-  if (c.vort) take(c.omega, n);
-  take(c.rho, n);
-  take(c.cellc, n);
-  take(c.key, n);
-  for (int q = 0; q < 2; ++q) {
-    take(c.sort_k[q], n);
-    take(c.sort_v[q], n);
-  }
-  c.radix_blocks = static_cast<int>((n + fluidhip::kRadixTile - 1) / fluidhip::kRadixTile);
-  take(c.radix_hist, 256 * static_cast<size_t>(c.radix_blocks));
-  take(c.radix_off, 256 * static_cast<size_t>(c.radix_blocks) + 1);
-  take(c.radix_len, 1);
-  take(c.slot_cell, n);
-  take(c.slot_key, n);
-  take(c.noff, n);
-  take(c.nwords, n);
-  take(c.ncount, n);
-  take(c.bbox, 6);
-  take(c.tile_bbox, 6 * (n / 64 + 1));
-  take(c.run_no, n);
-  take(c.rep_list, n + 1);
-  take(c.units, n);
-  take(c.dense, n);
-  take(c.info, 4);
-  take(c.grid, 1);
-  take(c.total_cells, 1);
-  take(c.scan_partial, 3 * static_cast<size_t>(c.scan_blocks) + 2);
-  take(c.nbr_total, 1);
-  take(c.need_cells, 1);
-  take(c.pair_total, 1);
-  take(c.seg, 2);
-  take(c.planes, 1);
-  take(c.flags, 1);
-  take(c.steps_started, 1);
-  c.tile_cap = static_cast<long long>(n / 32 + 256);
-  take(c.in_tile, n);
-  take(c.tile_count, 2);
-  take(c.tile_cand, static_cast<size_t>(c.tile_cap));
-  take(c.tile_rec, 2 * static_cast<size_t>(c.tile_cap));
-  take(c.tile_seg, static_cast<size_t>(c.tile_cap) * 217);
-  take(c.tile_src, static_cast<size_t>(c.tile_cap) * 216);
-  c.tile_list_cap = tile_list_cap_for(c.n);
-  take(c.tile_list, static_cast<size_t>(c.tile_list_cap / 8) * n);
-  take(c.tile_cnt, n);
-  if (!ok) return false;
-  off = (off + 255) & ~static_cast<size_t>(255);
-  const size_t rest = bytes - off;
+  Carver a{base, bytes};
+  c.lane_cap = 3ll * c.n + 64;
+  carve_arrays(c, a, c.vort);
+  if (!a.ok) return false;
+  a.off = (a.off + 255) & ~static_cast<size_t>(255);
+  const size_t rest = bytes - a.off;
   const long long words = static_cast<long long>(rest / 8 * 5 / sizeof(int));
   const long long cells = static_cast<long long>((rest - static_cast<size_t>(words) * sizeof(int)) /
                                                  (2 * sizeof(int))) - 512;
   if (words < 1 || cells < 1) return false;
-  take(c.nbr, static_cast<size_t>(words));
+  a.take(c.nbr, static_cast<size_t>(words));
   c.nbr_cap = words;
   c.cell_cap = std::min<long long>(cells, INT_MAX - 1);
-  take(c.count, static_cast<size_t>(c.cell_cap));
-  take(c.start, static_cast<size_t>(c.cell_cap) + 1);
-  return ok;
+  a.take(c.count, static_cast<size_t>(c.cell_cap));
+  a.take(c.start, static_cast<size_t>(c.cell_cap) + 1);
+  return a.ok;
 }
 
 // What must start at zero or at a known value: the scene tables, counters,
@@ -820,81 +941,28 @@ int fluid_hip_create(fluid_hip_ctx** out, int32_t n_scenes, const int64_t* scene
   };
   hipError_t e = hipSetDevice(c.device);
   if (e != hipSuccess) return bail(hip_fail(e, "hipSetDevice"));
-  e = hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking);
+  e = make_streams(c);
   if (e != hipSuccess) return bail(hip_fail(e, "hipStreamCreate"));
-  c.own_stream = true;
-  // the side stream of the LDS-tile kernels and its fork/join events
-  e = hipStreamCreateWithFlags(&c.side, hipStreamNonBlocking);
-  if (e != hipSuccess) return bail(hip_fail(e, "hipStreamCreate"));
-  e = hipEventCreateWithFlags(&c.ev_fork, hipEventDisableTiming);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&c.ev_join, hipEventDisableTiming);
-  if (e != hipSuccess) return bail(hip_fail(e, "hipEventCreate"));
 
   const size_t n = static_cast<size_t>(c.n);
-  const bool need_omega = c.vort;
-#define ALLOC(ptr, cnt)                                        \
-  do {                                                         \
-    e = dalloc(&(ptr), (cnt));                                 \
-    if (e != hipSuccess) return bail(hip_fail(e, "hipMalloc " #ptr)); \
-  } while (0)
-  ALLOC(c.posA, n);
-  ALLOC(c.velA, n);
-  ALLOC(c.posB, n);
-  ALLOC(c.velB, n);
-  ALLOC(c.pred[0], n);
-  ALLOC(c.pred[1], n);
-  ALLOC(c.pred[2], n);
-  if (need_omega) ALLOC(c.omega, n);
-  ALLOC(c.rho, n);
-  ALLOC(c.cellc, n);
-  ALLOC(c.key, n);
-  for (int q = 0; q < 2; ++q) {
-    ALLOC(c.sort_k[q], n);
-    ALLOC(c.sort_v[q], n);
-  }
-  c.radix_blocks = (n + fluidhip::kRadixTile - 1) / fluidhip::kRadixTile;
-  ALLOC(c.radix_hist, 256 * static_cast<size_t>(c.radix_blocks));
-  ALLOC(c.radix_off, 256 * static_cast<size_t>(c.radix_blocks) + 1);
-  ALLOC(c.radix_len, 1);
-  ALLOC(c.slot_cell, n);
-  ALLOC(c.slot_key, n);
-  ALLOC(c.noff, n);
-  ALLOC(c.nwords, n);
-  ALLOC(c.ncount, n);
-  ALLOC(c.bbox, 6 * static_cast<size_t>(n_scenes));
-  ALLOC(c.tile_bbox, 6 * (n / 64 + 1));
-  ALLOC(c.run_no, n);
-  ALLOC(c.rep_list, n + 1);
-  ALLOC(c.units, n);
-  ALLOC(c.dense, n);
-  ALLOC(c.info, 4);
   c.lane_cap = 3ll * n + 64;
   if (cfg.lane_capacity > 0)
     c.lane_cap = std::min<long long>(c.lane_cap, std::max<long long>(cfg.lane_capacity, n));
-  ALLOC(c.grid, static_cast<size_t>(n_scenes));
-  ALLOC(c.total_cells, 1);
-  ALLOC(c.scan_partial, 3 * static_cast<size_t>(c.scan_blocks) + 2);
-  ALLOC(c.nbr_total, 1);
-  ALLOC(c.need_cells, 1);
-  ALLOC(c.pair_total, 1);
-  ALLOC(c.seg, static_cast<size_t>(n_scenes) + 1);
-  ALLOC(c.planes, static_cast<size_t>(n_scenes));
-  ALLOC(c.flags, 1);
-  ALLOC(c.steps_started, 1);
-  ALLOC(c.stage, 6 * n);
-  // brick tiles (at least 32 particles each): beyond this capacity bricks
-  // take the per-lane passes
-  c.tile_cap = static_cast<long long>(n / 32 + 256);
-  ALLOC(c.in_tile, n);
-  ALLOC(c.tile_count, 2);
-  ALLOC(c.tile_cand, static_cast<size_t>(c.tile_cap));
-  ALLOC(c.tile_rec, 2 * static_cast<size_t>(c.tile_cap));
-  ALLOC(c.tile_seg, static_cast<size_t>(c.tile_cap) * 217);
-  ALLOC(c.tile_src, static_cast<size_t>(c.tile_cap) * 216);
-  c.tile_list_cap = tile_list_cap_for(c.n);
-  ALLOC(c.tile_list, static_cast<size_t>(c.tile_list_cap / 8) * n);
-  ALLOC(c.tile_cnt, n);
-#undef ALLOC
+  {
+    // one block for all fixed arrays (omega too: set_params may turn
+    // vorticity on)
+    Carver count{nullptr, 0};
+    carve_arrays(c, count, true);
+    count.take(c.stage, 6 * n);
+    void* p = nullptr;
+    e = take_block(c.device, count.off, &p, &c.arena_bytes);
+    if (e != hipSuccess) return bail(hip_fail(e, "hipMalloc(context)"));
+    c.arena = static_cast<unsigned char*>(p);
+    Carver a{c.arena, c.arena_bytes};
+    carve_arrays(c, a, true);
+    a.take(c.stage, 6 * n);
+    if (!a.ok) return bail(fail(FLUID_HIP_EHIP, "context layout"));
+  }
   {
     const int len = 256 * c.radix_blocks;
     e = hipMemcpy(c.radix_len, &len, sizeof(int), hipMemcpyHostToDevice);
@@ -944,11 +1012,9 @@ int fluid_hip_set_params(fluid_hip_ctx* ctx, const fluid_hip_params* params) {
   if (rc) return rc;
   Ctx& c = ctx->c;
   if ((rc = validate(c.n_scenes, params))) return rc;
-  const bool had_omega = c.omega != nullptr;
   c.params.assign(params, params + c.n_scenes);
   compute_consts(c);
   invalidate_record(c);
-  if (c.vort && !had_omega) HIP_TRY(dalloc(&c.omega, std::max(c.n, 1)), "hipMalloc omega");
   auto tables = scene_tables(c);
   HIP_TRY(hipMemcpyAsync(c.planes, tables.data(), sizeof(fluidhip::ScenePlanes) * c.n_scenes,
                          hipMemcpyHostToDevice, c.stream),

@@ -108,6 +108,11 @@ struct Ctx {
   int brick_shift = 2;  // log2 of the cells per brick edge of the cell table
   int tile_gather = 0;  // 0 default (on), 1 on, 2 off: LDS-tiled passes for sparse bricks
 
+  // device memory of the context: one block for the arrays below but for the
+  // cell table and the neighbor lists, which grow in blocks of their own
+  unsigned char* arena = nullptr;
+  size_t arena_bytes = 0, count_bytes = 0, start_bytes = 0, nbr_bytes = 0;
+
   // state (A = committed state between substeps)
   float4* posA = nullptr;  // xyz, w = original id bits
   float4* velA = nullptr;  // xyz, w = rho of the last lambda pass (scratch)
@@ -226,6 +231,7 @@ hipError_t enqueue_substep(Ctx& c, const SubstepRec* rec = nullptr);
 // What the adjoint of one substep reads (device arrays, that substep's slot
 // order; P, SQ and M hold `iterations` consecutive blocks of n entries).
 struct SubTape {
+  unsigned char* block = nullptr;  // holds every array below but the lists
   float4* X = nullptr;    // input positions, w = original id
   float4* PI = nullptr;   // committed positions p^I
   float4* VC = nullptr;   // commit velocity (xyz) and rho of the last lambda pass (w)
