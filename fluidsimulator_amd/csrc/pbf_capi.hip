@@ -373,7 +373,6 @@ void carve_arrays(Ctx& c, Carver& a, bool omega) {
   if (omega) a.take(c.omega, n);
   a.take(c.rho, n);
   a.take(c.cellc, n);
-  a.take(c.key, n);
   for (int q = 0; q < 2; ++q) {
     a.take(c.sort_k[q], n);
     a.take(c.sort_v[q], n);
@@ -381,7 +380,6 @@ void carve_arrays(Ctx& c, Carver& a, bool omega) {
   c.radix_blocks = static_cast<int>((n + fluidhip::kRadixTile - 1) / fluidhip::kRadixTile);
   a.take(c.radix_hist, 256 * static_cast<size_t>(c.radix_blocks));
   a.take(c.radix_off, 256 * static_cast<size_t>(c.radix_blocks) + 1);
-  a.take(c.radix_len, 1);
   a.take(c.slot_cell, n);
   a.take(c.slot_key, n);
   a.take(c.noff, n);
@@ -393,7 +391,7 @@ void carve_arrays(Ctx& c, Carver& a, bool omega) {
   a.take(c.rep_list, n + 1);
   a.take(c.units, n);
   a.take(c.dense, n);
-  a.take(c.info, 4);
+  a.take(c.info, 5);
   a.take(c.grid, ns);
   a.take(c.total_cells, 1);
   a.take(c.scan_partial, 3 * static_cast<size_t>(c.scan_blocks) + 2);
@@ -430,11 +428,10 @@ void free_all(Ctx& c) {
   drop_graph(c);
   free_adj(c);
   give_block(c.device, c.arena, c.arena_bytes);
-  give_block(c.device, c.count, c.count_bytes);
   give_block(c.device, c.start, c.start_bytes);
   give_block(c.device, c.nbr, c.nbr_bytes);
   c.arena = nullptr;
-  c.count = c.start = c.nbr = nullptr;
+  c.start = c.nbr = nullptr;
   for (auto& q : c.prof.pending) {
     hipEventDestroy(q.a);
     hipEventDestroy(q.b);
@@ -447,14 +444,10 @@ void free_all(Ctx& c) {
 }
 
 int alloc_cells(Ctx& c, long long cap) {
-  give_block(c.device, c.count, c.count_bytes);
   give_block(c.device, c.start, c.start_bytes);
-  c.count = c.start = nullptr;
-  HIP_TRY(take_array(c.device, static_cast<size_t>(cap), &c.count, &c.count_bytes),
-          "hipMalloc(cell counts)");
+  c.start = nullptr;
   HIP_TRY(take_array(c.device, static_cast<size_t>(cap) + 1, &c.start, &c.start_bytes),
           "hipMalloc(cell starts)");
-  HIP_TRY(hipMemsetAsync(c.count, 0, sizeof(int) * cap, c.stream), "hipMemset(cell counts)");
   c.cell_cap = cap;
   return FLUID_HIP_OK;
 }
@@ -828,39 +821,31 @@ bool noalloc_layout(Ctx& c, unsigned char* base, size_t bytes) {
   const size_t rest = bytes - a.off;
   const long long words = static_cast<long long>(rest / 8 * 5 / sizeof(int));
   const long long cells = static_cast<long long>((rest - static_cast<size_t>(words) * sizeof(int)) /
-                                                 (2 * sizeof(int))) - 512;
+                                                 sizeof(int)) - 512;
   if (words < 1 || cells < 1) return false;
   a.take(c.nbr, static_cast<size_t>(words));
   c.nbr_cap = words;
   c.cell_cap = std::min<long long>(cells, INT_MAX - 1);
-  a.take(c.count, static_cast<size_t>(c.cell_cap));
   a.take(c.start, static_cast<size_t>(c.cell_cap) + 1);
   return a.ok;
 }
 
 // What must start at zero or at a known value: the scene tables, counters,
-// flags and bounding box, and the cell histogram (kernel stores, so the
+// flags and bounding box (kernel stores, so the
 // sequence holds no memset node if a caller captures it).
-__global__ void k_noalloc_init(int n, int radix_len, fluidhip::ScenePlanes sp, int* seg,
-                               fluidhip::ScenePlanes* planes, int* rlen, int* bbox,
+__global__ void k_noalloc_init(int n, fluidhip::ScenePlanes sp, int* seg,
+                               fluidhip::ScenePlanes* planes, int* info, int* bbox,
                                unsigned* flags, int* steps_started) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     seg[0] = 0;
     seg[1] = n;
     *planes = sp;
-    *rlen = radix_len;
+    info[4] = 0;
     bbox[0] = bbox[1] = bbox[2] = INT_MAX;
     bbox[3] = bbox[4] = bbox[5] = INT_MIN;
     *flags = 0u;
     *steps_started = 0;
   }
-}
-
-__global__ void k_zero_ints(int* p, long long count) {
-  const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
-  for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < count;
-       i += stride)
-    p[i] = 0;
 }
 
 }  // namespace
@@ -962,11 +947,6 @@ int fluid_hip_create(fluid_hip_ctx** out, int32_t n_scenes, const int64_t* scene
     carve_arrays(c, a, true);
     a.take(c.stage, 6 * n);
     if (!a.ok) return bail(fail(FLUID_HIP_EHIP, "context layout"));
-  }
-  {
-    const int len = 256 * c.radix_blocks;
-    e = hipMemcpy(c.radix_len, &len, sizeof(int), hipMemcpyHostToDevice);
-    if (e != hipSuccess) return bail(hip_fail(e, "hipMemcpy(radix length)"));
   }
   // Defaults leave room for the spray and pile-up of violent scenes (cell
   // tables of tens of millions of cells, run-length lists well above the
@@ -1817,12 +1797,10 @@ int fluid_hip_step_noalloc(const fluid_hip_params* params, int64_t n, float* pos
   if (!noalloc_layout(c, base, kNoAllocBytes))
     return fail(FLUID_HIP_ECAPACITY, "buffers do not fit the scratch array");
 
-  k_noalloc_init<<<1, 64, 0, c.stream>>>(c.n, 256 * c.radix_blocks, scene_table(*params), c.seg,
-                                         c.planes, c.radix_len, c.bbox, c.flags,
+  k_noalloc_init<<<1, 64, 0, c.stream>>>(c.n, scene_table(*params), c.seg,
+                                         c.planes, c.info, c.bbox, c.flags,
                                          c.steps_started);
   HIP_TRY(hipGetLastError(), "scratch set-up");
-  k_zero_ints<<<1024, 256, 0, c.stream>>>(c.count, c.cell_cap);
-  HIP_TRY(hipGetLastError(), "cell table clear");
   HIP_TRY(fluidhip::enqueue_upload(c, pos, vel), "upload kernel");
   for (int s = 0; s < nsteps; ++s) {
     const hipError_t e = fluidhip::enqueue_substep(c);

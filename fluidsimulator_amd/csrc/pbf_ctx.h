@@ -111,7 +111,7 @@ struct Ctx {
   // device memory of the context: one block for the arrays below but for the
   // cell table and the neighbor lists, which grow in blocks of their own
   unsigned char* arena = nullptr;
-  size_t arena_bytes = 0, count_bytes = 0, start_bytes = 0, nbr_bytes = 0;
+  size_t arena_bytes = 0, start_bytes = 0, nbr_bytes = 0;
 
   // state (A = committed state between substeps)
   float4* posA = nullptr;  // xyz, w = original id bits
@@ -127,16 +127,13 @@ struct Ctx {
 
   // grid
   uint64_t* cellc = nullptr;  // packed cell of pred0, previous order
-  int* key = nullptr;  // per slot of the previous order: cell key
   // stable radix sort of (cell key) over particles in id order; values are
   // previous slots, so the sorted values list the new (cell, id) order
   int* sort_k[2] = {nullptr, nullptr};
   int* sort_v[2] = {nullptr, nullptr};
   int* radix_hist = nullptr;  // 256 digits x radix_blocks
   int* radix_off = nullptr;   // its exclusive scan (+1)
-  int* radix_len = nullptr;   // 256 * radix_blocks, on the device (scan length)
   int radix_blocks = 0;
-  int* count = nullptr;  // cell_cap
   int* start = nullptr;  // cell_cap + 1
   long long cell_cap = 0;
   int* bbox = nullptr;   // n_scenes * 6
@@ -151,7 +148,7 @@ struct Ctx {
   int* rep_list = nullptr;     // n + 1: per run its first slot; [runs] = n
   int4* units = nullptr;       // per list head: {slot, neighbors or -1, slots of its run, scene}
   int2* dense = nullptr;       // groups of heads without a row: {first slot, scene | kSingle}
-  int* info = nullptr;         // 4: runs, list heads, dense units, heads per unit
+  int* info = nullptr;         // 5: runs, list heads, dense units, heads per unit, workgroups done
   long long lane_cap = 0;      // reported by the tuner; no layout depends on it
 
   // brick tiles (sparse bricks whose passes run through LDS)

@@ -30,6 +30,10 @@ constexpr unsigned kFlagFatal = kFlagRange | kFlagCells | kFlagNeighbors;
 // one from 148 to 135 us against 4096 (2048: 71 and 133 us).
 constexpr int kRadixTile = 1024;
 
+// Batches of up to this many particles are sorted, and their heads listed, by
+// one workgroup.
+constexpr int kSmallSort = 8192;
+
 struct StepConsts {
   int n;            // particles, all scenes
   int n_scenes;

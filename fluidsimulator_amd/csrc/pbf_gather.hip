@@ -278,6 +278,89 @@ __global__ __launch_bounds__(kBlock) void k_heads(
   }
 }
 
+// Both kernels in one workgroup, for batches of up to kSmallSort particles
+// (two launches of 5 us each become one): thread t holds slots t, t + 1024, ...
+__global__ __launch_bounds__(1024) void k_heads_small(
+    StepConsts c, const float4* __restrict__ posB, const float4* __restrict__ velB,
+    const int* __restrict__ slot_key, const int* __restrict__ start,
+    const int* __restrict__ in_tile, int* __restrict__ run_no, int* __restrict__ rep,
+    int4* __restrict__ units, int2* __restrict__ dense, int* __restrict__ info,
+    long long* __restrict__ noff, int* __restrict__ nwords, int* __restrict__ ncount,
+    const unsigned* __restrict__ flags) {
+  constexpr int kT = 1024, kW = kT / kWave, kR = kSmallSort / kT;
+  __shared__ int runs[kR * kW], lists[kR * kW];
+  __shared__ int nd_sh, ndense;
+  if (fatal(flags)) return;
+  const int n = c.n, tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  if (tid == 0) nd_sh = ndense = 0;
+  int cls[kR];
+#pragma unroll
+  for (int r = 0; r < kR; ++r) {
+    const int s = r * kT + tid;
+    cls[r] = s < n ? slot_class(c, s, posB, velB, slot_key, start, in_tile) : 0;
+  }
+  __syncthreads();
+  int nd = 0;
+#pragma unroll
+  for (int r = 0; r < kR; ++r) {
+    const int h = __popcll(__ballot(cls[r] & kHead)), l = __popcll(__ballot(cls[r] & kList));
+    nd += __popcll(__ballot(cls[r] & kDense));
+    if (lane == 0) {
+      runs[r * kW + w] = h;
+      lists[r * kW + w] = l;
+    }
+  }
+  if (lane == 0 && nd) atomicAdd(&nd_sh, nd);
+  __syncthreads();
+  // exclusive sums over the (round, wavefront) counts, in slot order
+  if (w < 2) {
+    int* a = w == 0 ? runs : lists;
+    int carry = 0;
+#pragma unroll
+    for (int i = 0; i < kR * kW; i += kWave) {
+      const int v = a[i + lane];
+      const int inc = incl_scan<kWave>(v);
+      a[i + lane] = carry + inc - v;
+      carry += __shfl(inc, kWave - 1);
+    }
+    if (lane == 0) {
+      info[w] = carry;
+      if (w == 0) rep[carry] = n;
+    }
+  }
+  __syncthreads();
+  const int unit = unit_heads(nd_sh);
+#pragma unroll
+  for (int r = 0; r < kR; ++r) {
+    const int s = r * kT + tid;
+    const unsigned long long mh = __ballot(cls[r] & kHead), ml = __ballot(cls[r] & kList);
+    const int run = runs[r * kW + w] + __popcll(mh & below);
+    if (s < n) {
+      const bool head = (cls[r] & kHead) != 0;
+      run_no[s] = head ? run : run - 1;
+      if (head) rep[run] = s;
+      if (cls[r] & (kList | kDense)) {
+        const int sc = __float_as_int(velB[s].w);
+        if (cls[r] & kList)
+          units[lists[r * kW + w] + __popcll(ml & below)] = make_int4(s, 0, 0, sc);
+        else if ((cls[r] & kCell) || (run & (unit - 1)) == 0)
+          dense[atomicAdd(&ndense, 1)] = make_int2(s, sc);
+      }
+      if (!(in_tile && in_tile[s])) {
+        noff[s] = 0;
+        nwords[s] = -1;
+        ncount[s] = 0;
+      }
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    info[2] = ndense;
+    info[3] = unit;
+  }
+}
+
 // ------------------------------------------------------------ cells
 
 // The slot range of cell `ci` (0..26, in (dz, dy, dx) order) around the cell
@@ -1428,6 +1511,12 @@ GatherView gather_view(const Ctx& c, const float4* p0) {
 hipError_t enqueue_heads(Ctx& c, const StepConsts& k) {
   const int G = std::min(c.scan_blocks, blocks_for(c.n, 4 * kBlock));
   const int* tile = k.tiles ? c.in_tile : nullptr;
+  if (c.n <= kSmallSort) {
+    k_heads_small<<<1, 1024, 0, c.stream>>>(k, c.posB, c.velB, c.slot_key, c.start, tile,
+                                            c.run_no, c.rep_list, c.units, c.dense, c.info,
+                                            c.noff, c.nwords, c.ncount, c.flags);
+    return hipGetLastError();
+  }
   k_head_count<<<G, kBlock, 0, c.stream>>>(k, c.posB, c.velB, c.slot_key, c.start, tile, c.run_no,
                                            c.scan_partial, c.flags);
   k_heads<<<G, kBlock, 0, c.stream>>>(k, c.scan_partial, c.velB, c.run_no, c.rep_list, c.units,

@@ -12,15 +12,13 @@
 //   predict_bbox  v' = v + g dt, pred0 = x + v' dt, cell = floor(pred0/h),
 //                 per-tile bounding boxes of cells        (core.cpp:150-161)
 //   grid_setup    per-scene table origin/extent, key offsets, counters
-//   cell_keys     key of each particle
-//   sort          keys in original-id order, then 8-bit LSD radix passes
-//                 (digit histogram, its scan, stable ballot-ranked scatter):
-//                 sorting stably by key leaves each cell's particles in
-//                 ascending id, the reference's order (core.cpp:164-203)
-//   cell_count    cell histogram from the sorted keys' runs, its exclusive
-//                 scan -> cell starts (two launches: range sums, then each
-//                 range scanned)
-//   reorder       gather each particle's state into its slot, recompute pred0
+//   sort          cell keys in original-id order, then 8-bit LSD radix passes
+//                 (digit histogram, its scan, stable ballot-ranked scatter;
+//                 small batches in one workgroup): sorting stably by key
+//                 leaves each cell's particles in ascending id, the
+//                 reference's order (core.cpp:164-203)
+//   reorder       gather each particle's state into its slot, recompute
+//                 pred0; cell starts from the sorted keys
 //   tiles         with 4-cell bricks: the bricks that run through LDS (the
 //                 particles of their good cells) and their neighbor lists
 //                 (pbf_tiles.hip; on the side stream in large batches)
@@ -37,6 +35,7 @@
 //                                                      (core.cpp:573-612)
 // Each gather pass also runs its tile kernel.
 
+#include <algorithm>
 #include <climits>
 
 #include "pbf_ctx.h"
@@ -127,10 +126,11 @@ __global__ void k_download(int n, const float4* __restrict__ posA, const float4*
   vel[2 * N + id] = v.z;
 }
 
-__global__ void k_reset_flags(unsigned* flags, int* steps_started) {
+__global__ void k_reset_flags(unsigned* flags, int* steps_started, int* info) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     *flags = 0u;
     *steps_started = 0;
+    info[4] = 0;  // workgroups of k_predict_setup that have finished
   }
 }
 
@@ -165,8 +165,8 @@ __device__ __forceinline__ void for_each_key_group(bool want, int key, Fn&& fn) 
   }
 }
 
-__global__ __launch_bounds__(1024) void k_predict_bbox(
-    StepConsts c, const float4* __restrict__ pos, const float4* __restrict__ vel,
+__device__ __forceinline__ void predict_bbox(
+    const StepConsts& c, const float4* __restrict__ pos, const float4* __restrict__ vel,
     const ScenePlanes* __restrict__ sp, const int* __restrict__ seg,
     uint64_t* __restrict__ cellc, int* __restrict__ bbox, int* __restrict__ tile_bbox,
     unsigned* __restrict__ flags) {
@@ -248,21 +248,31 @@ __global__ __launch_bounds__(1024) void k_predict_bbox(
   }
 }
 
-// One workgroup of kGridSetupThreads: per-scene table extents and key
-// offsets; resets the per-step counters.
+// What the grid setup reads and writes besides the boxes.
+struct GridSetup {
+  int n_scenes;
+  const int* __restrict__ seg;
+  int tile_size;
+  GridDesc* __restrict__ grid;
+  int* __restrict__ total_cells;
+  long long cell_cap;
+  int bshift;
+  unsigned long long* __restrict__ nbr_total;
+  unsigned long long* __restrict__ need_cells;
+  int* __restrict__ steps_started;
+  int* __restrict__ tile_count;  // null without tiles
+  int* __restrict__ info;
+};
+
+// One workgroup: per-scene table extents and key offsets; resets the per-step
+// counters.
 constexpr int kGridSetupThreads = 1024;
-__global__ __launch_bounds__(kGridSetupThreads) void k_grid_setup(int n_scenes, const int* __restrict__ seg,
-                                                    const int* __restrict__ tile_bbox,
-                                                    int tile_size, int* __restrict__ bbox,
-                                                    GridDesc* __restrict__ grid,
-                                                    int* __restrict__ total_cells,
-                                                    long long cell_cap, int bshift,
-                                                    unsigned* __restrict__ flags,
-                                                    unsigned long long* __restrict__ nbr_total,
-                                                    unsigned long long* __restrict__ need_cells,
-                                                    int* __restrict__ steps_started,
-                                                    int* __restrict__ tile_count,
-                                                    int* __restrict__ info) {
+__device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_bbox, int* bbox,
+                                           unsigned* flags) {
+  const int n_scenes = gs.n_scenes, tile_size = gs.tile_size, bshift = gs.bshift;
+  const long long cell_cap = gs.cell_cap;
+  const int* __restrict__ seg = gs.seg;
+  GridDesc* __restrict__ grid = gs.grid;
   __shared__ long long sh[kGridSetupThreads];
   __shared__ long long carry;
   // After a failed substep the counters keep what the host needs to size
@@ -342,168 +352,122 @@ __global__ __launch_bounds__(kGridSetupThreads) void k_grid_setup(int n_scenes, 
     __syncthreads();
   }
   if (threadIdx.x == 0 && !was_fatal) {
-    *nbr_total = 0ull;
-    info[2] = 0;  // dense units
-    if (tile_count) {
-      tile_count[0] = 0;  // tiles
-      tile_count[1] = 0;  // candidate bricks
+    *gs.nbr_total = 0ull;
+    gs.info[2] = 0;  // dense units
+    if (gs.tile_count) {
+      gs.tile_count[0] = 0;  // tiles
+      gs.tile_count[1] = 0;  // candidate bricks
     }
     if (carry > cell_cap) {
       atomicOr(flags, kFlagCells);
-      *total_cells = 0;
-      *need_cells = static_cast<unsigned long long>(carry);
+      *gs.total_cells = 0;
+      *gs.need_cells = static_cast<unsigned long long>(carry);
     } else {
-      *total_cells = static_cast<int>(carry);
-      atomicAdd(steps_started, 1);
+      *gs.total_cells = static_cast<int>(carry);
+      atomicAdd(gs.steps_started, 1);
     }
   }
 }
 
+__global__ __launch_bounds__(1024) void k_predict_bbox(
+    StepConsts c, const float4* __restrict__ pos, const float4* __restrict__ vel,
+    const ScenePlanes* __restrict__ sp, const int* __restrict__ seg,
+    uint64_t* __restrict__ cellc, int* __restrict__ bbox, int* __restrict__ tile_bbox,
+    unsigned* __restrict__ flags) {
+  predict_bbox(c, pos, vel, sp, seg, cellc, bbox, tile_bbox, flags);
+}
 
-// Each particle's cell key, in the previous substep's slot order.
-__global__ __launch_bounds__(1024) void k_cell_keys(StepConsts c,
-                                                    const uint64_t* __restrict__ cellc,
-                                                    const int* __restrict__ seg,
-                                                    const GridDesc* __restrict__ grid,
-                                                    int* __restrict__ key,
-                                                    const unsigned* __restrict__ flags) {
-  const int i = tile_index(c.xcd_remap) * blockDim.x + threadIdx.x;
-  if (fatal(flags) || i >= c.n) return;
-  const GridDesc g = grid[scene_of(i, seg, c.n_scenes)];
+__global__ __launch_bounds__(kGridSetupThreads) void k_grid_setup(GridSetup gs,
+                                                                  const int* tile_bbox, int* bbox,
+                                                                  unsigned* flags) {
+  grid_setup(gs, tile_bbox, bbox, flags);
+}
+
+// Both in one launch: the workgroup that finishes last (a device counter,
+// which it clears again) sets the grid up from all workgroups' boxes.
+__global__ __launch_bounds__(1024) void k_predict_setup(
+    StepConsts c, GridSetup gs, const float4* __restrict__ pos, const float4* __restrict__ vel,
+    const ScenePlanes* __restrict__ sp, uint64_t* __restrict__ cellc, int* bbox, int* tile_bbox,
+    int* finished, unsigned* flags) {
+  __shared__ int last_sh;
+  predict_bbox(c, pos, vel, sp, gs.seg, cellc, bbox, tile_bbox, flags);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __threadfence();  // this workgroup's box before its count
+    last_sh = atomicAdd(finished, 1) == static_cast<int>(gridDim.x) - 1;
+    __threadfence();  // every workgroup's box after the last count
+  }
+  __syncthreads();
+  if (!last_sh) return;
+  if (threadIdx.x == 0) *finished = 0;
+  grid_setup(gs, tile_bbox, bbox, flags);
+}
+
+// The cell key of slot p of the previous substep's order.
+__device__ __forceinline__ int slot_cell_key(const StepConsts& c, int p,
+                                             const uint64_t* __restrict__ cellc,
+                                             const int* __restrict__ seg,
+                                             const GridDesc* __restrict__ grid) {
+  const GridDesc g = grid[scene_of(p, seg, c.n_scenes)];
   int x, y, z;
-  unpack_cell(cellc[i], x, y, z);
-  key[i] = cell_key(x - g.ox, y - g.oy, z - g.oz, g);
+  unpack_cell(cellc[p], x, y, z);
+  return cell_key(x - g.ox, y - g.oy, z - g.oz, g);
 }
 
-// The cell histogram from the sorted keys, where each cell's particles are
-// one run.  A run inside one wavefront stores its length; a run that crosses
-// a wavefront boundary adds each wavefront's part atomically.  A substep
-// thus takes about one atomic per wavefront instead of one per cell and
-// wavefront (device-scope atomics are carried out in memory on this
-// multi-XCD part).  The histogram is all zeros on entry: the scan that reads
-// it clears it.
-__global__ __launch_bounds__(1024) void k_cell_runs(int n, const int* __restrict__ sk,
-                                                    int* __restrict__ count,
-                                                    const unsigned* __restrict__ flags) {
-  if (fatal(flags)) return;  // uniform
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & (kWave - 1);
-  const bool active = s < n;
-  const int k = active ? sk[s] : 0;
-  const bool head = active && (s == 0 || sk[s - 1] != k);
-  const bool tail = active && (s == n - 1 || sk[s + 1] != k);
-  // segments: a run's slots within one wavefront; active lanes are a prefix
-  const unsigned long long starts = __ballot(active && (head || lane == 0));
-  const unsigned long long tails = __ballot(tail);
-  const int nact = __popcll(__ballot(active));
-  if (!active || ((starts >> lane) & 1ull) == 0ull) return;
-  const unsigned long long above = starts & ~((2ull << lane) - 1ull);
-  const int next = above != 0ull ? __builtin_ctzll(above) : nact;
-  const int len = next - lane;
-  if (head && ((tails >> (next - 1)) & 1ull) != 0ull)
-    count[k] = len;  // the whole run: its only writer
-  else
-    atomicAdd(count + k, len);
-}
+// ---- exclusive scan (fixed grid)
 
-// ---- exclusive scan over a device-sized array (three launches, fixed grid)
-
-// Exclusive scans of one array, or of two arrays of one length at once (in2
-// and out2 non-null), in two launches: k_scan_reduce writes each workgroup's
-// range sums to partial ([0, G) for in, [G, 2G) for in2), k_scan_down scans.
-__global__ __launch_bounds__(256) void k_scan_reduce(const int* __restrict__ in,
-                                                     const int* __restrict__ in2,
-                                                     const int* __restrict__ d_len,
+// In two launches: k_scan_reduce writes each workgroup's range sum to
+// partial, k_scan_down scans.
+__global__ __launch_bounds__(256) void k_scan_reduce(const int* __restrict__ in, int len,
                                                      int* __restrict__ partial,
                                                      const unsigned* __restrict__ flags) {
   __shared__ int lds[8];
   if (fatal(flags)) return;
-  const int len = *d_len;
   const int G = gridDim.x;
   const int chunk = (len + G - 1) / G;
   const int b0 = blockIdx.x * chunk;
   const int b1 = min(len, b0 + chunk);
-  int acc = 0, acc2 = 0;
-  for (int i = b0 + threadIdx.x; i < b1; i += blockDim.x) {
-    acc += in[i];
-    if (in2) acc2 += in2[i];
-  }
+  int acc = 0;
+  for (int i = b0 + threadIdx.x; i < b1; i += blockDim.x) acc += in[i];
   int total;
   block_excl_scan(acc, lds, &total);
   if (threadIdx.x == 0) partial[blockIdx.x] = total;
-  if (in2) {
-    block_excl_scan(acc2, lds, &total);
-    if (threadIdx.x == 0) partial[G + blockIdx.x] = total;
-  }
 }
 
-// Sum of the partials of the workgroups before this one (*pre) and of all
-// of them (*grand).
-__device__ __forceinline__ void partial_prefix(const int* __restrict__ partial, int G, int* lds,
-                                               int* pre, int* grand) {
-  int p = 0, a = 0;
-  for (int j = threadIdx.x; j < G; j += blockDim.x) {
-    const int v = partial[j];
-    a += v;
-    p += j < static_cast<int>(blockIdx.x) ? v : 0;
-  }
-  block_excl_scan(p, lds, pre);
-  block_excl_scan(a, lds, grand);
-}
-
-// out[i] = exclusive prefix; out[len] = grand total (and so for in2/out2).
-// zero_in clears `in` (the cell histogram is reused by the next substep).
-// Each workgroup first sums the partials of the workgroups before it, then
-// scans its own range, each thread taking four consecutive elements per
-// block scan.
-__global__ __launch_bounds__(256) void k_scan_down(int* __restrict__ in,
-                                                   const int* __restrict__ in2,
-                                                   const int* __restrict__ d_len,
+// out[i] = exclusive prefix.  Each workgroup first sums the partials of the
+// workgroups before it, then scans its own range, each thread taking four
+// consecutive elements per block scan.
+__global__ __launch_bounds__(256) void k_scan_down(const int* __restrict__ in, int len,
                                                    const int* __restrict__ partial,
-                                                   int* __restrict__ out, int* __restrict__ out2,
-                                                   int zero_in,
+                                                   int* __restrict__ out,
                                                    const unsigned* __restrict__ flags) {
   __shared__ int lds[8];
   if (fatal(flags)) return;
-  const int len = *d_len;
   const int G = gridDim.x;
   const int chunk = (len + G - 1) / G;
   const int b0 = blockIdx.x * chunk;
   const int b1 = min(len, b0 + chunk);
-  int run, grand, run2 = 0, grand2 = 0;
-  partial_prefix(partial, G, lds, &run, &grand);
-  if (in2) partial_prefix(partial + G, G, lds, &run2, &grand2);
+  int run, p = 0;
+  for (int j = threadIdx.x; j < static_cast<int>(blockIdx.x); j += blockDim.x) p += partial[j];
+  block_excl_scan(p, lds, &run);
   constexpr int kPer = 4;
   for (int t0 = b0; t0 < b1; t0 += kPer * static_cast<int>(blockDim.x)) {
     const int i0 = t0 + kPer * static_cast<int>(threadIdx.x);
-    int v[kPer], w[kPer];
-    int sum = 0, sum2 = 0;
+    int v[kPer];
+    int sum = 0;
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
       v[q] = (i0 + q < b1) ? in[i0 + q] : 0;
-      w[q] = (in2 && i0 + q < b1) ? in2[i0 + q] : 0;
       sum += v[q];
-      sum2 += w[q];
     }
-    int total, total2 = 0;
+    int total;
     int e = run + block_excl_scan(sum, lds, &total);
-    int e2 = in2 ? run2 + block_excl_scan(sum2, lds, &total2) : 0;
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
-      if (i0 + q < b1) {
-        out[i0 + q] = e;
-        if (zero_in) in[i0 + q] = 0;
-        if (in2) out2[i0 + q] = e2;
-      }
+      if (i0 + q < b1) out[i0 + q] = e;
       e += v[q];
-      e2 += w[q];
     }
     run += total;
-    run2 += total2;
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    out[len] = grand;
-    if (in2) out2[len] = grand2;
   }
 }
 
@@ -515,10 +479,12 @@ __global__ __launch_bounds__(256) void k_scan_down(int* __restrict__ in,
 // of the histogram in digit-major order, and a stable scatter.
 
 // Keys and values in original-id order: k[id] = cell key, v[id] = slot.
-__global__ __launch_bounds__(1024) void k_sort_keys(StepConsts c, const float4* __restrict__ pos,
-                                                    const int* __restrict__ key,
-                                                    int* __restrict__ kout, int* __restrict__ vout,
-                                                    unsigned* __restrict__ flags) {
+__global__ __launch_bounds__(256) void k_sort_keys(StepConsts c, const float4* __restrict__ pos,
+                                                   const uint64_t* __restrict__ cellc,
+                                                   const int* __restrict__ seg,
+                                                   const GridDesc* __restrict__ grid,
+                                                   int* __restrict__ kout, int* __restrict__ vout,
+                                                   unsigned* __restrict__ flags) {
   if (fatal(flags)) return;
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= c.n) return;
@@ -527,7 +493,7 @@ __global__ __launch_bounds__(1024) void k_sort_keys(StepConsts c, const float4* 
     atomicOr(flags, kFlagRange);
     return;
   }
-  kout[id] = key[p];
+  kout[id] = slot_cell_key(c, p, cellc, seg, grid);
   vout[id] = p;
 }
 
@@ -538,9 +504,10 @@ __device__ __forceinline__ bool pass_is_identity(const int* total_cells, int shi
   return static_cast<long long>(*total_cells) <= (1ll << shift);
 }
 
-// hist[d * G + b]: items of workgroup b (kRadixTile of them) with digit d.
+// Items of each workgroup (kRadixTile of them) per digit: hist[d * G + b] for
+// the scan, or with `rows` hist[b * 256 + d] for the scatter's own sums.
 __global__ __launch_bounds__(256) void k_radix_hist(int n, const int* __restrict__ kin, int shift,
-                                                    int* __restrict__ hist,
+                                                    int* __restrict__ hist, int rows,
                                                     const int* __restrict__ total_cells,
                                                     const unsigned* __restrict__ flags) {
   __shared__ int h[256];
@@ -552,21 +519,38 @@ __global__ __launch_bounds__(256) void k_radix_hist(int n, const int* __restrict
   for (int i = b0 + static_cast<int>(threadIdx.x); i < b1; i += 256)
     atomicAdd(&h[(kin[i] >> shift) & 255], 1);
   __syncthreads();
-  hist[threadIdx.x * gridDim.x + blockIdx.x] = h[threadIdx.x];
+  hist[rows ? blockIdx.x * 256 + threadIdx.x : threadIdx.x * gridDim.x + blockIdx.x] =
+      h[threadIdx.x];
+}
+
+// The lanes among `ok` whose digit equals this lane's.
+__device__ __forceinline__ unsigned long long digit_peers(int d, bool ok) {
+  unsigned long long peers = __ballot(ok);
+#pragma unroll
+  for (int bit = 0; bit < 8; ++bit) {
+    const bool x = (d >> bit) & 1;
+    const unsigned long long bb = __ballot(x);
+    peers &= x ? bb : ~bb;
+  }
+  return ok ? peers : 0ull;
 }
 
 // Stable scatter of one pass: the workgroup's items in index order, 256 per
 // round; an item goes to its digit's offset for this workgroup, plus the
 // items of that digit in earlier rounds, earlier wavefronts and lower lanes.
+// The offsets come from the scanned histogram, or with `hist` (up to
+// kRowScatter workgroups) each workgroup sums the histogram's rows itself.
 __global__ __launch_bounds__(256) void k_radix_scatter(int n, const int* __restrict__ kin,
                                                        const int* __restrict__ vin,
                                                        int* __restrict__ kout,
                                                        int* __restrict__ vout, int shift,
                                                        const int* __restrict__ off,
+                                                       const int* __restrict__ hist,
                                                        const int* __restrict__ total_cells,
                                                        const unsigned* __restrict__ flags) {
   __shared__ int run[256];      // per digit: where the next item of this workgroup goes
   __shared__ int wcnt[4][256];  // per wavefront of the round: items per digit
+  __shared__ int scan_lds[8];
   if (fatal(flags)) return;
   const int tid = threadIdx.x;
   if (pass_is_identity(total_cells, shift)) {
@@ -579,21 +563,26 @@ __global__ __launch_bounds__(256) void k_radix_scatter(int n, const int* __restr
   }
   const int lane = tid & (kWave - 1);
   const int w = tid >> 6;
-  run[tid] = off[tid * gridDim.x + blockIdx.x];
+  if (hist) {
+    int before = 0, total = 0;
+#pragma unroll 8
+    for (int b = 0; b < static_cast<int>(gridDim.x); ++b) {
+      const int v = hist[b * 256 + tid];
+      total += v;
+      before += b < static_cast<int>(blockIdx.x) ? v : 0;
+    }
+    int all;
+    run[tid] = block_excl_scan(total, scan_lds, &all) + before;
+  } else {
+    run[tid] = off[tid * gridDim.x + blockIdx.x];
+  }
   const int b0 = blockIdx.x * kRadixTile;
   for (int r = 0; r < kRadixTile / 256; ++r) {
     const int i = b0 + r * 256 + tid;
     const bool ok = i < n;
     const int kk = ok ? kin[i] : 0;
     const int d = (kk >> shift) & 255;
-    // the lanes of this wavefront with the same digit
-    unsigned long long peers = __ballot(ok);
-    for (int bit = 0; bit < 8; ++bit) {
-      const bool x = (d >> bit) & 1;
-      const unsigned long long bb = __ballot(x);
-      peers &= x ? bb : ~bb;
-    }
-    if (!ok) peers = 0ull;
+    const unsigned long long peers = digit_peers(d, ok);
     const int below = __popcll(peers & ((1ull << lane) - 1ull));
     for (int v = 0; v < 4; ++v) wcnt[v][tid] = 0;
     __syncthreads();
@@ -613,17 +602,123 @@ __global__ __launch_bounds__(256) void k_radix_scatter(int n, const int* __restr
   }
 }
 
-// Gathers each particle into its slot of the (cell, id) order (sv: the
-// sorted previous slots, sk: their cell keys) and recomputes pred there.
-__global__ __launch_bounds__(1024) void k_reorder(
-    StepConsts c, const int* __restrict__ sk, const int* __restrict__ sv,
+// The whole sort of a batch of up to kSmallSort particles in one workgroup:
+// keys in original-id order in LDS, then as many stable 8-bit passes as the
+// table's size has digits.  A wavefront ranks its consecutive items 64 at a
+// time against its own digit counts (no barrier inside a pass but for the two
+// around the scan of the counts).  Replaces k_sort_keys and two launches per
+// pass, each of which takes about 4 us whatever its size: 2,431 particles 32
+// -> 9 us.
+__global__ __launch_bounds__(1024) void k_small_sort(
+    StepConsts c, const float4* __restrict__ pos, const uint64_t* __restrict__ cellc,
+    const int* __restrict__ seg, const GridDesc* __restrict__ grid,
+    const int* __restrict__ total_cells, int* __restrict__ kout, int* __restrict__ vout,
+    unsigned* __restrict__ flags) {
+  constexpr int kT = 1024, kW = kT / kWave, kR = kSmallSort / kT;
+  __shared__ int key[kSmallSort];
+  __shared__ unsigned short val[kSmallSort];
+  __shared__ unsigned short cnt[kW][256];
+  __shared__ int dbase[256];
+  __shared__ int scan_lds[kW + 1];
+  __shared__ int stop;
+  if (threadIdx.x == 0) stop = fatal(flags) ? 1 : 0;
+  __syncthreads();
+  if (stop) return;
+  const int n = c.n, tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+  for (int p = tid; p < n; p += kT) {
+    const int id = __float_as_int(reinterpret_cast<const float*>(pos + p)[3]);
+    if (id < 0 || id >= n) {  // ids are 0..n-1; refuse rather than write outside
+      atomicOr(flags, kFlagRange);
+      continue;
+    }
+    key[id] = slot_cell_key(c, p, cellc, seg, grid);
+    val[id] = static_cast<unsigned short>(p);
+  }
+  __syncthreads();
+  const int rounds = (n + kT - 1) / kT;
+  const int last = *total_cells - 1;
+  for (int shift = 0; shift < 31 && (last >> shift) > 0; shift += 8) {
+    int kk[kR], rank[kR];
+    unsigned short vv[kR];
+    for (int i = lane; i < 256; i += kWave) cnt[w][i] = 0;
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+      if (r < rounds) {
+        const int i = (w * rounds + r) * kWave + lane;
+        const bool ok = i < n;
+        kk[r] = ok ? key[i] : 0;
+        vv[r] = ok ? val[i] : 0;
+        const int d = (kk[r] >> shift) & 255;
+        const unsigned long long peers = digit_peers(d, ok);
+        const int below = __popcll(peers & ((1ull << lane) - 1ull));
+        const int before = cnt[w][d];
+        rank[r] = before + below;
+        // a wavefront's LDS accesses complete in order
+        if (ok && below == 0)
+          cnt[w][d] = static_cast<unsigned short>(before + __popcll(peers));
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+    __syncthreads();
+    int total = 0;
+    if (tid < 256)
+      for (int v = 0; v < kW; ++v) {
+        const int x = cnt[v][tid];
+        cnt[v][tid] = static_cast<unsigned short>(total);
+        total += x;
+      }
+    int all;
+    const int excl = block_excl_scan(total, scan_lds, &all);
+    if (tid < 256) dbase[tid] = excl;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+      if (r < rounds) {
+        const int i = (w * rounds + r) * kWave + lane;
+        const int d = (kk[r] >> shift) & 255;
+        const int at = dbase[d] + cnt[w][d] + rank[r];
+        if (i < n && at < n) {  // always at < n, as the counts are of these items
+          key[at] = kk[r];
+          val[at] = vv[r];
+        }
+      }
+    }
+    __syncthreads();
+  }
+  for (int i = tid; i < n; i += kT) {
+    kout[i] = key[i];
+    vout[i] = val[i];
+  }
+}
+
+// First index in the sorted sk[0, n) whose key is not below `target`: a
+// wavefront probes 64 places at a time.
+__device__ __forceinline__ int lower_bound64(const int* __restrict__ sk, int n, int target) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int lo = 0, hi = n;
+  while (lo < hi) {
+    const int step = (hi - lo + kWave - 1) / kWave;
+    const int i = lo + lane * step;
+    const int less = __popcll(__ballot(i < hi && sk[i] < target));
+    if (less == 0) return lo;
+    hi = min(hi, lo + less * step);
+    lo += (less - 1) * step + 1;
+  }
+  return lo;
+}
+
+// Cells a workgroup of k_table fills at a time.
+constexpr int kTableCells = 4096;
+
+// Gathers the particle of slot dest of the (cell, id) order (sv: the sorted
+// previous slots, sk: their cell keys) and recomputes pred there.
+__device__ __forceinline__ void reorder_slot(
+    const StepConsts& c, int dest, const int* __restrict__ sk, const int* __restrict__ sv,
     const int* __restrict__ seg, const ScenePlanes* __restrict__ sp,
     const float4* __restrict__ posA, const float4* __restrict__ velA, float4* __restrict__ posB,
     float4* __restrict__ velB, float4* __restrict__ pred, const uint64_t* __restrict__ cellc,
     uint64_t* __restrict__ slot_cell, int* __restrict__ slot_key,
     unsigned* __restrict__ flags) {
-  if (fatal(flags)) return;
-  const int dest = blockIdx.x * blockDim.x + threadIdx.x;
   if (dest >= c.n) return;
   const int p = sv[dest];
   if (p < 0 || p >= c.n) {  // never for a complete sort; refuse rather than read outside
@@ -642,6 +737,95 @@ __global__ __launch_bounds__(1024) void k_reorder(
   pred[dest] = make_float4(x.x + vx * c.dt, x.y + vy * c.dt, x.z + vz * c.dt, 0.0f);
   slot_cell[dest] = cellc[p];
   slot_key[dest] = sk[dest];
+}
+
+// The first `reorder_blocks` workgroups gather the particles into their slots;
+// the others write the cell table, start[k] = first slot of cell k, straight
+// from the sorted keys, kTableCells cells at a time: two searches give the
+// cells' slots, whose runs' heads set their cells' starts in LDS, and a suffix
+// minimum gives an empty cell the next cell's start.  The table is written
+// once; its histogram, scanned and cleared in three launches before, moved
+// four times as much: the 256-scene ensemble's table of 44 M cells took 270
+// us and takes 60, small batches save two launches.
+__global__ __launch_bounds__(256) void k_table(
+    StepConsts c, const int* __restrict__ sk, const int* __restrict__ sv,
+    const int* __restrict__ seg, const ScenePlanes* __restrict__ sp,
+    const float4* __restrict__ posA, const float4* __restrict__ velA, float4* __restrict__ posB,
+    float4* __restrict__ velB, float4* __restrict__ pred, const uint64_t* __restrict__ cellc,
+    uint64_t* __restrict__ slot_cell, int* __restrict__ slot_key, int reorder_blocks,
+    const int* __restrict__ total_cells, int* __restrict__ start,
+    unsigned* __restrict__ flags) {
+  constexpr int kPer = kTableCells / 256;
+  __shared__ __align__(16) int first[kTableCells];
+  __shared__ int range[2];
+  __shared__ int wmin[4];
+  if (fatal(flags)) return;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+  if (static_cast<int>(blockIdx.x) < reorder_blocks) {
+    reorder_slot(c, blockIdx.x * 256 + tid, sk, sv, seg, sp, posA, velA, posB, velB, pred, cellc,
+                 slot_cell, slot_key, flags);
+    return;
+  }
+  const int total = *total_cells;
+  const int blocks = static_cast<int>(gridDim.x) - reorder_blocks;
+  for (long long q = static_cast<int>(blockIdx.x) - reorder_blocks; q * kTableCells < total;
+       q += blocks) {
+    const int c0 = static_cast<int>(q) * kTableCells;
+    const int m = min(kTableCells, total - c0);
+    if (w < 2) {
+      // (the last cells' end: every key lies below the table's size)
+      const int at = w == 1 && c0 + m == total ? c.n : lower_bound64(sk, c.n, c0 + w * m);
+      if (lane == 0) range[w] = at;
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) first[i * 256 + tid] = INT_MAX;
+    __syncthreads();
+    const int lo = range[0], hi = range[1];
+    for (int i = lo + tid; i < hi; i += 256) {
+      const int k = sk[i];
+      if (i == lo || sk[i - 1] != k) first[k - c0] = i;
+    }
+    __syncthreads();
+    int v[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; i += 4) {
+      const int4 x = *reinterpret_cast<const int4*>(first + tid * kPer + i);
+      v[i] = x.x;
+      v[i + 1] = x.y;
+      v[i + 2] = x.z;
+      v[i + 3] = x.w;
+    }
+#pragma unroll
+    for (int i = kPer - 2; i >= 0; --i) v[i] = min(v[i], v[i + 1]);
+    // the least start in the cells of the threads after this one, else hi
+    int suf = v[0];
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int u = __shfl_down(suf, o, kWave);
+      if (lane + o < kWave) suf = min(suf, u);
+    }
+    if (lane == 0) wmin[w] = suf;
+    int after = __shfl_down(suf, 1, kWave);
+    if (lane == kWave - 1) after = INT_MAX;
+    __syncthreads();
+    for (int u = w + 1; u < 4; ++u) after = min(after, wmin[u]);
+    after = min(after, hi);
+    int* out = start + c0 + tid * kPer;
+#pragma unroll
+    for (int i = 0; i < kPer; i += 4) {
+      const int4 x = make_int4(min(v[i], after), min(v[i + 1], after), min(v[i + 2], after),
+                               min(v[i + 3], after));
+      const int at = tid * kPer + i;
+      if (at + 4 <= m) {
+        *reinterpret_cast<int4*>(out + i) = x;
+      } else {
+        if (at < m) out[i] = x.x;
+        if (at + 1 < m) out[i + 1] = x.y;
+        if (at + 2 < m) out[i + 2] = x.z;
+      }
+    }
+    if (tid == 0 && c0 + m == total) start[total] = c.n;
+    __syncthreads();  // LDS is reused
+  }
 }
 
 // ---------------------------------------------------------------- launching
@@ -685,7 +869,7 @@ inline int blocks_for(long long n, int bs) { return static_cast<int>((n + bs - 1
 }  // namespace
 
 hipError_t enqueue_reset_flags(Ctx& c) {
-  k_reset_flags<<<1, 64, 0, c.stream>>>(c.flags, c.steps_started);
+  k_reset_flags<<<1, 64, 0, c.stream>>>(c.flags, c.steps_started, c.info);
   return hipGetLastError();
 }
 
@@ -705,6 +889,14 @@ hipError_t enqueue_download(Ctx& c, float* d_pos, float* d_vel) {
   k_download<<<blocks_for(c.n, 256), 256, 0, c.stream>>>(c.n, c.posA, c.velA, d_pos, d_vel);
   return hipGetLastError();
 }
+
+// Batches of up to this many particles fuse the prediction and the grid setup.
+constexpr int kFusedSetup = 1 << 16;
+// Workgroups of the radix sort up to which each sums the digit counts of the
+// others itself (a chain of 64 loads a digit, about what two launches take).
+constexpr int kRowScatter = 64;
+// Workgroups of k_table that write the cell table.
+constexpr int kTableGrid = 2048;
 
 hipError_t enqueue_substep(Ctx& c, const SubstepRec* rec) {
   if (c.n == 0) return hipSuccess;
@@ -740,53 +932,64 @@ hipError_t enqueue_substep(Ctx& c, const SubstepRec* rec) {
     if (e != hipSuccess) return e;     \
   } while (0)
 
-  FH_TRY(L("predict_bbox", [&] {
-    k_predict_bbox<<<nb, bs, 0, st>>>(k, c.posA, c.velA, c.planes, c.seg, c.cellc, c.bbox,
-                                      c.tile_bbox, c.flags);
-  }));
-  FH_TRY(L("grid_setup", [&] {
-    k_grid_setup<<<1, kGridSetupThreads, 0, st>>>(c.n_scenes, c.seg, c.tile_bbox, bs, c.bbox, c.grid,
-                                    c.total_cells, c.cell_cap, c.brick_shift,
-                                    c.flags, c.nbr_total, c.need_cells, c.steps_started,
-                                    tiles ? c.tile_count : nullptr, c.info);
-  }));
-  FH_TRY(L("cell_keys", [&] {
-    k_cell_keys<<<nb, bs, 0, st>>>(k, c.cellc, c.seg, c.grid, c.key, c.flags);
-  }));
+  const GridSetup gs{c.n_scenes,    c.seg,        bs,           c.grid,
+                     c.total_cells, c.cell_cap,   c.brick_shift, c.nbr_total,
+                     c.need_cells,  c.steps_started, tiles ? c.tile_count : nullptr, c.info};
+  // A small batch's launches take about 4 us each, whatever they do: one less.
+  // (In a large one the workgroups' fences cost more, and many scenes' boxes
+  // are folded by 1,024 threads.)
+  const bool fused_setup = c.n <= kFusedSetup && c.n_scenes <= 16;
+  if (fused_setup) {
+    FH_TRY(L("predict_bbox", [&] {
+      k_predict_setup<<<nb, bs, 0, st>>>(k, gs, c.posA, c.velA, c.planes, c.cellc, c.bbox,
+                                         c.tile_bbox, c.info + 4, c.flags);
+    }));
+  } else {
+    FH_TRY(L("predict_bbox", [&] {
+      k_predict_bbox<<<nb, bs, 0, st>>>(k, c.posA, c.velA, c.planes, c.seg, c.cellc, c.bbox,
+                                        c.tile_bbox, c.flags);
+    }));
+    FH_TRY(L("grid_setup", [&] {
+      k_grid_setup<<<1, kGridSetupThreads, 0, st>>>(gs, c.tile_bbox, c.bbox, c.flags);
+    }));
+  }
   // keys lie below the cell table's capacity: 8 bits per pass
   int key_bits = 1;
   while (key_bits < 31 && (1ll << key_bits) < c.cell_cap) ++key_bits;
   const int passes = (key_bits + 7) / 8;
+  int sorted = passes & 1;  // which buffers end up sorted
   FH_TRY(L("sort", [&] {
-    k_sort_keys<<<blocks_for(c.n, 256), 256, 0, st>>>(k, c.posA, c.key, c.sort_k[0],
-                                                       c.sort_v[0], c.flags);
+    if (c.n <= kSmallSort) {
+      sorted = 0;
+      k_small_sort<<<1, 1024, 0, st>>>(k, c.posA, c.cellc, c.seg, c.grid, c.total_cells,
+                                       c.sort_k[0], c.sort_v[0], c.flags);
+      return;
+    }
+    k_sort_keys<<<blocks_for(c.n, 256), 256, 0, st>>>(k, c.posA, c.cellc, c.seg, c.grid,
+                                                      c.sort_k[0], c.sort_v[0], c.flags);
+    const bool rows = c.radix_blocks <= kRowScatter;
+    const int len = 256 * c.radix_blocks;
     for (int q = 0; q < passes; ++q) {
       const int i = q & 1, o = i ^ 1;
       k_radix_hist<<<c.radix_blocks, 256, 0, st>>>(c.n, c.sort_k[i], 8 * q, c.radix_hist,
-                                                   c.total_cells, c.flags);
-      k_scan_reduce<<<c.scan_blocks, 256, 0, st>>>(c.radix_hist, nullptr, c.radix_len,
-                                                   c.scan_partial, c.flags);
-      k_scan_down<<<c.scan_blocks, 256, 0, st>>>(c.radix_hist, nullptr, c.radix_len,
-                                                 c.scan_partial, c.radix_off, nullptr, 0,
-                                                 c.flags);
-      k_radix_scatter<<<c.radix_blocks, 256, 0, st>>>(c.n, c.sort_k[i], c.sort_v[i], c.sort_k[o],
-                                                      c.sort_v[o], 8 * q, c.radix_off,
-                                                      c.total_cells, c.flags);
+                                                   rows ? 1 : 0, c.total_cells, c.flags);
+      if (!rows) {
+        k_scan_reduce<<<c.scan_blocks, 256, 0, st>>>(c.radix_hist, len, c.scan_partial, c.flags);
+        k_scan_down<<<c.scan_blocks, 256, 0, st>>>(c.radix_hist, len, c.scan_partial,
+                                                   c.radix_off, c.flags);
+      }
+      k_radix_scatter<<<c.radix_blocks, 256, 0, st>>>(
+          c.n, c.sort_k[i], c.sort_v[i], c.sort_k[o], c.sort_v[o], 8 * q, c.radix_off,
+          rows ? c.radix_hist : nullptr, c.total_cells, c.flags);
     }
   }));
-  FH_TRY(L("cell_count", [&] {
-    // the histogram of the sorted keys and its scan: each cell's first slot
-    k_cell_runs<<<blocks_for(c.n, 1024), 1024, 0, st>>>(c.n, c.sort_k[passes & 1], c.count,
-                                                        c.flags);
-    k_scan_reduce<<<c.scan_blocks, 256, 0, st>>>(c.count, nullptr, c.total_cells,
-                                                 c.scan_partial, c.flags);
-    k_scan_down<<<c.scan_blocks, 256, 0, st>>>(c.count, nullptr, c.total_cells, c.scan_partial,
-                                               c.start, nullptr, 1, c.flags);
-  }));
   FH_TRY(L("reorder", [&] {
-    k_reorder<<<nb, bs, 0, st>>>(k, c.sort_k[passes & 1], c.sort_v[passes & 1], c.seg, c.planes,
-                                 c.posA, c.velA, c.posB, c.velB, PK(0), c.cellc, c.slot_cell,
-                                 c.slot_key, c.flags);
+    const int rb = blocks_for(c.n, 256);
+    const int tb = static_cast<int>(
+        std::min<long long>(kTableGrid, (c.cell_cap + kTableCells - 1) / kTableCells));
+    k_table<<<rb + tb, 256, 0, st>>>(k, c.sort_k[sorted], c.sort_v[sorted], c.seg, c.planes,
+                                     c.posA, c.velA, c.posB, c.velB, PK(0), c.cellc, c.slot_cell,
+                                     c.slot_key, rb, c.total_cells, c.start, c.flags);
   }));
   // Each pass's tile kernel runs on the side stream beside the heads' kernel
   // on the main stream: they write disjoint slots (a run lies in one cell,
