@@ -191,8 +191,7 @@ void compute_consts_of(Ctx& c, const fluid_hip_params* params, int n_scenes) {
   k.xcd_remap = c.xcd_remap;
   k.runs = (c.wave_mode == 2 && !c.record_diag) ? 1 : 0;
   k.full_lists = (c.record_diag || c.wave_mode == 1) ? 1 : 0;
-  // tile mode 0 (default) tiles from kTileAutoMinParticles particles: below
-  // that a substep is bound by launches, to which the tile kernels add
+  // tile mode 0 (default) tiles from kTileAutoMinParticles particles on
   const bool tile_mode = c.tile_gather == 1 || (c.tile_gather == 0 && c.n >= fluidhip::kTileAutoMinParticles);
   k.tiles = (k.runs && c.brick_shift == 2 && tile_mode && p.solver_iterations > 0 &&
              tile_terms_exact(h, h2, k.min_r2))

@@ -114,14 +114,16 @@ __device__ __forceinline__ int slot_class(const StepConsts& c, int s,
                                           const int* __restrict__ slot_key,
                                           const int* __restrict__ start,
                                           const int* __restrict__ in_tile) {
-  const int k = slot_key[s];
-  bool head = !c.runs || s == 0 || slot_key[s - 1] != k;
-  if (!head)
-    head = !same_bits3(ld3(posB, s), ld3(posB, s - 1)) || !same_bits3(ld3(velB, s), ld3(velB, s - 1));
-  if (!head) return 0;
-  if (in_tile && in_tile[s]) return kHead;
-  const int a = start[k];
-  if (start[k + 1] - a < kDenseCell) return kHead | kList;
+  // every load is issued before any test
+  const int before = max(s - 1, 0);
+  const int k = slot_key[s], kb = slot_key[before];
+  const float3 x = ld3(posB, s), xb = ld3(posB, before);
+  const float3 v = ld3(velB, s), vb = ld3(velB, before);
+  const int tile = in_tile ? in_tile[s] : 0;
+  const int a = start[k], b = start[k + 1];
+  if (c.runs && s > 0 && k == kb && same_bits3(x, xb) && same_bits3(v, vb)) return 0;
+  if (tile) return kHead;
+  if (b - a < kDenseCell) return kHead | kList;
   return s == a ? kHead | kDense | kCell : kHead | kDense;
 }
 

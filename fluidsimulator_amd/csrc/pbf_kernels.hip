@@ -267,25 +267,31 @@ struct GridSetup {
 // One workgroup: per-scene table extents and key offsets; resets the per-step
 // counters.
 constexpr int kGridSetupThreads = 1024;
+constexpr int kLocalBoxes = 64;  // scenes whose boxes are folded in LDS
 __device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_bbox, int* bbox,
                                            unsigned* flags) {
   const int n_scenes = gs.n_scenes, tile_size = gs.tile_size, bshift = gs.bshift;
   const long long cell_cap = gs.cell_cap;
   const int* __restrict__ seg = gs.seg;
   GridDesc* __restrict__ grid = gs.grid;
-  __shared__ long long sh[kGridSetupThreads];
-  __shared__ long long carry;
+  __shared__ long long sh[kGridSetupThreads / kWave];
+  __shared__ int box[6 * kLocalBoxes];
+  long long carry = 0;
   // After a failed substep the counters keep what the host needs to size
   // the retry; only the bounding boxes are reset.
   const bool was_fatal = (*flags & kFlagFatal) != 0u;
-  if (threadIdx.x == 0) carry = 0;
   // Fold each scene's tile partials into its box (which already holds the
   // atomics of tiles that straddle two scenes): `per` wavefronts per scene,
-  // each folding every per-th stretch of 64 tiles.
+  // each folding every per-th stretch of 64 tiles; with one wavefront or a few
+  // per scene, through LDS.
+  const int lane = threadIdx.x & (kWave - 1);
+  const int nw = static_cast<int>(blockDim.x) / kWave;
+  const int w = static_cast<int>(threadIdx.x) / kWave;
+  const bool local = n_scenes <= kLocalBoxes;
+  if (local)
+    for (int i = threadIdx.x; i < 6 * n_scenes; i += blockDim.x) box[i] = bbox[i];
+  __syncthreads();
   {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int nw = static_cast<int>(blockDim.x) / kWave;
-    const int w = static_cast<int>(threadIdx.x) / kWave;
     const int per = n_scenes >= nw ? 1 : nw / n_scenes;
     for (int sc = w / per; sc < n_scenes; sc += nw / per) {
       const int a = seg[sc], b = seg[sc + 1];
@@ -301,7 +307,7 @@ __device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_
       for (int k = 0; k < 3; ++k) v[k] = wave_min(v[k]);
       for (int k = 3; k < 6; ++k) v[k] = wave_max(v[k]);
       if (lane == 0) {
-        int* bb = bbox + 6 * sc;
+        int* bb = (local ? box : bbox) + 6 * sc;
         for (int k = 0; k < 3; ++k) atomicMin(bb + k, v[k]);
         for (int k = 3; k < 6; ++k) atomicMax(bb + k, v[k]);
       }
@@ -313,9 +319,9 @@ __device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_
     long long nc = 0;
     GridDesc g{};
     if (s < n_scenes) {
-      int* bb = bbox + 6 * s;
-      const long long lx = bb[0], ly = bb[1], lz = bb[2];
-      const long long hx = bb[3], hy = bb[4], hz = bb[5];
+      const int* from = (local ? box : bbox) + 6 * s;
+      const long long lx = from[0], ly = from[1], lz = from[2];
+      const long long hx = from[3], hy = from[4], hz = from[5];
       if (lx <= hx && ly <= hy && lz <= hz) {
         const long long sx = hx - lx + 3, sy = hy - ly + 3, sz = hz - lz + 3;
         const long long e = 1ll << bshift;
@@ -329,27 +335,31 @@ __device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_
         g.nbz = static_cast<int>(bz);
       }
       g.bshift = bshift;
+      int* bb = bbox + 6 * s;
       bb[0] = INT_MAX, bb[1] = INT_MAX, bb[2] = INT_MAX;
       bb[3] = INT_MIN, bb[4] = INT_MIN, bb[5] = INT_MIN;
     }
     // exclusive scan of nc over the workgroup
-    sh[threadIdx.x] = nc;
-    __syncthreads();
-    for (int o = 1; o < static_cast<int>(blockDim.x); o <<= 1) {
-      const long long t = (threadIdx.x >= static_cast<unsigned>(o)) ? sh[threadIdx.x - o] : 0;
-      __syncthreads();
-      sh[threadIdx.x] += t;
-      __syncthreads();
+    long long inc = nc;
+    for (int o = 1; o < kWave; o <<= 1) {
+      const long long u = __shfl_up(inc, o, kWave);
+      if (lane >= o) inc += u;
     }
-    const long long excl = sh[threadIdx.x] - nc + carry;
+    if (lane == kWave - 1) sh[w] = inc;
+    __syncthreads();
+    long long before = 0, all = 0;
+    for (int u = 0; u < nw; ++u) {
+      before += u < w ? sh[u] : 0;
+      all += sh[u];
+    }
+    const long long excl = inc - nc + before + carry;
     if (s < n_scenes) {
       g.cell_off = static_cast<int>(excl < cell_cap ? excl : 0);
       g.ncells = static_cast<int>(nc < cell_cap ? nc : 0);
       grid[s] = g;
     }
-    __syncthreads();
-    if (threadIdx.x == blockDim.x - 1) carry += sh[threadIdx.x];
-    __syncthreads();
+    carry += all;
+    __syncthreads();  // sh is reused
   }
   if (threadIdx.x == 0 && !was_fatal) {
     *gs.nbr_total = 0ull;
@@ -707,8 +717,10 @@ __device__ __forceinline__ int lower_bound64(const int* __restrict__ sk, int n, 
   return lo;
 }
 
-// Cells a workgroup of k_table fills at a time.
-constexpr int kTableCells = 4096;
+// Cells a workgroup of k_table fills at a time: kTableCells of a sparse table,
+// kTableDense of one with fewer than kTableSparse cells per particle (whose
+// ranges hold more keys to read).
+constexpr int kTableCells = 4096, kTableDense = 512, kTableSparse = 8;
 
 // Gathers the particle of slot dest of the (cell, id) order (sv: the sorted
 // previous slots, sk: their cell keys) and recomputes pred there.
@@ -739,14 +751,83 @@ __device__ __forceinline__ void reorder_slot(
   slot_key[dest] = sk[dest];
 }
 
+// Writes start[c0 .. c0 + m), m <= 256 kPer, from the sorted keys: two searches
+// give the cells' slots, whose runs' heads set their cells' starts in LDS, and a
+// suffix minimum gives an empty cell the next cell's start.
+template <int kPer>
+__device__ __forceinline__ void table_range(int n, const int* __restrict__ sk, int c0, int m,
+                                            int total, int* first, int* range, int* wmin,
+                                            int* __restrict__ start) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+  if (w < 2) {
+    // (the last cells' end: every key lies below the table's size)
+    const int at = w == 1 && c0 + m == total ? n : lower_bound64(sk, n, c0 + w * m);
+    if (lane == 0) range[w] = at;
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) first[i * 256 + tid] = INT_MAX;
+  __syncthreads();
+  const int lo = range[0], hi = range[1];
+  for (int i0 = lo; i0 < hi;) {
+    int k[4], before[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = min(i0 + q * 256 + tid, hi - 1);
+      k[q] = sk[i];
+      before[q] = sk[max(i - 1, 0)];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = i0 + q * 256 + tid;
+      if (i < hi && (i == lo || before[q] != k[q])) first[k[q] - c0] = i;
+    }
+    i0 += 1024;
+    // a pile of particles in one cell: on to the next cell's first
+    if (i0 + 8192 < hi) {
+      const int pile = sk[i0 - 1];
+      if (sk[i0 + 8192] == pile) {
+        __syncthreads();
+        if (w == 0) {
+          const int at = lower_bound64(sk, n, pile + 1);
+          if (lane == 0) range[1] = at;
+        }
+        __syncthreads();
+        i0 = range[1];
+      }
+    }
+  }
+  __syncthreads();
+  int v[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) v[i] = first[tid * kPer + i];
+#pragma unroll
+  for (int i = kPer - 2; i >= 0; --i) v[i] = min(v[i], v[i + 1]);
+  // the least start in the cells of the threads after this one, else hi
+  int suf = v[0];
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int u = __shfl_down(suf, o, kWave);
+    if (lane + o < kWave) suf = min(suf, u);
+  }
+  if (lane == 0) wmin[w] = suf;
+  int after = __shfl_down(suf, 1, kWave);
+  if (lane == kWave - 1) after = INT_MAX;
+  __syncthreads();
+  for (int u = w + 1; u < 4; ++u) after = min(after, wmin[u]);
+  after = min(after, hi);
+  int* out = start + c0 + tid * kPer;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i)
+    if (tid * kPer + i < m) out[i] = min(v[i], after);
+  if (tid == 0 && c0 + m == total) start[total] = n;
+  __syncthreads();  // LDS is reused
+}
+
 // The first `reorder_blocks` workgroups gather the particles into their slots;
 // the others write the cell table, start[k] = first slot of cell k, straight
-// from the sorted keys, kTableCells cells at a time: two searches give the
-// cells' slots, whose runs' heads set their cells' starts in LDS, and a suffix
-// minimum gives an empty cell the next cell's start.  The table is written
-// once; its histogram, scanned and cleared in three launches before, moved
-// four times as much: the 256-scene ensemble's table of 44 M cells took 270
-// us and takes 60, small batches save two launches.
+// from the sorted keys.  The table is written once; its histogram, scanned and
+// cleared in three launches before, moved four times as much: 270 us for the
+// 256-scene ensemble's table of 44 M cells, whose cells and particles take 170
+// together here (the particles alone 80).
 __global__ __launch_bounds__(256) void k_table(
     StepConsts c, const int* __restrict__ sk, const int* __restrict__ sv,
     const int* __restrict__ seg, const ScenePlanes* __restrict__ sp,
@@ -755,76 +836,26 @@ __global__ __launch_bounds__(256) void k_table(
     uint64_t* __restrict__ slot_cell, int* __restrict__ slot_key, int reorder_blocks,
     const int* __restrict__ total_cells, int* __restrict__ start,
     unsigned* __restrict__ flags) {
-  constexpr int kPer = kTableCells / 256;
-  __shared__ __align__(16) int first[kTableCells];
+  __shared__ int first[kTableCells];
   __shared__ int range[2];
   __shared__ int wmin[4];
   if (fatal(flags)) return;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
   if (static_cast<int>(blockIdx.x) < reorder_blocks) {
-    reorder_slot(c, blockIdx.x * 256 + tid, sk, sv, seg, sp, posA, velA, posB, velB, pred, cellc,
-                 slot_cell, slot_key, flags);
+    reorder_slot(c, blockIdx.x * 256 + threadIdx.x, sk, sv, seg, sp, posA, velA, posB, velB,
+                 pred, cellc, slot_cell, slot_key, flags);
     return;
   }
   const int total = *total_cells;
   const int blocks = static_cast<int>(gridDim.x) - reorder_blocks;
-  for (long long q = static_cast<int>(blockIdx.x) - reorder_blocks; q * kTableCells < total;
-       q += blocks) {
-    const int c0 = static_cast<int>(q) * kTableCells;
-    const int m = min(kTableCells, total - c0);
-    if (w < 2) {
-      // (the last cells' end: every key lies below the table's size)
-      const int at = w == 1 && c0 + m == total ? c.n : lower_bound64(sk, c.n, c0 + w * m);
-      if (lane == 0) range[w] = at;
-    }
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) first[i * 256 + tid] = INT_MAX;
-    __syncthreads();
-    const int lo = range[0], hi = range[1];
-    for (int i = lo + tid; i < hi; i += 256) {
-      const int k = sk[i];
-      if (i == lo || sk[i - 1] != k) first[k - c0] = i;
-    }
-    __syncthreads();
-    int v[kPer];
-#pragma unroll
-    for (int i = 0; i < kPer; i += 4) {
-      const int4 x = *reinterpret_cast<const int4*>(first + tid * kPer + i);
-      v[i] = x.x;
-      v[i + 1] = x.y;
-      v[i + 2] = x.z;
-      v[i + 3] = x.w;
-    }
-#pragma unroll
-    for (int i = kPer - 2; i >= 0; --i) v[i] = min(v[i], v[i + 1]);
-    // the least start in the cells of the threads after this one, else hi
-    int suf = v[0];
-    for (int o = 1; o < kWave; o <<= 1) {
-      const int u = __shfl_down(suf, o, kWave);
-      if (lane + o < kWave) suf = min(suf, u);
-    }
-    if (lane == 0) wmin[w] = suf;
-    int after = __shfl_down(suf, 1, kWave);
-    if (lane == kWave - 1) after = INT_MAX;
-    __syncthreads();
-    for (int u = w + 1; u < 4; ++u) after = min(after, wmin[u]);
-    after = min(after, hi);
-    int* out = start + c0 + tid * kPer;
-#pragma unroll
-    for (int i = 0; i < kPer; i += 4) {
-      const int4 x = make_int4(min(v[i], after), min(v[i + 1], after), min(v[i + 2], after),
-                               min(v[i + 3], after));
-      const int at = tid * kPer + i;
-      if (at + 4 <= m) {
-        *reinterpret_cast<int4*>(out + i) = x;
-      } else {
-        if (at < m) out[i] = x.x;
-        if (at + 1 < m) out[i + 1] = x.y;
-        if (at + 2 < m) out[i + 2] = x.z;
-      }
-    }
-    if (tid == 0 && c0 + m == total) start[total] = c.n;
-    __syncthreads();  // LDS is reused
+  const bool sparse = total / kTableSparse > c.n;
+  const int cells = sparse ? kTableCells : kTableDense;
+  for (long long c0 = static_cast<long long>(static_cast<int>(blockIdx.x) - reorder_blocks) * cells;
+       c0 < total; c0 += static_cast<long long>(blocks) * cells) {
+    const int at = static_cast<int>(c0), m = min(cells, total - at);
+    if (sparse)
+      table_range<kTableCells / 256>(c.n, sk, at, m, total, first, range, wmin, start);
+    else
+      table_range<kTableDense / 256>(c.n, sk, at, m, total, first, range, wmin, start);
   }
 }
 
@@ -891,7 +922,7 @@ hipError_t enqueue_download(Ctx& c, float* d_pos, float* d_vel) {
 }
 
 // Batches of up to this many particles fuse the prediction and the grid setup.
-constexpr int kFusedSetup = 1 << 16;
+constexpr int kFusedSetup = 1 << 15;
 // Workgroups of the radix sort up to which each sums the digit counts of the
 // others itself (a chain of 64 loads a digit, about what two launches take).
 constexpr int kRowScatter = 64;
@@ -986,7 +1017,7 @@ hipError_t enqueue_substep(Ctx& c, const SubstepRec* rec) {
   FH_TRY(L("reorder", [&] {
     const int rb = blocks_for(c.n, 256);
     const int tb = static_cast<int>(
-        std::min<long long>(kTableGrid, (c.cell_cap + kTableCells - 1) / kTableCells));
+        std::min<long long>(kTableGrid, (c.cell_cap + kTableDense - 1) / kTableDense));
     k_table<<<rb + tb, 256, 0, st>>>(k, c.sort_k[sorted], c.sort_v[sorted], c.seg, c.planes,
                                      c.posA, c.velA, c.posB, c.velB, PK(0), c.cellc, c.slot_cell,
                                      c.slot_key, rb, c.total_cells, c.start, c.flags);
