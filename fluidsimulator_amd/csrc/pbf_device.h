@@ -61,8 +61,8 @@ struct StepConsts {
   int record_diag;
   int xcd_remap;
   int runs;         // 1: a run of identical consecutive slots is computed once
-  int full_lists;   // 1: every particle's list is stored (the adjoint and the
-                    //    diagnostics read them)
+  int full_lists;   // 1: every particle's list is stored (diagnostics), 2: as
+                    //    plain slots where it fits a row (the adjoint's)
   int tiles;        // 1: sparse 4x4x4-cell bricks run the LDS-tiled passes
 };
 
@@ -296,9 +296,10 @@ __device__ __forceinline__ unsigned restitute(float& vx, float& vy, float& vz, f
   return mask;
 }
 
-// Run-length-encoded neighbor lists in slot space: a word t >= 0 is the
-// single neighbor t; a word with the top bit set starts a run of
-// consecutive slots (t & 0x7fffffff) .. + next word - 1.
+// Neighbor lists in slot space: a word t >= 0 is the single neighbor t; a word
+// with the top bit set starts a run of consecutive slots (t & 0x7fffffff) .. +
+// next word - 1, three or more of them.  A list of as many words as neighbors
+// holds single neighbors only.
 struct NbrView {
   const long long* __restrict__ off;
   const int* __restrict__ nw;

@@ -448,7 +448,8 @@ __device__ __forceinline__ void run_range(const GatherView& gv, int a, int b, in
 
 // Encodes a list as run-length words: a word t >= 0 is the single neighbor
 // t; a word with the top bit set starts a run of consecutive slots, the next
-// word being its length.  The words in order give the neighbors in order.
+// word being its length (3 or more, so that a list of as many words as
+// neighbors is plain slots).  The words in order give the neighbors in order.
 // Used by whole wavefronts with uniform values; `write` marks the lane that
 // stores.
 struct RunWriter {
@@ -460,10 +461,11 @@ struct RunWriter {
   int run_len = 0;
   template <bool kFill>
   __device__ __forceinline__ void flush() {
-    if (run_len == 1) {
-      if (kFill && write) out[words] = run_start;
-      words += 1;
-    } else if (run_len > 1) {
+    if (run_len == 1 || run_len == 2) {  // (two words either way)
+      if (kFill && write)
+        for (int i = 0; i < run_len; ++i) out[words + i] = run_start + i;
+      words += run_len;
+    } else if (run_len > 2) {
       if (kFill && write) {
         out[words] = run_start | static_cast<int>(0x80000000u);
         out[words + 1] = run_len;
@@ -496,7 +498,7 @@ struct RunWriter {
 // run) and stops once its neighbors outgrow the row: it becomes a dense unit,
 // and its own unit is left without neighbors.  units[u] becomes {slot, neighbors
 // (-1: dense), slots of the run, scene}.  kFull also stores every list as
-// run-length words (the adjoint and the diagnostics read them).
+// words (the adjoint and the diagnostics read them).
 //
 // One lane per particle used to walk the 27 cells twice (count, then fill),
 // a chain of dependent loads: 127 us per launch for a 19x17x13 block, where
@@ -641,8 +643,8 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
           const int wi = incl_scan<kNbrLanes>(w);
           if (at && head) {
             int* out = at + sum + wi - w;
-            if (len == 1) {
-              out[0] = buf[k];
+            if (len <= 2) {
+              for (int i = 0; i < len; ++i) out[i] = buf[k + i];
             } else {
               out[0] = buf[k] | static_cast<int>(0x80000000u);
               out[1] = len;
@@ -652,7 +654,10 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
         }
         return sum;
       };
-      words = encode(nullptr);
+      // (a recorded substep's lists are plain: the reverse pass reads them
+      // side by side)
+      const bool plain = c.full_lists == 2;
+      words = plain ? (row ? cnt : 0) : encode(nullptr);
       if (g == 0) cnt_sh[grp] = words;
       __syncthreads();
       int pre = 0, total = 0;
@@ -667,7 +672,10 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
       off = base_sh + pre;
       stored = row && off + words <= nbr_cap;
       if (row && !stored && g == 0) atomicOr(flags, kFlagNeighbors);
-      (void)encode(stored ? nbr + off : nullptr);
+      if (!plain)
+        (void)encode(stored ? nbr + off : nullptr);
+      else if (stored)
+        for (int k = g; k < cnt; k += kNbrLanes) nbr[off + k] = buf[k];
     }
     if (ok && g == 0) {
       const int r = gv.run_no[s];

@@ -941,7 +941,7 @@ hipError_t enqueue_substep(Ctx& c, const SubstepRec* rec) {
   // a recorded substep keeps every particle's own list (the adjoint reads them)
   if (rec) {
     k.runs = 0;
-    k.full_lists = 1;
+    k.full_lists = 2;
   }
   // sparse bricks through the LDS-tiled passes: their slots are no heads of
   // the other passes
