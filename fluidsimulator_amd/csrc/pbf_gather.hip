@@ -498,7 +498,7 @@ struct RunWriter {
 // run) and stops once its neighbors outgrow the row: it becomes a dense unit,
 // and its own unit is left without neighbors.  units[u] becomes {slot, neighbors
 // (-1: dense), slots of the run, scene}.  kFull also stores every list as
-// words (the adjoint and the diagnostics read them).
+// run-length words (the diagnostics read them).
 //
 // One lane per particle used to walk the 27 cells twice (count, then fill),
 // a chain of dependent loads: 127 us per launch for a 19x17x13 block, where
@@ -654,10 +654,7 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
         }
         return sum;
       };
-      // (a recorded substep's lists are plain: the reverse pass reads them
-      // side by side)
-      const bool plain = c.full_lists == 2;
-      words = plain ? (row ? cnt : 0) : encode(nullptr);
+      words = encode(nullptr);
       if (g == 0) cnt_sh[grp] = words;
       __syncthreads();
       int pre = 0, total = 0;
@@ -672,10 +669,7 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
       off = base_sh + pre;
       stored = row && off + words <= nbr_cap;
       if (row && !stored && g == 0) atomicOr(flags, kFlagNeighbors);
-      if (!plain)
-        (void)encode(stored ? nbr + off : nullptr);
-      else if (stored)
-        for (int k = g; k < cnt; k += kNbrLanes) nbr[off + k] = buf[k];
+      (void)encode(stored ? nbr + off : nullptr);
     }
     if (ok && g == 0) {
       const int r = gv.run_no[s];
@@ -689,6 +683,72 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
     }
     if (kFull) __syncthreads();  // cnt_sh and base_sh are reused
     wave_sync();                 // ... and the buffer
+  }
+}
+
+// The rows of a recorded substep's list heads as plain words: a workgroup
+// takes consecutive units, whose lists it allocates with one atomic (atomics on
+// one address take about 10 ns each: one for every 8 heads made the neighbor kernel take 107 us at 65,536
+// particles; now it takes 27 and this one 21).
+__global__ __launch_bounds__(kBlock) void k_store_rows(
+    StepConsts c, GatherView gv, long long* __restrict__ noff, int* __restrict__ nwords,
+    int* __restrict__ nbr, long long nbr_cap, unsigned long long* __restrict__ nbr_total,
+    unsigned* __restrict__ flags) {
+  constexpr int kLanes = 8, kUnits = kBlock / kLanes;
+  __shared__ int wsum[kWaves];
+  __shared__ long long base_sh;
+  __shared__ int abort_sh;
+  if (threadIdx.x == 0) abort_sh = fatal(flags) ? 1 : 0;
+  __syncthreads();
+  if (abort_sh) return;
+  const int L = gv.info[1];
+  const int per = (L + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
+  const int u0 = blockIdx.x * per, u1 = min(L, u0 + per);
+  if (u0 >= u1) return;  // uniform
+  int sum = 0;
+  for (int u = u0 + static_cast<int>(threadIdx.x); u < u1; u += kBlock)
+    sum += max(gv.units[u].y, 0);
+  for (int o = kWave / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+  if (lane_id() == 0) wsum[threadIdx.x / kWave] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int total = 0;
+    for (int w = 0; w < kWaves; ++w) total += wsum[w];
+    const long long at =
+        static_cast<long long>(atomicAdd(nbr_total, static_cast<unsigned long long>(total)));
+    base_sh = at + total <= nbr_cap ? at : -1;
+    if (base_sh < 0) atomicOr(flags, kFlagNeighbors);
+  }
+  __syncthreads();
+  long long at = base_sh;
+  if (at < 0) return;
+  const int* rows = reinterpret_cast<const int*>(gv.rows);
+  const int g = static_cast<int>(threadIdx.x) / kLanes, q = lane_id() & (kLanes - 1);
+  for (int b = u0; b < u1; b += kUnits) {
+    const int u = b + g;
+    const int4 unit = u < u1 ? gv.units[u] : make_int4(0, -1, 0, 0);
+    const int cnt = max(unit.y, 0);
+    // the lists before this one: within the wavefront (its groups' first
+    // lanes), then the wavefronts before
+    int inc = cnt;
+    for (int o = kLanes; o < kWave; o <<= 1) {
+      const int v = __shfl_up(inc, o);
+      if (lane_id() >= o) inc += v;
+    }
+    __syncthreads();  // wsum is reused
+    if (lane_id() == kWave - 1) wsum[threadIdx.x / kWave] = inc;
+    __syncthreads();
+    long long off = at + inc - cnt;
+    for (int w = 0; w < kWaves; ++w) {
+      off += w < static_cast<int>(threadIdx.x) / kWave ? wsum[w] : 0;
+      at += wsum[w];
+    }
+    for (int k = q; k < cnt; k += kLanes)
+      nbr[off + k] = rows[(static_cast<size_t>(k >> 2) * c.n + unit.x) * 4 + (k & 3)];
+    if (q == 0 && unit.y >= 0) {
+      noff[unit.x] = off;
+      nwords[unit.x] = cnt;
+    }
   }
 }
 
@@ -1538,15 +1598,18 @@ hipError_t enqueue_heads(Ctx& c, const StepConsts& k) {
 hipError_t enqueue_neighbors(Ctx& c, const StepConsts& k, const GatherView& gv) {
   const int nb = std::min(4096, blocks_for(c.n, kBlock / kNbrLanes));
   int4* rows = reinterpret_cast<int4*>(c.tile_list);
-  if (!k.full_lists) {
-    k_neighbors<false><<<nb, kBlock, 0, c.stream>>>(k, gv, c.units, c.dense, c.info, rows,
-                                                    c.noff, c.nwords, c.ncount, c.nbr, c.nbr_cap,
+  if (k.full_lists == 1)
+    k_neighbors<true><<<nb, kBlock, 0, c.stream>>>(k, gv, c.units, c.dense, c.info, rows, c.noff,
+                                                   c.nwords, c.ncount, c.nbr, c.nbr_cap,
+                                                   c.nbr_total, c.flags);
+  else
+    k_neighbors<false><<<nb, kBlock, 0, c.stream>>>(k, gv, c.units, c.dense, c.info, rows, c.noff,
+                                                    c.nwords, c.ncount, c.nbr, c.nbr_cap,
                                                     c.nbr_total, c.flags);
-    return hipGetLastError();
-  }
-  k_neighbors<true><<<nb, kBlock, 0, c.stream>>>(k, gv, c.units, c.dense, c.info, rows,
-                                                 c.noff, c.nwords, c.ncount, c.nbr, c.nbr_cap,
-                                                 c.nbr_total, c.flags);
+  if (!k.full_lists) return hipGetLastError();
+  if (k.full_lists == 2)
+    k_store_rows<<<std::min(kDenseGrid, blocks_for(c.n, 32)), kBlock, 0, c.stream>>>(
+        k, gv, c.noff, c.nwords, c.nbr, c.nbr_cap, c.nbr_total, c.flags);
   k_long_lists<<<std::min(kDenseGrid, blocks_for(c.n, kWaves)), kBlock, 0, c.stream>>>(
       k, gv, 0, c.noff, c.nwords, c.ncount, c.nbr, c.nbr_cap, c.nbr_total,
       c.flags);
