@@ -127,7 +127,7 @@ int validate(int n_scenes, const fluid_hip_params* params) {
   return FLUID_HIP_OK;
 }
 
-// The tile passes evaluate the spiky factor of a pair with r2 < h2 as the
+// The passes evaluate the spiky factor of a pair with r2 < h2 as the
 // correctly rounded square root of max(r2, min_r2) without sqrtf's range
 // handling and without spiky's r > h test; both are exact when the largest
 // such argument rounds to a root <= h and the smallest is >= 2^-96.
@@ -193,8 +193,9 @@ void compute_consts_of(Ctx& c, const fluid_hip_params* params, int n_scenes) {
   k.full_lists = (c.record_diag || c.wave_mode == 1) ? 1 : 0;
   // tile mode 0 (default) tiles from kTileAutoMinParticles particles on
   const bool tile_mode = c.tile_gather == 1 || (c.tile_gather == 0 && c.n >= fluidhip::kTileAutoMinParticles);
+  k.exact_terms = tile_terms_exact(h, h2, k.min_r2) ? 1 : 0;
   k.tiles = (k.runs && c.brick_shift == 2 && tile_mode && p.solver_iterations > 0 &&
-             tile_terms_exact(h, h2, k.min_r2))
+             k.exact_terms)
                 ? 1
                 : 0;
   c.consts = k;

@@ -10,6 +10,8 @@
 #include <limits.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace fluidhip {
 
 constexpr int kMaxPlanes = 8;
@@ -64,6 +66,7 @@ struct StepConsts {
   int full_lists;   // 1: every particle's list is stored (diagnostics), 2: as
                     //    plain slots where it fits a row (the adjoint's)
   int tiles;        // 1: sparse 4x4x4-cell bricks run the LDS-tiled passes
+  int exact_terms;  // 1: pair terms need no range tests (tile_spiky)
 };
 
 struct ScenePlanes {
@@ -96,22 +99,20 @@ __device__ __forceinline__ float poly6(float r2, const StepConsts& c) {
 }
 
 // The correctly rounded square root (IEEE sqrt, as sqrtf under
-// -fhip-fp32-correctly-rounded-divide-sqrt).  For finite x >= 2^-96 the
-// hardware estimate s is corrected by the residuals x - s*s' of its float
-// neighbours s' -- the same correction the compiler emits for sqrtf, whose
-// other parts (scaling tiny inputs, passing 0 and inf through) do nothing
-// there, so both give the same bits; other x go through sqrtf itself.  The
-// gather passes call it once per neighbor, where those parts cost a third of
-// the square root.
+// -fhip-fp32-correctly-rounded-divide-sqrt).  For finite x >= 2^-96 the root
+// g = x y from the hardware's reciprocal root y is corrected once by its
+// residual x - g^2 (one fused operation, exact up to its rounding) times y / 2:
+// a Newton step that leaves an error far below the distance of a square root of
+// a float from the midpoint of two floats, so rounding it gives sqrtf's bits
+// (checked on every such float); other x go through sqrtf itself.  Five
+// instructions, where testing the hardware root's two neighbors takes nine; the
+// gather passes take one root per neighbor (with the range tests gone too, lambda
+// of 262,144 particles without tiles went from 31.1 to 29.1 us).
 __device__ __forceinline__ float sqrt_core(float x) {
   // the correction alone: finite x >= 2^-96 only
-  const float s = __builtin_amdgcn_sqrtf(x);
-  const float dn = __int_as_float(__float_as_int(s) - 1);
-  const float up = __int_as_float(__float_as_int(s) + 1);
-  const float rdn = fmaf(-dn, s, x);
-  const float rup = fmaf(-up, s, x);
-  const float r = rdn <= 0.0f ? dn : s;
-  return rup > 0.0f ? up : r;
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float g = x * y;
+  return fmaf(fmaf(-g, g, x), 0.5f * y, g);
 }
 
 __device__ __forceinline__ float sqrt_rn(float x) {
@@ -138,10 +139,63 @@ __device__ __forceinline__ float pow_ratio(float ratio, int n) {
   return powf(ratio, static_cast<float>(n));
 }
 
+// Pair terms of a pair with r2 < h2 (other pairs' values are not used).  With
+// c.exact_terms (min_r2 >= 2^-96 and sqrt(max(pred(h2), min_r2)) <= h, checked
+// on the host) the clamped argument of the square root is a finite float >=
+// 2^-96, where sqrt_core is the correctly rounded square root, and r <= h,
+// where spiky's r > h test is false: tile_poly6 and tile_spiky return what
+// poly6 and pair_spiky return (core.cpp:35-57 and the clamp of core.cpp:303),
+// bit for bit, without their range tests.
+__device__ __forceinline__ float tile_poly6(float r2, const StepConsts& c) {
+  const float diff = c.h2 - r2;
+  const float diff3 = diff * diff * diff;
+  return c.w_coeff * diff3;
+}
+
+__device__ __forceinline__ float tile_spiky(float r2, const StepConsts& c) {
+  // r2 < min_r2 ? min_r2 : r2 for 0 <= r2 < h2 and min_r2 > 0, where the
+  // bit patterns order as the floats do (one integer max)
+  const float r = sqrt_core(__int_as_float(max(__float_as_int(r2), __float_as_int(c.min_r2))));
+  const float diff = c.h - r;
+  return c.s_coeff * diff * diff;
+}
+
+// li + lj and the tensile correction -k (W / W(dq))^n (core.cpp:334-407).  The
+// exponent's kind is a template parameter (corr_kind) so that a walk's terms
+// hold no branches: off, one of 2, 3, 4 (selected factors; a factor of 1 is
+// exact), or any other, through powf.
+constexpr int kCorrOff = 0, kCorrFew = 1, kCorrPow = 2;
+inline int corr_kind(const StepConsts& c) {
+  if (!c.scorr_on) return kCorrOff;
+  return c.scorr_n >= 2 && c.scorr_n <= 4 ? kCorrFew : kCorrPow;
+}
+
+// Calls f with the constant of the exponent's kind.
+template <typename F>
+inline void with_corr(const StepConsts& c, F&& f) {
+  if (corr_kind(c) == kCorrOff)
+    f(std::integral_constant<int, kCorrOff>{});
+  else if (corr_kind(c) == kCorrFew)
+    f(std::integral_constant<int, kCorrFew>{});
+  else
+    f(std::integral_constant<int, kCorrPow>{});
+}
+
+template <int kCorr>
+__device__ __forceinline__ float pair_lambda(float li, float lj, float r2, const StepConsts& c) {
+  float sv = li + lj;
+  if (kCorr == kCorrOff) return sv;
+  const float ratio = tile_poly6(r2, c) * c.scorr_inv_wdq;
+  const float sq = ratio * ratio;
+  const float more = c.scorr_n == 3 ? ratio : c.scorr_n == 4 ? sq : 1.0f;
+  sv += c.scorr_neg_k * (kCorr == kCorrFew ? sq * more : pow_ratio(ratio, c.scorr_n));
+  return sv;
+}
+
 // Spiky factor of a pair at squared distance r2 < h2: pairs closer than
-// min_r share one precomputed factor (core.cpp:303-304 clamps r there), so
-// only the others pay for the IEEE square root.
+// min_r share one factor (core.cpp:303-304 clamps r there).
 __device__ __forceinline__ float pair_spiky(float r2, const StepConsts& c) {
+  if (c.exact_terms) return tile_spiky(r2, c);
   if (r2 < c.min_r2) return c.f_min;
   return spiky(sqrt_rn(r2), c);
 }

@@ -688,8 +688,9 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
 
 // The rows of a recorded substep's list heads as plain words: a workgroup
 // takes consecutive units, whose lists it allocates with one atomic (atomics on
-// one address take about 10 ns each: one for every 8 heads made the neighbor kernel take 107 us at 65,536
-// particles; now it takes 27 and this one 21).
+// one address take about 10 ns each: one for every 8 heads made the neighbor
+// kernel take 107 us at 65,536 particles; without them it takes 27, and this
+// one 21).
 __global__ __launch_bounds__(kBlock) void k_store_rows(
     StepConsts c, GatherView gv, long long* __restrict__ noff, int* __restrict__ nwords,
     int* __restrict__ nbr, long long nbr_cap, unsigned long long* __restrict__ nbr_total,
@@ -1236,8 +1237,8 @@ struct LambdaPass {
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2 = dx * dx + dy * dy + dz * dz;
     const float ngs = -c.grad_scale;
-    const float f = r2 < c.h2 ? pair_spiky(r2, c) : 0.0f;
     const bool grad = r2 < c.h2;
+    const float f = pair_spiky(r2, c);  // used for grad only
     const float gx = f * dx, gy = f * dy, gz = f * dz;
     const float jx = ngs * gx, jy = ngs * gy, jz = ngs * gz;
     o[0] = poly6(r2, c);
@@ -1308,7 +1309,7 @@ __device__ __forceinline__ void commit_run(const StepConsts& c, const Commit& k,
 // delta with plane projection and apply (core.cpp:334-407).  kLast also
 // commits, kRest fuses plane restitution (core.cpp:573-612).  A recorded
 // substep stores the planes that pushed (pmask).
-template <bool kLast, bool kRest>
+template <bool kLast, bool kRest, int kCorr>
 struct DeltaPass {
   static constexpr int kAcc = 3;
   using Self = float4;
@@ -1324,12 +1325,7 @@ struct DeltaPass {
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2 = dx * dx + dy * dy + dz * dz;
     const bool in = r2 < c.h2;
-    float sv = p.w + q.w;
-    if (c.scorr_on) {
-      const float ratio = poly6(r2, c) * c.scorr_inv_wdq;
-      sv += c.scorr_neg_k * pow_ratio(ratio, c.scorr_n);
-    }
-    const float sf = sv * (in ? pair_spiky(r2, c) : 0.0f);
+    const float sf = pair_lambda<kCorr>(p.w, q.w, r2, c) * pair_spiky(r2, c);
     o[0] = in ? sf * dx : 0.0f;
     o[1] = in ? sf * dy : 0.0f;
     o[2] = in ? sf * dz : 0.0f;
@@ -1358,7 +1354,7 @@ struct DeltaPass {
   }
 };
 
-template <bool kLast, bool kRest>
+template <bool kLast, bool kRest, int kCorr>
 __global__ __launch_bounds__(kBlock) void k_delta(StepConsts c, GatherView gv,
                                                   const float4* __restrict__ P,
                                                   float4* __restrict__ Pnext, Commit k,
@@ -1366,7 +1362,7 @@ __global__ __launch_bounds__(kBlock) void k_delta(StepConsts c, GatherView gv,
                                                   const unsigned* __restrict__ flags) {
   __shared__ PassLds lds;
   if (fatal(flags)) return;
-  gather(c, gv, DeltaPass<kLast, kRest>{c, P, Pnext, k, pmask}, lds);
+  gather(c, gv, DeltaPass<kLast, kRest, kCorr>{c, P, Pnext, k, pmask}, lds);
 }
 
 // The commit of a substep without iterations: every slot on its own.
@@ -1413,7 +1409,7 @@ struct XsphPass {
     const float dx = p.x.x - q.x.x, dy = p.x.y - q.x.y, dz = p.x.z - q.x.z;
     const float r2 = dx * dx + dy * dy + dz * dz;
     const bool in = r2 < c.h2;
-    const float W = poly6(r2, c);
+    const float W = tile_poly6(r2, c);
     const float m = (q.m > 0.0f) ? (c.mass / q.m) : 0.0f;
     o[0] = in ? (q.v.x - p.v.x) * W * m : 0.0f;
     o[1] = in ? (q.v.y - p.v.y) * W * m : 0.0f;
@@ -1463,7 +1459,7 @@ struct OmegaPass {
     const float dx = p.x.x - q.x.x, dy = p.x.y - q.x.y, dz = p.x.z - q.x.z;
     const float r2 = dx * dx + dy * dy + dz * dz;
     const bool in = r2 < c.h2;
-    const float f = in ? pair_spiky(r2, c) : 0.0f;
+    const float f = pair_spiky(r2, c);
     const float gx = f * dx, gy = f * dy, gz = f * dz;
     const float dvx = q.v.x - p.v.x, dvy = q.v.y - p.v.y, dvz = q.v.z - p.v.z;
     o[0] = in ? dvy * gz - dvz * gy : 0.0f;
@@ -1508,7 +1504,7 @@ struct EtaPass {
     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     const float r2 = dx * dx + dy * dy + dz * dz;
     const bool in = r2 < c.h2;
-    const float f = in ? pair_spiky(r2, c) : 0.0f;
+    const float f = pair_spiky(r2, c);
     const float gx = f * dx, gy = f * dy, gz = f * dz;
     const float co = q.w - p.w;
     o[0] = in ? co * gx : 0.0f;
@@ -1648,12 +1644,15 @@ hipError_t enqueue_delta(Ctx& c, const StepConsts& k, const GatherView& gv, cons
                          unsigned* rm) {
   const int nb = gv.dense_blocks + list_blocks(c);
   const Commit cm{c.planes, c.posB, c.posA, vout, c.rho, rm};
-  if (!last)
-    k_delta<false, false><<<nb, kBlock, 0, c.stream>>>(k, gv, P, Pn, cm, pm, c.flags);
-  else if (rest)
-    k_delta<true, true><<<nb, kBlock, 0, c.stream>>>(k, gv, P, Pn, cm, pm, c.flags);
-  else
-    k_delta<true, false><<<nb, kBlock, 0, c.stream>>>(k, gv, P, Pn, cm, pm, c.flags);
+  with_corr(k, [&](auto corr) {
+    constexpr int kCorr = decltype(corr)::value;
+    if (!last)
+      k_delta<false, false, kCorr><<<nb, kBlock, 0, c.stream>>>(k, gv, P, Pn, cm, pm, c.flags);
+    else if (rest)
+      k_delta<true, true, kCorr><<<nb, kBlock, 0, c.stream>>>(k, gv, P, Pn, cm, pm, c.flags);
+    else
+      k_delta<true, false, kCorr><<<nb, kBlock, 0, c.stream>>>(k, gv, P, Pn, cm, pm, c.flags);
+  });
   return hipGetLastError();
 }
 

@@ -56,6 +56,7 @@ constexpr int kHalo = 6;           // cells per halo edge
 constexpr int kHaloCells = 216;
 constexpr int kThreads = 256;      // workgroup of the classify kernel
 constexpr int kPass = 512;         // workgroup of the neighbor and gather kernels
+constexpr int kWavesPerSimd = 8;  // 64 registers: four workgroups of a pass on a CU
 constexpr int kPerThread = kTileMaxHalo / kPass;  // halo records staged per thread
 // In batches of kForkMinParticles particles or more, bricks with fewer
 // particles take the per-lane passes: a tile's fixed cost (layout, halo
@@ -71,27 +72,6 @@ __device__ __forceinline__ bool tile_fatal(const unsigned* flags) {
 __device__ __forceinline__ bool coincide(const float3& a, const float3& b) {
   return ((__float_as_uint(a.x) ^ __float_as_uint(b.x)) | (__float_as_uint(a.y) ^ __float_as_uint(b.y)) |
           (__float_as_uint(a.z) ^ __float_as_uint(b.z))) == 0u;
-}
-
-// Pair terms of the gather passes for a pair with r2 < h2.  Tiles run only
-// when min_r2 >= 2^-96 and sqrt(max(pred(h2), min_r2)) <= h (tile_terms_exact
-// in pbf_capi.hip), so for such a pair the clamped argument of the square
-// root is a finite float >= 2^-96, where sqrt_core is the correctly rounded
-// square root, and r <= h, where spiky's r > h test is false: tile_poly6 and
-// tile_spiky return what poly6 and pair_spiky return (core.cpp:35-57 and the
-// clamp of core.cpp:303), bit for bit, without their range tests.
-__device__ __forceinline__ float tile_poly6(float r2, const StepConsts& c) {
-  const float diff = c.h2 - r2;
-  const float diff3 = diff * diff * diff;
-  return c.w_coeff * diff3;
-}
-
-__device__ __forceinline__ float tile_spiky(float r2, const StepConsts& c) {
-  // r2 < min_r2 ? min_r2 : r2 for 0 <= r2 < h2 and min_r2 > 0, where the
-  // bit patterns order as the floats do (one integer max)
-  const float r = sqrt_core(__int_as_float(max(__float_as_int(r2), __float_as_int(c.min_r2))));
-  const float diff = c.h - r;
-  return c.s_coeff * diff * diff;
 }
 
 // Scene of the brick whose first cell has key `k0` (scenes own whole bricks).
@@ -360,23 +340,44 @@ __device__ __forceinline__ void stage_halo(const TileLayout& L, int nrec, Fetch&
     if (r0 + k * kPass < nrec) store(r0 + k * kPass, v[k]);
 }
 
-// Calls visit(r) for the LDS records r of a tile particle's cnt neighbors,
-// in list (= candidate) order.  A list is chunks of 8 16-bit entries (one
-// uint4, chunk-major: chunk q of every particle together, so one load of a
-// pass coalesces); each chunk is loaded one chunk ahead, and the 8 visits of
-// a chunk are unrolled (a visit that no lane of the wavefront needs is
-// skipped as a whole).
-template <typename Visit>
+// Visits the LDS records r of a tile particle's cnt neighbors in list (=
+// candidate) order: add(term(r, used)), with used = false for the entries past
+// the list's end in the last group of kBatch (record 0, which is in bounds).
+// A list is chunks of 8 16-bit entries (one uint4, chunk-major: chunk q of
+// every particle together, so one load of a pass coalesces; the entries past
+// the end of its last chunk are 0); each chunk is loaded one chunk ahead.  The
+// terms of a group are computed side by side, without branches (terms that do
+// not count are +0, and no sum is ever -0: each starts at +0, and a rounded
+// sum is -0 only of two -0), so one lane has kBatch square roots and LDS reads
+// in flight; the additions alone follow the list's order.  Bound by vector
+// instructions (about 50 a neighbor); with four terms side by side the passes
+// take more registers and 1% more time.  Against a branch per neighbor (and the
+// correction's exponent tested for each), delta of the million-particle block
+// went from 77 to 60 us a launch, the other passes by 3 us at most either way,
+// its substep from 1,314 to 1,282.
+constexpr int kBatch = 2;
+static_assert(kBatch % 2 == 0 && 8 % kBatch == 0, "a group is whole words of a chunk");
+
+template <typename Term, typename Add>
 __device__ __forceinline__ void tile_walk(const uint4* __restrict__ list, int n, int s, int cnt,
-                                          uint4 first, Visit&& visit) {
+                                          uint4 first, Term&& term, Add&& add) {
   uint4 q = first;
   for (int k = 0; k < cnt; k += 8) {
     const uint4 nq = k + 8 < cnt ? list[static_cast<size_t>((k >> 3) + 1) * n + s]
                                  : make_uint4(0u, 0u, 0u, 0u);
     const unsigned w[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      if (k + e < cnt) visit(static_cast<int>((w[e >> 1] >> (16 * (e & 1))) & 0xffffu));
+    for (int g = 0; g < 8; g += kBatch) {
+      if (k + g < cnt) {
+        decltype(term(0, true)) t[kBatch];
+#pragma unroll
+        for (int e = 0; e < kBatch; ++e)
+          t[e] = term(static_cast<int>((w[(g + e) >> 1] >> (16 * (e & 1))) & 0xffffu),
+                      k + g + e < cnt);
+#pragma unroll
+        for (int e = 0; e < kBatch; ++e) add(t[e]);
+      }
+    }
     q = nq;
   }
 }
@@ -464,21 +465,20 @@ __device__ __forceinline__ void tile_loop(const TileArgs& ta, int n, int xcd, Ti
 // cells get the count -1.  With nbr (a recorded substep) the
 // live tiles' lists are also stored there as slots (noff, nwords), as the
 // per-lane neighbor kernel stores its lists.
-// A halo record's p^0 and slot.
-struct RecSlot {
-  float3 p;
-  int t;
-};
+// Candidates tested side by side: 148 us at 1,048,576 particles in place of 161
+// for one at a time (8: the same).  Bound by vector instructions, about 11 a
+// candidate.
+constexpr int kTests = 4;
+static_assert(32 % kTests == 0, "a mask holds whole groups of tests");
 
 template <bool kStore>
-__global__ __launch_bounds__(kPass) void k_tile_neighbors(
+__global__ __launch_bounds__(kPass, kWavesPerSimd) void k_tile_neighbors(
     StepConsts c, TileArgs ta, const float4* __restrict__ p0, int4* __restrict__ tile_rec,
     int* __restrict__ in_tile, int* __restrict__ ncount, long long* __restrict__ noff,
     int* __restrict__ nwords, int* __restrict__ nbr, long long nbr_cap,
     unsigned long long* __restrict__ nbr_total, unsigned* __restrict__ flags) {
   __shared__ TileLayout L;
-  __shared__ float X[kTileMaxHalo], Y[kTileMaxHalo], Z[kTileMaxHalo];
-  __shared__ int Sl[kStore ? kTileMaxHalo : 1];  // each record's slot (stored lists)
+  __shared__ float4 R[kTileMaxHalo + kTests];  // p^0; w: the record's slot (its bits)
   __shared__ int scan_lds[kPass / 64 + 1];
   __shared__ long long base_sh;
   if (tile_fatal(flags)) return;
@@ -494,13 +494,12 @@ __global__ __launch_bounds__(kPass) void k_tile_neighbors(
     const TileInfo T = tile_info(tile_rec, i);
     load_layout(L, ta.tile_seg, ta.tile_src, i);
     __syncthreads();
-    stage_halo(L, T.nrec, [&](int t) { return RecSlot{ld3(p0, t), t}; },
-               [&](int r, const RecSlot& v) {
-                 X[r] = v.p.x;
-                 Y[r] = v.p.y;
-                 Z[r] = v.p.z;
-                 if (kStore) Sl[r] = v.t;
-               });
+    stage_halo(L, T.nrec,
+               [&](int t) {
+                 const float3 p = ld3(p0, t);
+                 return make_float4(p.x, p.y, p.z, __int_as_float(t));
+               },
+               [&](int r, const float4& v) { R[r] = v; });
     __syncthreads();
     int over = 0;
     for (int s = T.a + static_cast<int>(threadIdx.x); s < T.e; s += kPass) {
@@ -512,7 +511,7 @@ __global__ __launch_bounds__(kPass) void k_tile_neighbors(
       local_cell(ta.slot_cell[s], T.cx0, T.cy0, T.cz0, lx, ly, lz);
       const int own = ((lz + 1) * kHalo + ly + 1) * kHalo + lx + 1;
       const int self = L.seg[own] + (s - L.src[own]);
-      const float3 me = make_float3(X[self], Y[self], Z[self]);
+      const float3 me = make_float3(R[self].x, R[self].y, R[self].z);
       // entries enter a 128-bit shift register w3:w2:w1:w0 at the top, 16
       // bits at a time, so after 8 of them entry 0 is w0's low half; a chunk
       // goes out every 8 entries
@@ -522,19 +521,29 @@ __global__ __launch_bounds__(kPass) void k_tile_neighbors(
         const int hc = ((lz + row / 3) * kHalo + ly + row % 3) * kHalo + lx;
         const int lo = L.seg[hc], hi = L.seg[hc + 3];
         // 32 candidates at a time: first the neighbor tests as a bit mask,
-        // then the mask's bits in ascending order (the candidates' order);
+        // then the mask's bits from the top (the candidates' order);
         // the insertion runs once per neighbor, not once per candidate
         for (int b = lo; b < hi; b += 32) {
           const int nb = min(32, hi - b);
+          // kTests tests at a time, side by side, each shifting its bit in at
+          // the bottom of m; those past the row's end read the next cells'
+          // records (or the array's spare ones) and their bits are cleared.
+          // Then candidate b + j is bit 31 - j.
           unsigned m = 0u;
-          for (int j = 0; j < nb; ++j) {
-            const int r = b + j;
-            if (near0(me, make_float3(X[r], Y[r], Z[r]), c)) m |= 1u << j;
+          int j = 0;
+          for (; j < nb; j += kTests) {
+#pragma unroll
+            for (int e = 0; e < kTests; ++e) {
+              const float4 q = R[b + j + e];
+              m = m + m + (near0(me, make_float3(q.x, q.y, q.z), c) ? 1u : 0u);
+            }
           }
-          if (self >= b && self < b + 32) m &= ~(1u << (self - b));
+          m = (m << (32 - j)) & (~0u << (32 - nb));
+          if (self >= b && self < b + 32) m &= ~(0x80000000u >> (self - b));
           while (m != 0u) {
-            const int r = b + __builtin_ctz(m);
-            m &= m - 1u;
+            const int at = __builtin_clz(m);
+            const int r = b + at;
+            m &= ~(0x80000000u >> at);
             w0 = __builtin_amdgcn_alignbit(w1, w0, 16);
             w1 = __builtin_amdgcn_alignbit(w2, w1, 16);
             w2 = __builtin_amdgcn_alignbit(w3, w2, 16);
@@ -590,7 +599,9 @@ __global__ __launch_bounds__(kPass) void k_tile_neighbors(
             const unsigned w[4] = {ch.x, ch.y, ch.z, ch.w};
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-              if (q8 + e < cnt) nbr[off + q8 + e] = Sl[(w[e >> 1] >> (16 * (e & 1))) & 0xffffu];
+              if (q8 + e < cnt) 
+                nbr[off + q8 + e] =
+                    __float_as_int(R[(w[e >> 1] >> (16 * (e & 1))) & 0xffffu].w);
           }
           noff[s] = off;
           nwords[s] = cnt;
@@ -604,50 +615,55 @@ __global__ __launch_bounds__(kPass) void k_tile_neighbors(
 
 // ------------------------------------------------------------ lambda
 
+struct LambdaTerm {
+  float w, gx, gy, gz, g2;
+};
+
 // lambda pass (core.cpp:281-329) of the tiles; the per-lane term and its
 // accumulation order of k_lambda.  A recorded substep also stores the
 // gradient sum S and the denominator sum Q (sq_out).
-__global__ __launch_bounds__(kPass) void k_tile_lambda(StepConsts c, TileArgs ta,
+__global__ __launch_bounds__(kPass, kWavesPerSimd) void k_tile_lambda(StepConsts c, TileArgs ta,
                                                        float4* __restrict__ P,
                                                        float* __restrict__ rho_out,
                                                        int write_rho,
                                                        float4* __restrict__ sq_out,
                                                        const unsigned* __restrict__ flags) {
   __shared__ TileLayout L;
-  __shared__ float X[kTileMaxHalo], Y[kTileMaxHalo], Z[kTileMaxHalo];
+  __shared__ float4 R[kTileMaxHalo];
   if (tile_fatal(flags)) return;
   const float ngs = -c.grad_scale;
   tile_loop<float3>(
       ta, c.n, c.xcd_remap, L, [&](int s) { return ld3(P, s); },
-      [&](int t) { return ld3(P, t); },
-      [&](int r, const float3& q) {
-        X[r] = q.x;
-        Y[r] = q.y;
-        Z[r] = q.z;
-      },
+      [&](int t) { return P[t]; }, [&](int r, const float4& q) { R[r] = q; },
       [&](int s, const TileInfo&, const Nbrs& nb, const float3& p) {
         float rho = 0.0f, gsx = 0.0f, gsy = 0.0f, gsz = 0.0f, sg2 = 0.0f;
-        tile_walk(ta.tile_list, c.n, s, nb.cnt, nb.first, [&](int r) {
-          const float dx = p.x - X[r];
-          const float dy = p.y - Y[r];
-          const float dz = p.z - Z[r];
-          const float r2 = dx * dx + dy * dy + dz * dz;
-          // A coincident neighbor (r2 = 0) adds gradient terms of +-0, which
-          // leave the sums as they are: none of them is ever -0 (each starts
-          // at +0 and a rounded sum is -0 only of two -0).
-          if (r2 < c.h2) {
-            rho += tile_poly6(r2, c);
-            const float f = tile_spiky(r2, c);
-            const float gx = f * dx, gy = f * dy, gz = f * dz;
-            const float jx = ngs * gx, jy = ngs * gy, jz = ngs * gz;
-            gsx += gx;
-            gsy += gy;
-            gsz += gz;
-            sg2 += jx * jx + jy * jy + jz * jz;
-          } else {
-            rho += r2 > c.h2 ? 0.0f : tile_poly6(r2, c);  // poly6: +0, or NaN
-          }
-        });
+        tile_walk(
+            ta.tile_list, c.n, s, nb.cnt, nb.first,
+            [&](int r, bool used) {
+              const float4 q = R[r];
+              const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+              const float r2 = dx * dx + dy * dy + dz * dz;
+              // A coincident neighbor (r2 = 0) adds gradient terms of +-0.
+              const bool grad = used && r2 < c.h2;
+              const float f = tile_spiky(r2, c);
+              const float gx = f * dx, gy = f * dy, gz = f * dz;
+              const float jx = ngs * gx, jy = ngs * gy, jz = ngs * gz;
+              const float g2 = jx * jx + jy * jy + jz * jz;
+              LambdaTerm t;
+              t.w = used && !(r2 > c.h2) ? tile_poly6(r2, c) : 0.0f;  // poly6; NaN stays
+              t.gx = grad ? gx : 0.0f;
+              t.gy = grad ? gy : 0.0f;
+              t.gz = grad ? gz : 0.0f;
+              t.g2 = grad ? g2 : 0.0f;
+              return t;
+            },
+            [&](const LambdaTerm& t) {
+              rho += t.w;
+              gsx += t.gx;
+              gsy += t.gy;
+              gsz += t.gz;
+              sg2 += t.g2;
+            });
         rho += c.w0;
         rho *= c.mass;
         const float C = rho * c.inv_density - 1.0f;
@@ -666,45 +682,37 @@ __global__ __launch_bounds__(kPass) void k_tile_lambda(StepConsts c, TileArgs ta
 // tiles; kLast also commits (core.cpp:414-421), kRest fuses restitution.  A
 // recorded substep also stores the planes that pushed (pmask) and the
 // restitution decisions (rmask).
-template <bool kLast, bool kRest>
-__global__ __launch_bounds__(kPass) void k_tile_delta(
+template <bool kLast, bool kRest, int kCorr>
+__global__ __launch_bounds__(kPass, kWavesPerSimd) void k_tile_delta(
     StepConsts c, TileArgs ta, const float4* __restrict__ P, float4* __restrict__ Pnext,
     const ScenePlanes* __restrict__ sp,
     const float4* __restrict__ posB, float4* __restrict__ posA, float4* __restrict__ vout,
     const float* __restrict__ rho, unsigned* __restrict__ pmask, unsigned* __restrict__ rmask,
     const unsigned* __restrict__ flags) {
   __shared__ TileLayout L;
-  __shared__ float X[kTileMaxHalo], Y[kTileMaxHalo], Z[kTileMaxHalo], W[kTileMaxHalo];
+  __shared__ float4 R[kTileMaxHalo];
   if (tile_fatal(flags)) return;
   tile_loop<float4>(
       ta, c.n, c.xcd_remap, L, [&](int s) { return P[s]; },
-      [&](int t) { return P[t]; },
-      [&](int r, const float4& q) {
-        X[r] = q.x;
-        Y[r] = q.y;
-        Z[r] = q.z;
-        W[r] = q.w;
-      },
+      [&](int t) { return P[t]; }, [&](int r, const float4& q) { R[r] = q; },
       [&](int s, const TileInfo& T, const Nbrs& nb, const float4& pi) {
         float ddx = 0.0f, ddy = 0.0f, ddz = 0.0f;
-        tile_walk(ta.tile_list, c.n, s, nb.cnt, nb.first, [&](int r) {
-          const float dx = pi.x - X[r];
-          const float dy = pi.y - Y[r];
-          const float dz = pi.z - Z[r];
-          const float r2 = dx * dx + dy * dy + dz * dz;
-          if (!(r2 < c.h2)) return;
-          const float f = tile_spiky(r2, c);
-          float sv = pi.w + W[r];
-          if (c.scorr_on) {
-            const float Wr = tile_poly6(r2, c);
-            const float ratio = Wr * c.scorr_inv_wdq;
-            sv += c.scorr_neg_k * pow_ratio(ratio, c.scorr_n);
-          }
-          const float sf = sv * f;
-          ddx += sf * dx;
-          ddy += sf * dy;
-          ddz += sf * dz;
-        });
+        tile_walk(
+            ta.tile_list, c.n, s, nb.cnt, nb.first,
+            [&](int r, bool used) {
+              const float4 q = R[r];
+              const float dx = pi.x - q.x, dy = pi.y - q.y, dz = pi.z - q.z;
+              const float r2 = dx * dx + dy * dy + dz * dz;
+              const bool in = used && r2 < c.h2;
+              const float f = tile_spiky(r2, c);
+              const float sf = pair_lambda<kCorr>(pi.w, q.w, r2, c) * f;
+              return in ? make_float3(sf * dx, sf * dy, sf * dz) : make_float3(0.0f, 0.0f, 0.0f);
+            },
+            [&](const float3& t) {
+              ddx += t.x;
+              ddy += t.y;
+              ddz += t.z;
+            });
         ddx *= c.inv_density;
         ddy *= c.inv_density;
         ddz *= c.inv_density;
@@ -750,38 +758,40 @@ __global__ __launch_bounds__(kPass) void k_tile_xsph(
     float4* __restrict__ vout, const ScenePlanes* __restrict__ sp, unsigned* __restrict__ rmask,
     const unsigned* __restrict__ flags) {
   __shared__ TileLayout L;
-  __shared__ float X[kTileMaxHalo], Y[kTileMaxHalo], Z[kTileMaxHalo];
-  __shared__ float U[kTileMaxHalo], V[kTileMaxHalo], Q[kTileMaxHalo], M[kTileMaxHalo];
+  __shared__ float4 R[kTileMaxHalo];  // x, mass / rho
+  __shared__ float U[kTileMaxHalo], V[kTileMaxHalo], Q[kTileMaxHalo];
   if (tile_fatal(flags)) return;
   tile_loop<PosVel>(
       ta, c.n, c.xcd_remap, L, [&](int s) { return PosVel{ld3(pos, s), vin[s]}; },
       [&](int t) { return PosVel{ld3(pos, t), vin[t]}; },
       [&](int r, const PosVel& pv) {
-        const float3 q = pv.x;
         const float4 v = pv.v;
-        X[r] = q.x;
-        Y[r] = q.y;
-        Z[r] = q.z;
+        R[r] = make_float4(pv.x.x, pv.x.y, pv.x.z, (v.w > 0.0f) ? (c.mass / v.w) : 0.0f);
         U[r] = v.x;
         V[r] = v.y;
         Q[r] = v.z;
-        M[r] = (v.w > 0.0f) ? (c.mass / v.w) : 0.0f;
       },
       [&](int s, const TileInfo& T, const Nbrs& nb, const PosVel& me) {
         const float3 xi = me.x;
         const float4 vi = me.v;
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
-        tile_walk(ta.tile_list, c.n, s, nb.cnt, nb.first, [&](int r) {
-          const float dx = xi.x - X[r];
-          const float dy = xi.y - Y[r];
-          const float dz = xi.z - Z[r];
-          const float r2 = dx * dx + dy * dy + dz * dz;
-          if (!(r2 < c.h2)) return;
-          const float Wr = tile_poly6(r2, c);
-          ax += (U[r] - vi.x) * Wr * M[r];
-          ay += (V[r] - vi.y) * Wr * M[r];
-          az += (Q[r] - vi.z) * Wr * M[r];
-        });
+        tile_walk(
+            ta.tile_list, c.n, s, nb.cnt, nb.first,
+            [&](int r, bool used) {
+              const float4 q = R[r];
+              const float dx = xi.x - q.x, dy = xi.y - q.y, dz = xi.z - q.z;
+              const float r2 = dx * dx + dy * dy + dz * dz;
+              const bool in = used && r2 < c.h2;
+              const float Wr = tile_poly6(r2, c);
+              const float3 t = make_float3((U[r] - vi.x) * Wr * q.w, (V[r] - vi.y) * Wr * q.w,
+                                           (Q[r] - vi.z) * Wr * q.w);
+              return in ? t : make_float3(0.0f, 0.0f, 0.0f);
+            },
+            [&](const float3& t) {
+              ax += t.x;
+              ay += t.y;
+              az += t.z;
+            });
         float vx = vi.x + c.visc_c * ax;
         float vy = vi.y + c.visc_c * ay;
         float vz = vi.z + c.visc_c * az;
@@ -804,37 +814,39 @@ __global__ __launch_bounds__(kPass) void k_tile_vort_omega(
     StepConsts c, TileArgs ta, const float4* __restrict__ pos, const float4* __restrict__ vel,
     float4* __restrict__ omega, const unsigned* __restrict__ flags) {
   __shared__ TileLayout L;
-  __shared__ float X[kTileMaxHalo], Y[kTileMaxHalo], Z[kTileMaxHalo];
-  __shared__ float U[kTileMaxHalo], V[kTileMaxHalo], Q[kTileMaxHalo];
+  __shared__ float4 R[kTileMaxHalo];  // x, velocity's x
+  __shared__ float V[kTileMaxHalo], Q[kTileMaxHalo];
   if (tile_fatal(flags)) return;
   tile_loop<PosVel3>(
       ta, c.n, c.xcd_remap, L, [&](int s) { return PosVel3{ld3(pos, s), ld3(vel, s)}; },
       [&](int t) { return PosVel3{ld3(pos, t), ld3(vel, t)}; },
       [&](int r, const PosVel3& pv) {
-        const float3 q = pv.x, v = pv.v;
-        X[r] = q.x;
-        Y[r] = q.y;
-        Z[r] = q.z;
-        U[r] = v.x;
-        V[r] = v.y;
-        Q[r] = v.z;
+        R[r] = make_float4(pv.x.x, pv.x.y, pv.x.z, pv.v.x);
+        V[r] = pv.v.y;
+        Q[r] = pv.v.z;
       },
       [&](int s, const TileInfo&, const Nbrs& nb, const PosVel3& me) {
         const float3 xi = me.x, vi = me.v;
         float ox = 0.0f, oy = 0.0f, oz = 0.0f;
-        tile_walk(ta.tile_list, c.n, s, nb.cnt, nb.first, [&](int r) {
-          const float dx = xi.x - X[r];
-          const float dy = xi.y - Y[r];
-          const float dz = xi.z - Z[r];
-          const float r2 = dx * dx + dy * dy + dz * dz;
-          if (!(r2 < c.h2)) return;
-          const float f = tile_spiky(r2, c);
-          const float gx = f * dx, gy = f * dy, gz = f * dz;
-          const float dvx = U[r] - vi.x, dvy = V[r] - vi.y, dvz = Q[r] - vi.z;
-          ox += dvy * gz - dvz * gy;
-          oy += dvz * gx - dvx * gz;
-          oz += dvx * gy - dvy * gx;
-        });
+        tile_walk(
+            ta.tile_list, c.n, s, nb.cnt, nb.first,
+            [&](int r, bool used) {
+              const float4 q = R[r];
+              const float dx = xi.x - q.x, dy = xi.y - q.y, dz = xi.z - q.z;
+              const float r2 = dx * dx + dy * dy + dz * dz;
+              const bool in = used && r2 < c.h2;
+              const float f = tile_spiky(r2, c);
+              const float gx = f * dx, gy = f * dy, gz = f * dz;
+              const float dvx = q.w - vi.x, dvy = V[r] - vi.y, dvz = Q[r] - vi.z;
+              const float3 t = make_float3(dvy * gz - dvz * gy, dvz * gx - dvx * gz,
+                                           dvx * gy - dvy * gx);
+              return in ? t : make_float3(0.0f, 0.0f, 0.0f);
+            },
+            [&](const float3& t) {
+              ox += t.x;
+              oy += t.y;
+              oz += t.z;
+            });
         omega[s] = make_float4(ox, oy, oz, sqrtf(ox * ox + oy * oy + oz * oz));
       });
 }
@@ -847,12 +859,12 @@ struct PosOmega {
 // eta, confinement force and velocity update (core.cpp:512-570) of the
 // tiles, in place on vel.
 template <bool kRest>
-__global__ __launch_bounds__(kPass) void k_tile_vort_apply(
+__global__ __launch_bounds__(kPass, kWavesPerSimd) void k_tile_vort_apply(
     StepConsts c, TileArgs ta, const float4* __restrict__ pos, const float4* __restrict__ omega,
     float4* __restrict__ vel, const ScenePlanes* __restrict__ sp,
     const unsigned* __restrict__ flags) {
   __shared__ TileLayout L;
-  __shared__ float X[kTileMaxHalo], Y[kTileMaxHalo], Z[kTileMaxHalo], O[kTileMaxHalo];
+  __shared__ float4 R[kTileMaxHalo];  // x, |omega|
   if (tile_fatal(flags)) return;
   tile_loop<PosOmega>(
       ta, c.n, c.xcd_remap, L, [&](int s) { return PosOmega{ld3(pos, s), omega[s]}; },
@@ -860,29 +872,28 @@ __global__ __launch_bounds__(kPass) void k_tile_vort_apply(
         return make_float4(ld3(pos, t).x, ld3(pos, t).y, ld3(pos, t).z,
                            reinterpret_cast<const float*>(omega + t)[3]);
       },
-      [&](int r, const float4& q) {
-        X[r] = q.x;
-        Y[r] = q.y;
-        Z[r] = q.z;
-        O[r] = q.w;
-      },
+      [&](int r, const float4& q) { R[r] = q; },
       [&](int s, const TileInfo& T, const Nbrs& nb, const PosOmega& me) {
         const float3 xi = me.x;
         const float4 om = me.om;
         float ex = 0.0f, ey = 0.0f, ez = 0.0f;
-        tile_walk(ta.tile_list, c.n, s, nb.cnt, nb.first, [&](int r) {
-          const float dx = xi.x - X[r];
-          const float dy = xi.y - Y[r];
-          const float dz = xi.z - Z[r];
-          const float r2 = dx * dx + dy * dy + dz * dz;
-          if (!(r2 < c.h2)) return;
-          const float f = tile_spiky(r2, c);
-          const float gx = f * dx, gy = f * dy, gz = f * dz;
-          const float co = O[r] - om.w;
-          ex += co * gx;
-          ey += co * gy;
-          ez += co * gz;
-        });
+        tile_walk(
+            ta.tile_list, c.n, s, nb.cnt, nb.first,
+            [&](int r, bool used) {
+              const float4 q = R[r];
+              const float dx = xi.x - q.x, dy = xi.y - q.y, dz = xi.z - q.z;
+              const float r2 = dx * dx + dy * dy + dz * dz;
+              const bool in = used && r2 < c.h2;
+              const float f = tile_spiky(r2, c);
+              const float gx = f * dx, gy = f * dy, gz = f * dz;
+              const float co = q.w - om.w;
+              return in ? make_float3(co * gx, co * gy, co * gz) : make_float3(0.0f, 0.0f, 0.0f);
+            },
+            [&](const float3& t) {
+              ex += t.x;
+              ey += t.y;
+              ez += t.z;
+            });
         const float len = sqrtf(ex * ex + ey * ey + ez * ez);
         float nx = 0.0f, ny = 0.0f, nz = 0.0f;
         if (len > c.vort_norm_eps) {
@@ -946,15 +957,18 @@ hipError_t enqueue_tile_lambda(Ctx& c, const StepConsts& k, const TileArgs& ta, 
 hipError_t enqueue_tile_delta(Ctx& c, const StepConsts& k, const TileArgs& ta, const float4* P,
                               float4* Pn, bool last, bool rest, float4* vout, unsigned* pm,
                               unsigned* rm, hipStream_t st) {
-  if (!last)
-    k_tile_delta<false, false><<<kTileGrid, kPass, 0, st>>>(
-        k, ta, P, Pn, c.planes, c.posB, c.posA, vout, c.rho, pm, rm, c.flags);
-  else if (rest)
-    k_tile_delta<true, true><<<kTileGrid, kPass, 0, st>>>(
-        k, ta, P, Pn, c.planes, c.posB, c.posA, vout, c.rho, pm, rm, c.flags);
-  else
-    k_tile_delta<true, false><<<kTileGrid, kPass, 0, st>>>(
-        k, ta, P, Pn, c.planes, c.posB, c.posA, vout, c.rho, pm, rm, c.flags);
+  with_corr(k, [&](auto corr) {
+    constexpr int kCorr = decltype(corr)::value;
+    if (!last)
+      k_tile_delta<false, false, kCorr><<<kTileGrid, kPass, 0, st>>>(
+          k, ta, P, Pn, c.planes, c.posB, c.posA, vout, c.rho, pm, rm, c.flags);
+    else if (rest)
+      k_tile_delta<true, true, kCorr><<<kTileGrid, kPass, 0, st>>>(
+          k, ta, P, Pn, c.planes, c.posB, c.posA, vout, c.rho, pm, rm, c.flags);
+    else
+      k_tile_delta<true, false, kCorr><<<kTileGrid, kPass, 0, st>>>(
+          k, ta, P, Pn, c.planes, c.posB, c.posA, vout, c.rho, pm, rm, c.flags);
+  });
   return hipGetLastError();
 }
 
