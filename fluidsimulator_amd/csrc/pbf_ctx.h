@@ -160,7 +160,7 @@ struct Ctx {
   // brick tiles (sparse bricks whose passes run through LDS)
   int* in_tile = nullptr;      // per slot: 1 + its tile's index this substep, 0 outside tiles
   int* tile_count = nullptr;   // [0] tiles found this substep, [1] candidate bricks
-  int* tile_cand = nullptr;    // tile_cap: bricks of at least 32 particles (classify input)
+  int* tile_cand = nullptr;    // tile_cap: bricks that may be tiles (classify input)
   int4* tile_rec = nullptr;    // 2 tile_cap: tile records
   int* tile_seg = nullptr;     // tile_cap x 217: LDS offset of each halo cell
   int* tile_src = nullptr;     // tile_cap x 216: first slot of each halo cell

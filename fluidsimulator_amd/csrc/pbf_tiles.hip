@@ -59,10 +59,14 @@ constexpr int kPass = 512;         // workgroup of the neighbor and gather kerne
 constexpr int kWavesPerSimd = 8;  // 64 registers: four workgroups of a pass on a CU
 constexpr int kPerThread = kTileMaxHalo / kPass;  // halo records staged per thread
 // In batches of kForkMinParticles particles or more, bricks with fewer
-// particles take the per-lane passes: a tile's fixed cost (layout, halo
-// staging, a 512-thread workgroup) is not worth it for a few particles of
-// sparse spray, of which such batches can hold 10^5 bricks.
-constexpr int kTileMinParticles = 32;
+// particles go to the list heads: a tile's fixed cost (layout, halo staging, a
+// 512-thread workgroup) is not worth it for the few particles of sparse spray,
+// of which such batches can hold 10^5 bricks.  Measured with 32 / 96 / 128 / 192
+// / 256 (us per substep): the 2,076,490-particle ensemble 2,636 / 2,401 / 2,375
+// / 2,367 / 2,387 at the start and 4,208 / 3,120 / 3,242 / 3,330 / 3,323 four
+// substeps later, the falling million-particle block 3,295 / 3,240 / 3,223 /
+// 3,244 / 3,253 after ten.
+constexpr int kTileMinParticles = 128;
 
 __device__ __forceinline__ bool tile_fatal(const unsigned* flags) {
   return (*flags & kFlagFatal) != 0u;
