@@ -67,6 +67,12 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Keep loads of these (uniform, or per lane) from being moved below the next branch.
+__device__ __forceinline__ void loaded(int a) { asm volatile("" ::"s"(a)); }
+__device__ __forceinline__ void loaded(const int4& v) {
+  asm volatile("" ::"v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w));
+}
+
 // Inclusive prefix sum over groups of kW lanes.
 template <int kW>
 __device__ __forceinline__ int incl_scan(int v) {
@@ -516,13 +522,22 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
   __shared__ int cnt_sh[kHeads];
   __shared__ long long base_sh;
   __shared__ int abort_sh;
-  // Other workgroups may raise the neighbor flag at any time: read it once
-  // per workgroup so that the barriers below stay uniform.
-  if (threadIdx.x == 0) abort_sh = fatal(flags) ? 1 : 0;
-  __syncthreads();
-  if (abort_sh) return;
-  const int L = info[1];
   const int grp = static_cast<int>(threadIdx.x) / kNbrLanes;
+  // asked for at once, as in the passes
+  const int4 ahead = units[min(c.n - 1, static_cast<int>(blockIdx.x) * kHeads + grp)];
+  const int L = info[1];
+  const bool failed = fatal(flags);
+  loaded(L);
+  loaded(ahead);
+  if (kFull) {
+    // Other workgroups may raise the neighbor flag at any time: read it once
+    // per workgroup so that the barriers below stay uniform.
+    if (threadIdx.x == 0) abort_sh = failed ? 1 : 0;
+    __syncthreads();
+    if (abort_sh) return;
+  } else if (failed) {
+    return;
+  }
   const int g = static_cast<int>(threadIdx.x) & (kNbrLanes - 1);
   const int half = lane_id() & ~(kNbrLanes - 1);
   const unsigned below = (1u << g) - 1u;
@@ -530,7 +545,12 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
   for (int u0 = blockIdx.x * kHeads; u0 < L; u0 += gridDim.x * kHeads) {
     const int u = u0 + grp;
     const bool on = u < L;
-    const int4 unit = on ? units[u] : make_int4(0, 0, 0, 0);
+    int4 unit = make_int4(0, 0, 0, 0);
+    if (u0 == static_cast<int>(blockIdx.x) * kHeads) {
+      if (on) unit = ahead;
+    } else if (on) {
+      unit = units[u];
+    }
     const int s = unit.x;
     const float3 me = ld3(gv.p0, s);
     int a = 0, b = 0;
@@ -753,13 +773,14 @@ __global__ __launch_bounds__(kBlock) void k_store_rows(
   }
 }
 
-// A dense unit: `heads` consecutive runs from run r0 on, the first at slot s.
+// A dense unit: `heads` consecutive runs from run r0 on, the first at slot s
+// (`unit`: the heads of a unit, at most).
 struct DenseUnit {
   int s, sc, r0, heads;
   bool single;
 };
 
-__device__ __forceinline__ DenseUnit dense_unit(const GatherView& gv, int u) {
+__device__ __forceinline__ DenseUnit dense_unit(const GatherView& gv, int u, int unit) {
   DenseUnit d;
   const int2 w = gv.dense[u];
   d.s = __builtin_amdgcn_readfirstlane(w.x);
@@ -771,7 +792,6 @@ __device__ __forceinline__ DenseUnit dense_unit(const GatherView& gv, int u) {
   if (!d.single) {
     const int end = gv.start[gv.slot_key[d.s] + 1];  // of the cell
     const int left = __builtin_amdgcn_readfirstlane(gv.run_no[end - 1]) + 1 - d.r0;
-    const int unit = gv.info[3];
     d.heads = min(left, unit - (d.r0 & (unit - 1)));
   }
   return d;
@@ -791,7 +811,7 @@ __global__ __launch_bounds__(kBlock) void k_long_lists(
   const int lane = lane_id();
   const int nw = static_cast<int>(gridDim.x) * kWaves;
   for (int u = blockIdx.x * kWaves + threadIdx.x / kWave; u < D; u += nw) {
-    const DenseUnit d = dense_unit(gv, u);
+    const DenseUnit d = dense_unit(gv, u, gv.info[3]);
     if (only_long && !d.single) continue;
     int a, b;
     if (!cell_range(gv, d.s, d.sc, lane, a, b)) continue;
@@ -896,7 +916,7 @@ __global__ __launch_bounds__(kBlock) void k_count_dense(StepConsts c, GatherView
   Ranges& R = rng[threadIdx.x / kWave];
   const int nw = static_cast<int>(gridDim.x) * kWaves;
   for (int u = blockIdx.x * kWaves + threadIdx.x / kWave; u < D; u += nw) {
-    const DenseUnit d = dense_unit(gv, u);
+    const DenseUnit d = dense_unit(gv, u, gv.info[3]);
     wave_sync();
     const int total = dense_ranges(gv, R, d.s, d.sc);
     for (int h = 0; h < d.heads; ++h) {
@@ -980,7 +1000,7 @@ __device__ __forceinline__ void add4(float& acc, const float4& x) {
 }
 
 // List heads: kListLanes lanes each, 32 neighbors at a time.  Bound by the
-// latency of unit, row and record loads in a small batch (4,199 particles: 5.3
+// latency of unit, row and record loads in a small batch (4,199 particles: 4.7
 // us per lambda launch, where one lane per particle walking its own list took
 // 49) and by vector instructions in a large one.  A wavefront
 // takes up to kWave consecutive heads, kWave / kListLanes at a time, and then
@@ -989,24 +1009,26 @@ __device__ __forceinline__ void add4(float& acc, const float4& x) {
 // over the wavefronts instead.
 template <typename Pass>
 __device__ __forceinline__ void pass_lists(const StepConsts& c, const GatherView& gv,
-                                           const Pass& pass, float* lds, float* sums, int block,
-                                           int nblocks) {
+                                           const Pass& pass, float* lds, float* sums, int first,
+                                           int waves, int L, const int4& ahead) {
   constexpr int kA = Pass::kAcc;
   constexpr int kHeads = kWave / kListLanes;
-  const int L = gv.info[1];
   const int lane = lane_id();
   const int q = lane & (kListLanes - 1);
   const int grp = lane / kListLanes;
   float* T = lds + grp * (kA * kListRow);
   const float4* mine = reinterpret_cast<const float4*>(T + min(q, kA - 1) * kListRow);
   const int* rows = reinterpret_cast<const int*>(gv.rows);
-  const int waves = nblocks * kWaves;
   const int chunk = kHeads * max(1, min(kListLanes, L / (waves * kHeads)));
-  const int first = block * kWaves + static_cast<int>(threadIdx.x) / kWave;
   for (int base = first * chunk; base < L; base += waves * chunk) {
     for (int h = 0; h < chunk && base + h < L; h += kHeads) {
       const int u = base + h + grp;
-      const int4 unit = u < L ? gv.units[u] : make_int4(0, -1, 0, 0);
+      int4 unit = make_int4(0, -1, 0, 0);
+      if (chunk == kHeads && base == first * kHeads) {
+        if (u < L) unit = ahead;
+      } else if (u < L) {
+        unit = gv.units[u];
+      }
       const int s = unit.x, cnt = unit.y;
       const typename Pass::Self me = pass.self(s);
       int mx = cnt;
@@ -1081,14 +1103,13 @@ __device__ __forceinline__ void pass_lists(const StepConsts& c, const GatherView
 template <typename Pass>
 __device__ __forceinline__ void pass_dense(const StepConsts& c, const GatherView& gv,
                                            const Pass& pass, float* lds, float* sums, Ranges& R,
-                                           int block, int nblocks) {
+                                           int block, int nblocks, int D, int unit) {
   constexpr int kA = Pass::kAcc;
   using Rec = typename Pass::Rec;
   constexpr int kRec = sizeof(Rec) / sizeof(float);
   constexpr int kQ = (1 + kRec + 3) / 4;  // the heads that take it, its record
   static_assert(kQ <= kEntryQuads, "an entry must fit");
   static_assert(kMaxAcc * kWave >= 2 * kWave, "an entry's run must fit the sums");
-  const int D = gv.info[2];
   const int lane = lane_id();
   float4* ent = reinterpret_cast<float4*>(lds);
   float* T = lds + 4 * kEntryQuads * kWave;
@@ -1097,7 +1118,7 @@ __device__ __forceinline__ void pass_dense(const StepConsts& c, const GatherView
                                                    static_cast<int>(threadIdx.x) / kWave);
   const int hp = lane / kA, ha = lane % kA;  // the head and accumulator this lane adds
   for (int u = first; u < D; u += waves) {
-    const DenseUnit d = dense_unit(gv, u);
+    const DenseUnit d = dense_unit(gv, u, unit);
     const int lg = d.heads > 4 ? 3 : d.heads > 2 ? 2 : d.heads > 1 ? 1 : 0;
     const int G = kWave >> lg;
     const int p = lane >> (6 - lg), g = lane & (G - 1);
@@ -1206,18 +1227,37 @@ __device__ __forceinline__ void pass_dense(const StepConsts& c, const GatherView
 }
 
 // The first gv.dense_blocks workgroups take the dense units (the longest
-// work, dispatched first), the others the list heads.
+// work, dispatched first), the others the list heads.  In a small batch a pass
+// is a chain of loads that miss (each about 0.5 us: the producer ran on other
+// XCDs), so the fatal flag, the counts and the list heads a wavefront will
+// take if it takes one round are asked for at once (the heads' array has an entry
+// for every particle).  One after the other before: lambda of 4,199 particles
+// 5.0 -> 4.7 us per launch, of 7,680 5.85 -> 5.3, delta 6.2 -> 5.8 and 7.3 -> 6.6;
+// of 262,144, bound by instructions, 29.2 either way.
 template <typename Pass>
 __device__ __forceinline__ void gather(const StepConsts& c, const GatherView& gv,
-                                       const Pass& pass, PassLds& lds) {
+                                       const Pass& pass, PassLds& lds, const unsigned* flags) {
   const int w = threadIdx.x / kWave;
   float* term = reinterpret_cast<float*>(lds.term[w]);
-  const int b = blockIdx.x;
-  if (b < gv.dense_blocks)
-    pass_dense(c, gv, pass, term, lds.sums[w], lds.rng[w], b, gv.dense_blocks);
-  else
-    pass_lists(c, gv, pass, term, lds.sums[w], b - gv.dense_blocks,
-               static_cast<int>(gridDim.x) - gv.dense_blocks);
+  const int b = static_cast<int>(blockIdx.x) - gv.dense_blocks;
+  if (b < 0) {
+    const int D = gv.info[2], unit = gv.info[3];
+    const bool failed = fatal(flags);
+    loaded(D);
+    loaded(unit);
+    if (failed) return;
+    pass_dense(c, gv, pass, term, lds.sums[w], lds.rng[w], blockIdx.x, gv.dense_blocks, D, unit);
+  } else {
+    const int first = b * kWaves + w;
+    const int4 ahead = gv.units[min(c.n - 1, first * (kWave / kListLanes) + lane_id() / kListLanes)];
+    const int L = gv.info[1];
+    const bool failed = fatal(flags);
+    loaded(L);
+    loaded(ahead);
+    if (failed) return;
+    pass_lists(c, gv, pass, term, lds.sums[w], first,
+               (static_cast<int>(gridDim.x) - gv.dense_blocks) * kWaves, L, ahead);
+  }
 }
 
 // lambda (core.cpp:281-329): rho, the gradient sum, the sum of squares.
@@ -1271,8 +1311,7 @@ __global__ __launch_bounds__(kBlock) void k_lambda(StepConsts c, GatherView gv,
                                                    float4* __restrict__ sq,
                                                    const unsigned* __restrict__ flags) {
   __shared__ PassLds lds;
-  if (fatal(flags)) return;
-  gather(c, gv, LambdaPass{c, P, rho, sq}, lds);
+  gather(c, gv, LambdaPass{c, P, rho, sq}, lds, flags);
 }
 
 // What the commit of the last iteration reads and writes (core.cpp:414-421).
@@ -1361,8 +1400,7 @@ __global__ __launch_bounds__(kBlock) void k_delta(StepConsts c, GatherView gv,
                                                   unsigned* __restrict__ pmask,
                                                   const unsigned* __restrict__ flags) {
   __shared__ PassLds lds;
-  if (fatal(flags)) return;
-  gather(c, gv, DeltaPass<kLast, kRest, kCorr>{c, P, Pnext, k, pmask}, lds);
+  gather(c, gv, DeltaPass<kLast, kRest, kCorr>{c, P, Pnext, k, pmask}, lds, flags);
 }
 
 // The commit of a substep without iterations: every slot on its own.
@@ -1440,8 +1478,7 @@ __global__ __launch_bounds__(kBlock) void k_xsph(StepConsts c, GatherView gv,
                                                  unsigned* __restrict__ rmask,
                                                  const unsigned* __restrict__ flags) {
   __shared__ PassLds lds;
-  if (fatal(flags)) return;
-  gather(c, gv, XsphPass<kRest>{c, pos, vin, vout, sp, rmask}, lds);
+  gather(c, gv, XsphPass<kRest>{c, pos, vin, vout, sp, rmask}, lds, flags);
 }
 
 // vorticity: omega and |omega| (core.cpp:472-508)
@@ -1479,8 +1516,7 @@ __global__ __launch_bounds__(kBlock) void k_vort_omega(StepConsts c, GatherView 
                                                        float4* __restrict__ omega,
                                                        const unsigned* __restrict__ flags) {
   __shared__ PassLds lds;
-  if (fatal(flags)) return;
-  gather(c, gv, OmegaPass{c, pos, vel, omega}, lds);
+  gather(c, gv, OmegaPass{c, pos, vel, omega}, lds, flags);
 }
 
 // vorticity: eta, confinement force, velocity update (core.cpp:512-570), in
@@ -1547,8 +1583,7 @@ __global__ __launch_bounds__(kBlock) void k_vort_apply(StepConsts c, GatherView 
                                                        const ScenePlanes* __restrict__ sp,
                                                        const unsigned* __restrict__ flags) {
   __shared__ PassLds lds;
-  if (fatal(flags)) return;
-  gather(c, gv, EtaPass<kRest>{c, pos, omega, vel, sp}, lds);
+  gather(c, gv, EtaPass<kRest>{c, pos, omega, vel, sp}, lds, flags);
 }
 
 __global__ void k_reset_total(unsigned long long* total) {
