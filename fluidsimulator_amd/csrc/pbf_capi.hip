@@ -234,19 +234,6 @@ std::vector<fluidhip::ScenePlanes> scene_tables(const Ctx& c) {
   return t;
 }
 
-template <typename T>
-hipError_t dalloc(T** p, size_t count) {
-  *p = nullptr;
-  if (count == 0) count = 1;
-  return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
-}
-
-template <typename T>
-void dfree(T*& p) {
-  if (p) hipFree(p);
-  p = nullptr;
-}
-
 // Device memory and streams of destroyed contexts, kept for the next ones:
 // a program that steps through the stateless call creates and destroys a
 // context for every substep, and hipMalloc and hipFree of its buffers took 0.9
@@ -280,6 +267,35 @@ Kept& kept() {
   return *k;
 }
 
+// hipMalloc; when memory runs out, again without the kept blocks.
+hipError_t device_malloc(void** p, size_t bytes) {
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  Kept& k = kept();
+  std::vector<Kept::Block> out;
+  {
+    std::lock_guard<std::mutex> lock(k.mu);
+    out.swap(k.blocks);
+    k.bytes = 0;
+  }
+  for (auto& b : out) (void)hipFree(b.p);
+  return hipMalloc(p, bytes);
+}
+
+template <typename T>
+hipError_t dalloc(T** p, size_t count) {
+  *p = nullptr;
+  if (count == 0) count = 1;
+  return device_malloc(reinterpret_cast<void**>(p), count * sizeof(T));
+}
+
+template <typename T>
+void dfree(T*& p) {
+  if (p) hipFree(p);
+  p = nullptr;
+}
+
 // The current device's memory of at least `bytes` (at most twice as much, so
 // that a small context does not hold a large one's); *got is its size.
 hipError_t take_block(int device, size_t bytes, void** p, size_t* got) {
@@ -303,17 +319,7 @@ hipError_t take_block(int device, size_t bytes, void** p, size_t* got) {
       return hipSuccess;
     }
   }
-  hipError_t e = hipMalloc(p, bytes);
-  if (e != hipErrorOutOfMemory) return e;
-  (void)hipGetLastError();
-  std::vector<Kept::Block> out;
-  {
-    std::lock_guard<std::mutex> lock(k.mu);
-    out.swap(k.blocks);
-    k.bytes = 0;
-  }
-  for (auto& b : out) (void)hipFree(b.p);
-  return hipMalloc(p, bytes);
+  return device_malloc(p, bytes);
 }
 
 // Gives back a block whose work has finished.
