@@ -286,7 +286,7 @@ __global__ __launch_bounds__(kBlock) void k_heads(
   }
 }
 
-// Both kernels in one workgroup, for batches of up to kSmallSort particles
+// Both kernels in one workgroup, for batches of up to kSmallHeads particles
 // (two launches of 5 us each become one): thread t holds slots t, t + 1024, ...
 __global__ __launch_bounds__(1024) void k_heads_small(
     StepConsts c, const float4* __restrict__ posB, const float4* __restrict__ velB,
@@ -295,7 +295,8 @@ __global__ __launch_bounds__(1024) void k_heads_small(
     int4* __restrict__ units, int2* __restrict__ dense, int* __restrict__ info,
     long long* __restrict__ noff, int* __restrict__ nwords, int* __restrict__ ncount,
     const unsigned* __restrict__ flags) {
-  constexpr int kT = 1024, kW = kT / kWave, kR = kSmallSort / kT;
+  constexpr int kT = 1024, kW = kT / kWave, kR = kSmallHeads / kT;
+  static_assert(kR * kT == kSmallHeads && kR * kW % kWave == 0, "whole rounds of the scan");
   __shared__ int runs[kR * kW], lists[kR * kW];
   __shared__ int nd_sh, ndense;
   if (fatal(flags)) return;
@@ -1612,7 +1613,7 @@ GatherView gather_view(const Ctx& c, const float4* p0) {
 hipError_t enqueue_heads(Ctx& c, const StepConsts& k) {
   const int G = std::min(c.scan_blocks, blocks_for(c.n, 4 * kBlock));
   const int* tile = k.tiles ? c.in_tile : nullptr;
-  if (c.n <= kSmallSort) {
+  if (c.n <= kSmallHeads) {
     k_heads_small<<<1, 1024, 0, c.stream>>>(k, c.posB, c.velB, c.slot_key, c.start, tile,
                                             c.run_no, c.rep_list, c.units, c.dense, c.info,
                                             c.noff, c.nwords, c.ncount, c.flags);

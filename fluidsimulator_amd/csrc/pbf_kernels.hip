@@ -612,92 +612,79 @@ __global__ __launch_bounds__(256) void k_radix_scatter(int n, const int* __restr
   }
 }
 
-// The whole sort of a batch of up to kSmallSort particles in one workgroup:
-// keys in original-id order in LDS, then as many stable 8-bit passes as the
-// table's size has digits.  A wavefront ranks its consecutive items 64 at a
-// time against its own digit counts (no barrier inside a pass but for the two
-// around the scan of the counts).  Replaces k_sort_keys and two launches per
-// pass, each of which takes about 4 us whatever its size: 2,431 particles 32
-// -> 9 us.
-__global__ __launch_bounds__(1024) void k_small_sort(
+// The whole sort of a batch of up to kRankSort particles in one launch: the slot
+// of a particle is the number of particles with a lower key, or the same key and
+// a lower id.  Every workgroup lays the keys of all particles out in LDS by id
+// and counts for kRankIds consecutive ids; lane l and l + 32 of its wavefronts
+// count for the same id over different blocks of 32 keys.  Ids below the
+// workgroup's count with key <= its key, ids above with key <, so each pair is
+// one comparison and one addition with carry.
+//
+// Bound by launch and load latency in the smallest batches and by the keys, which
+// every workgroup computes, and the comparisons in the largest: 1,728 / 4,199 /
+// 7,680 particles take 6.3 / 9.6 / 16.4 us; a radix sort in one workgroup, which
+// this replaces, 10.4 / 16.7 / 27.5.  Beyond kRankSort the work grows with the
+// square: k_sort_keys and the radix passes (us per 8 substeps, this against
+// them: 9,216 particles 1,295 / 1,303, 13,824 1,460 / 1,420, 16,250 1,558 / 1,423).
+constexpr int kRankIds = 32;
+constexpr int kRankSort = 8192;
+__global__ __launch_bounds__(1024) void k_rank_sort(
     StepConsts c, const float4* __restrict__ pos, const uint64_t* __restrict__ cellc,
-    const int* __restrict__ seg, const GridDesc* __restrict__ grid,
-    const int* __restrict__ total_cells, int* __restrict__ kout, int* __restrict__ vout,
-    unsigned* __restrict__ flags) {
-  constexpr int kT = 1024, kW = kT / kWave, kR = kSmallSort / kT;
-  __shared__ int key[kSmallSort];
-  __shared__ unsigned short val[kSmallSort];
-  __shared__ unsigned short cnt[kW][256];
-  __shared__ int dbase[256];
-  __shared__ int scan_lds[kW + 1];
-  __shared__ int stop;
-  if (threadIdx.x == 0) stop = fatal(flags) ? 1 : 0;
+    const int* __restrict__ seg, const GridDesc* __restrict__ grid, int* __restrict__ kout,
+    int* __restrict__ vout, unsigned* __restrict__ flags) {
+  constexpr int kT = 1024, kHalves = kT / kRankIds;
+  __shared__ __align__(16) unsigned key[kRankSort];
+  __shared__ int slot[kRankIds];
+  __shared__ int rank[kRankIds];
+  // (the flag may be raised by other workgroups at any time: no barrier depends on it)
+  const bool failed = fatal(flags);
+  const int n = c.n, tid = threadIdx.x;
+  const int i0 = blockIdx.x * kRankIds;
+  const int blocks = (n + kRankIds - 1) / kRankIds;
+  if (tid < kRankIds) {
+    rank[tid] = 0;
+    slot[tid] = -1;
+    if (n + tid < blocks * kRankIds) key[n + tid] = INT_MAX;  // below no key
+  }
   __syncthreads();
-  if (stop) return;
-  const int n = c.n, tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+#pragma unroll 4
   for (int p = tid; p < n; p += kT) {
     const int id = __float_as_int(reinterpret_cast<const float*>(pos + p)[3]);
     if (id < 0 || id >= n) {  // ids are 0..n-1; refuse rather than write outside
       atomicOr(flags, kFlagRange);
       continue;
     }
-    key[id] = slot_cell_key(c, p, cellc, seg, grid);
-    val[id] = static_cast<unsigned short>(p);
+    key[id] = static_cast<unsigned>(slot_cell_key(c, p, cellc, seg, grid));
+    if (id - i0 >= 0 && id - i0 < kRankIds) slot[id - i0] = p;
   }
   __syncthreads();
-  const int rounds = (n + kT - 1) / kT;
-  const int last = *total_cells - 1;
-  for (int shift = 0; shift < 31 && (last >> shift) > 0; shift += 8) {
-    int kk[kR], rank[kR];
-    unsigned short vv[kR];
-    for (int i = lane; i < 256; i += kWave) cnt[w][i] = 0;
+  const int i = tid & (kRankIds - 1);
+  const unsigned mine = key[i0 + i];
+  int count[2] = {0, 0};
+  for (int b = tid / kRankIds; b < blocks; b += kHalves) {
+    const uint4* q = reinterpret_cast<const uint4*>(key + b * kRankIds);
+    if (b != static_cast<int>(blockIdx.x)) {
+      const unsigned lim = mine + (b < static_cast<int>(blockIdx.x) ? 1u : 0u);
 #pragma unroll
-    for (int r = 0; r < kR; ++r) {
-      if (r < rounds) {
-        const int i = (w * rounds + r) * kWave + lane;
-        const bool ok = i < n;
-        kk[r] = ok ? key[i] : 0;
-        vv[r] = ok ? val[i] : 0;
-        const int d = (kk[r] >> shift) & 255;
-        const unsigned long long peers = digit_peers(d, ok);
-        const int below = __popcll(peers & ((1ull << lane) - 1ull));
-        const int before = cnt[w][d];
-        rank[r] = before + below;
-        // a wavefront's LDS accesses complete in order
-        if (ok && below == 0)
-          cnt[w][d] = static_cast<unsigned short>(before + __popcll(peers));
-        __builtin_amdgcn_wave_barrier();
+      for (int j = 0; j < kRankIds / 4; ++j) {
+        const uint4 k = q[j];
+        count[0] += k.x < lim ? 1 : 0;
+        count[1] += k.y < lim ? 1 : 0;
+        count[0] += k.z < lim ? 1 : 0;
+        count[1] += k.w < lim ? 1 : 0;
       }
+    } else {
+      const unsigned* k = key + b * kRankIds;
+#pragma unroll 1
+      for (int j = 0; j < kRankIds; ++j) count[0] += k[j] < mine + (j < i ? 1u : 0u) ? 1 : 0;
     }
-    __syncthreads();
-    int total = 0;
-    if (tid < 256)
-      for (int v = 0; v < kW; ++v) {
-        const int x = cnt[v][tid];
-        cnt[v][tid] = static_cast<unsigned short>(total);
-        total += x;
-      }
-    int all;
-    const int excl = block_excl_scan(total, scan_lds, &all);
-    if (tid < 256) dbase[tid] = excl;
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kR; ++r) {
-      if (r < rounds) {
-        const int i = (w * rounds + r) * kWave + lane;
-        const int d = (kk[r] >> shift) & 255;
-        const int at = dbase[d] + cnt[w][d] + rank[r];
-        if (i < n && at < n) {  // always at < n, as the counts are of these items
-          key[at] = kk[r];
-          val[at] = vv[r];
-        }
-      }
-    }
-    __syncthreads();
   }
-  for (int i = tid; i < n; i += kT) {
-    kout[i] = key[i];
-    vout[i] = val[i];
+  atomicAdd(&rank[i], count[0] + count[1]);
+  __syncthreads();
+  if (tid < kRankIds && i0 + tid < n && !failed) {
+    const int r = rank[tid];  // below n: the particle itself is not counted
+    kout[r] = static_cast<int>(mine);
+    vout[r] = slot[tid];
   }
 }
 
@@ -990,10 +977,10 @@ hipError_t enqueue_substep(Ctx& c, const SubstepRec* rec) {
   const int passes = (key_bits + 7) / 8;
   int sorted = passes & 1;  // which buffers end up sorted
   FH_TRY(L("sort", [&] {
-    if (c.n <= kSmallSort) {
+    if (c.n <= kRankSort) {
       sorted = 0;
-      k_small_sort<<<1, 1024, 0, st>>>(k, c.posA, c.cellc, c.seg, c.grid, c.total_cells,
-                                       c.sort_k[0], c.sort_v[0], c.flags);
+      k_rank_sort<<<blocks_for(c.n, kRankIds), 1024, 0, st>>>(
+          k, c.posA, c.cellc, c.seg, c.grid, c.sort_k[0], c.sort_v[0], c.flags);
       return;
     }
     k_sort_keys<<<blocks_for(c.n, 256), 256, 0, st>>>(k, c.posA, c.cellc, c.seg, c.grid,
