@@ -1098,9 +1098,9 @@ __device__ __forceinline__ void pass_lists(const StepConsts& c, const GatherView
 // entries in the piled-up million-particle block).  One lane per particle over
 // all candidates in turn, the walk this replaces, was bound by the latency of
 // its longest wavefronts (0.4 us per candidate): lambda of the splashing
-// 32,768-particle dam break took 237 us per launch and takes 30 beside the
-// tiles, the 262,144-particle dam breaks' 725 and 150, the piled-up
-// million-particle block's 2,000 and 800.
+// 32,768-particle dam break took 237 us per launch and takes 28, the
+// 262,144-particle dam breaks' 725 and 96, the piled-up million-particle
+// block's 2,000 and 344 (beside its tiles).
 template <typename Pass>
 __device__ __forceinline__ void pass_dense(const StepConsts& c, const GatherView& gv,
                                            const Pass& pass, float* lds, float* sums, Ranges& R,
@@ -1597,7 +1597,18 @@ inline int blocks_for(long long n, int bs) { return static_cast<int>((n + bs - 1
 // batch at once, a fixed grid that loops over the heads of a large one.
 constexpr int kDenseGrid = 1024;
 constexpr int kListGrid = 2048;
-int dense_blocks(const Ctx& c) { return std::min(kDenseGrid, blocks_for(c.n, kWaves)); }
+// A unit takes up to a hundred times as long as another: beyond the workgroups
+// the chip holds at once (kDenseGrid) the dispatcher hands the next units to
+// whichever CU is free.  Only a large batch has that many units, and workgroups
+// without one cost each pass 0.3 us a thousand.  Lambda of the piled-up
+// million-particle block with 1,024 / 2,048 / 4,096 / 8,192 workgroups: 440 / 365 /
+// 344 / 345 us per launch; of the 256-scene ensemble 101 / 102 / 103 / 104.
+// (A counter that the wavefronts of a workgroup share: 355 with 1,024, but 262,144
+// splashing particles 96 -> 99.)
+int dense_blocks(const Ctx& c) {
+  return std::min(std::max(kDenseGrid, std::min(4 * kDenseGrid, c.n / 256)),
+                  blocks_for(c.n, kWaves));
+}
 int list_blocks(const Ctx& c) {
   return std::min(kListGrid, blocks_for(c.n, kBlock / kListLanes));
 }
