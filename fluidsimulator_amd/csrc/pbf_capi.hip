@@ -172,15 +172,6 @@ void compute_consts_of(Ctx& c, const fluid_hip_params* params, int n_scenes) {
   const float wdq = scorr_enabled ? host_poly6(dq * dq, h) : 0.0f;
   const float inv_wdq = (wdq > 1e-12f) ? (1.0f / wdq) : 0.0f;
   k.scorr_on = (scorr_enabled && inv_wdq > 0.0f) ? 1 : 0;
-  {
-    // (li + lj + scorr(r=0)) * f_min stays finite when |l| < lam_safe
-    const double ratio = static_cast<double>(k.w0) * inv_wdq;
-    const double sc = k.scorr_on ? std::fabs(p.scorr_k) * 2.0 * std::pow(ratio, p.scorr_n) : 0.0;
-    const double fm = std::fabs(static_cast<double>(k.f_min));
-    double lim = 0.5 * (3.4e38 / 8.0 / (fm > 0.0 ? fm : 1.0) - sc);
-    if (!(lim > 0.0)) lim = 0.0;
-    k.lam_safe = static_cast<float>(std::min(lim, 1.0e30));
-  }
   k.scorr_inv_wdq = inv_wdq;
   k.scorr_neg_k = -p.scorr_k;
   k.scorr_n = p.scorr_n;
@@ -1433,9 +1424,9 @@ int fluid_hip_get_stats(fluid_hip_ctx* ctx, int64_t* out, int32_t n) {
                           hipMemcpyDeviceToHost),
                 "read tiles");
       for (int i = 0; i < tiles; ++i)
-        if (rec[2 * i + 1].w >= 0) ++v[8];  // live: not handed back to the per-lane passes
+        if (rec[2 * i + 1].w >= 0) ++v[8];  // live: not handed back to the passes over heads
       // the particles the tiles computed (a tile leaves its brick's dense or
-      // coincident cells to the per-lane passes)
+      // coincident cells to the passes over heads)
       std::vector<int> in_tile(static_cast<size_t>(c.n));
       if (c.n)
         HIP_TRY(hipMemcpy(in_tile.data(), c.in_tile, sizeof(int) * in_tile.size(),

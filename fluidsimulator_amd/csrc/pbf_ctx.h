@@ -18,10 +18,10 @@ constexpr int kTileMaxHalo = 2048;  // particles of a tile's 6^3-cell halo held 
 // A brick with a cell of this many candidates (particles in its 27 cells) or
 // more is no tile.
 constexpr int kTileMaxCand = 512;
-// neighbors of a tile particle, at most (else its tile goes per-lane).  In
+// neighbors of a tile particle, at most (else its tile goes to the passes over heads).  In
 // batches of kForkMinParticles particles or more a list holds every neighbor
 // a tile particle can have (fewer than kTileMaxCand), 1 KiB per particle, so
-// no tile goes back and the lane map is built before the tile lists; smaller
+// no tile goes back and the heads are listed before the tile lists; smaller
 // batches, which tile their piles of coincident particles too, keep
 // kTileListSmall entries and hand back the tiles that overflow.
 constexpr int kTileList = 512;
@@ -89,7 +89,7 @@ struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   // a second stream of the context (default priority) on which each pass's
-  // LDS-tile kernel runs beside the per-lane kernel, forked from and joined
+  // LDS-tile kernel runs beside the kernel over heads, forked from and joined
   // back into `stream` by the two events; null: the tile kernels run on
   // `stream` (contexts built for one call, e.g. the allocation-free entry)
   hipStream_t side = nullptr;

@@ -9,28 +9,28 @@
 // neighbors than a tile list holds (kTileList, or kTileListSmall in small
 // batches).  A cell is good when its 27-cell neighborhood holds fewer than
 // kTileMaxCand candidates and, in large batches, no two of its particles
-// coincide (the per-lane passes compute a run of coincident particles once).
+// coincide (the passes over heads compute a run of coincident particles once).
 // The tile computes the particles of its good cells; the other cells of the
-// brick go to the per-lane passes, their particles staged in the halo like
+// brick go to the passes over heads, their particles staged in the halo like
 // any other.  For a tile:
 //
 //   * classify (once per substep): records the tile, the LDS offset of each
 //     halo cell (the cells' particle counts, scanned in halo order z, y, x)
 //     and each halo cell's first slot, and marks the good cells' slots so
-//     that the lane map of the per-lane passes leaves them out;
-//   * neighbors (once per substep; in small batches before the lane map, in
-//     large ones, whose lists cannot overflow, beside the lanes' lists):
+//     that the lists of heads leave them out;
+//   * neighbors (once per substep; in small batches before the heads, in
+//     large ones, whose lists cannot overflow, beside the heads' lists):
 //     stages the halo's p^0 in LDS and writes each particle's neighbor list
 //     as LDS records of the halo: the candidates are the 27 cells in
 //     (dz, dy, dx) order, each
 //     by ascending slot (= ascending id), and candidate j is a neighbor when
 //     it is not the particle itself and |p^0_i - p^0_j|^2 < h^2 (near0, the
 //     reference's list predicate, core.cpp:205-247).  A tile with a particle
-//     of more neighbors than its list holds goes back to the per-lane passes;
+//     of more neighbors than its list holds goes back to the passes over heads;
 //   * each gather pass (lambda, delta, XSPH, omega, eta): stages the halo's
 //     records of the pass in LDS and visits every particle's list in order,
-//     i.e. the reference's list order, with the per-lane term arithmetic of
-//     pbf_kernels.hip, so every sum is bit-identical.
+//     i.e. the reference's list order, with the term arithmetic of
+//     pbf_gather.hip, so every sum is bit-identical.
 //
 // In halo order the three cells (dx = -1, 0, 1) of one (dz, dy) row are
 // consecutive, so a particle's 27 cells are 9 contiguous LDS segments.  A
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kThreads) void k_tile_bricks(
     const int at = base + __popcll(m & ((1ull << lane) - 1ull));
     if (big && at < tile_cap) {
       tile_cand[at] = b;
-    } else if (big) {  // beyond the capacity: the per-lane passes
+    } else if (big) {  // beyond the capacity: the passes over heads
       for (int s = start[b << 6]; s < start[(b << 6) + 64]; ++s) in_tile[s] = 0;
     }
   }
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(kThreads) void k_tile_classify(
   __shared__ int hsrc[kHaloCells];
   __shared__ int scan_lds[kThreads / 64 + 1];
   __shared__ int cst[65];   // the brick's cell starts (slots)
-  __shared__ int cbad[64];  // per brick cell: left to the per-lane passes
+  __shared__ int cbad[64];  // per brick cell: left to the passes over heads
   __shared__ int idx_sh;
   if (tile_fatal(flags)) return;
   const int ncand = min(tile_count[1], tile_cap);
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kThreads) void k_tile_classify(
     }
     __syncthreads();
     // coincident particles (consecutive slots at one position, so in one
-    // cell): in large batches the per-lane passes, which compute a run of
+    // cell): in large batches the passes over heads, which compute a run of
     // them once, take their cell.  Only a brick that can still be a tile
     // (at most kTileMaxHalo slots) is scanned; each thread keeps the cell of
     // its slot (cells lie in slot order) and jumps over excluded cells.
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(kThreads) void k_tile_classify(
       int q = 0;
       for (int s = a + 1 + t; s < e; s += kThreads) {
         while (cst[q + 1] <= s) ++q;
-        if (cbad[q]) {  // left to the per-lane passes: on to the next cell
+        if (cbad[q]) {  // left to the passes over heads: on to the next cell
           s += (cst[q + 1] - s - 1) / kThreads * kThreads;
           continue;
         }
@@ -387,7 +387,7 @@ __device__ __forceinline__ void tile_walk(const uint4* __restrict__ list, int n,
 }
 
 // A tile's slot range [a, e), halo records, scene and first cell; dead: the
-// tile went back to the per-lane passes (a particle with more neighbors than
+// tile went back to the passes over heads (a particle with more neighbors than
 // a tile list holds).
 struct TileInfo {
   int a, e, nrec, sc;
@@ -406,7 +406,7 @@ __device__ __forceinline__ int tiles_of(const int* tile_count, int tile_cap) {
 }
 
 // A tile particle's neighbor count (-1 for a slot of the tile's brick that
-// the per-lane passes compute) and first list chunk.
+// the passes over heads compute) and first list chunk.
 struct Nbrs {
   int cnt;
   uint4 first;  // the list's first chunk
@@ -447,7 +447,7 @@ __device__ __forceinline__ void tile_loop(const TileArgs& ta, int n, int xcd, Ti
     stage_halo(L, T.nrec, fetch, store);
     __syncthreads();
     while (s < T.e) {
-      if (nb.cnt >= 0) body(s, T, nb, x);  // count -1: a cell of the per-lane passes
+      if (nb.cnt >= 0) body(s, T, nb, x);  // count -1: a cell of the passes over heads
       s += kPass;
       if (s < T.e) {
         nb = load_nbrs(ta, n, s);
@@ -464,11 +464,11 @@ __device__ __forceinline__ void tile_loop(const TileArgs& ta, int n, int xcd, Ti
 // as LDS records of the tile's halo, in the 27 cells' (dz, dy, dx) order,
 // each cell by ascending slot (= ascending id); neighbors are the other
 // candidates j with near0(p^0_i, p^0_j).  A tile with a particle of more
-// neighbors than its list holds is dead: its slots go back to the per-lane passes
+// neighbors than its list holds is dead: its slots go back to the passes over heads
 // (in_tile = 0) and the passes skip it.  The slots of the brick's other
 // cells get the count -1.  With nbr (a recorded substep) the
 // live tiles' lists are also stored there as slots (noff, nwords), as the
-// per-lane neighbor kernel stores its lists.
+// heads' kernels store their lists.
 // Candidates tested side by side: 148 us at 1,048,576 particles in place of 161
 // for one at a time (8: the same).  Bound by vector instructions, about 11 a
 // candidate.
@@ -507,7 +507,7 @@ __global__ __launch_bounds__(kPass, kWavesPerSimd) void k_tile_neighbors(
     __syncthreads();
     int over = 0;
     for (int s = T.a + static_cast<int>(threadIdx.x); s < T.e; s += kPass) {
-      if (in_tile[s] == 0) {  // a cell of the per-lane passes: they write its lists
+      if (in_tile[s] == 0) {  // a cell of the passes over heads: they write its lists
         cnt_out[s] = -1;
         continue;
       }
@@ -623,7 +623,7 @@ struct LambdaTerm {
   float w, gx, gy, gz, g2;
 };
 
-// lambda pass (core.cpp:281-329) of the tiles; the per-lane term and its
+// lambda pass (core.cpp:281-329) of the tiles; the same term and
 // accumulation order of k_lambda.  A recorded substep also stores the
 // gradient sum S and the denominator sum Q (sq_out).
 __global__ __launch_bounds__(kPass, kWavesPerSimd) void k_tile_lambda(StepConsts c, TileArgs ta,
@@ -924,10 +924,10 @@ __global__ __launch_bounds__(kPass, kWavesPerSimd) void k_tile_vort_apply(
 
 hipError_t enqueue_tile_classify(Ctx& c, const StepConsts& k) {
   // small batches tile every brick they can (coincident particles
-  // included): their per-lane kernels then have no lanes, whose latency
+  // included): the passes over heads then have no heads, whose latency
   // costs each pass about 20 us for any number of them, and a few small
   // tiles cost little; large ones leave bricks of sparse spray and runs of
-  // coincident particles to the per-lane passes
+  // coincident particles to the passes over heads
   const bool large = c.n >= kForkMinParticles;
   const int min_particles = large ? kTileMinParticles : 1;
   k_tile_bricks<<<1024, kThreads, 0, c.stream>>>(c.start, c.total_cells, c.in_tile, c.tile_count,

@@ -299,7 +299,7 @@ class HipSolver:
         bytes of the rollout recording, substeps the last backward pass
         recomputed, and the bricks the last substep ran as LDS tiles and
         the particles those tiles computed (a tile leaves its brick's dense
-        or coincident cells to the per-lane passes)."""
+        or coincident cells to the passes over heads)."""
         out = (C.c_int64 * 10)()
         _check(self.lib.fluid_hip_get_stats(self.h, out, 10))
         keys = ("pairs", "words", "cells", "list_capacity", "cell_capacity", "grow_events",

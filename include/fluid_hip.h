@@ -92,18 +92,16 @@ typedef struct fluid_hip_config {
                                  (the tile, bounding-box and key kernels; 0, the
                                  default, measured as fast or faster) */
   int32_t record_diag;        /* 1: keep per-step grid diagnostics (slower) */
-  int32_t wave_mode;          /* gathers of wavefronts that share one cell: 0 default (2),
-                                 1 per-lane lists only, 2 shared candidate tiles,
-                                 3 shared tiles without the coincident-tile shortcut */
+  int32_t wave_mode;          /* gather mode: 0 default (2), 1 every particle computed and
+                                 its list stored, 2 runs of identical particles computed
+                                 once, 3 every particle computed (same results) */
   int32_t brick_edge;         /* cells per brick edge of the cell table's Z-order:
                                  0 default (4), 1, 2, 4 or 8 */
-  int64_t lane_capacity;      /* lanes of the gather passes (runs of identical
-                                 particles, each dense cell from a wave boundary):
-                                 0 default (3n + 64), otherwise clamped to
-                                 [n, 3n + 64]; a layout that does not fit
-                                 packs one lane per run */
+  int64_t lane_capacity;      /* 0 default (3n + 64), otherwise clamped to
+                                 [n, 3n + 64]; reported back, no layout
+                                 depends on it any more */
   int32_t tile_gather;        /* passes of sparse 4x4x4-cell bricks through LDS tiles:
-                                 0 default (on from 32,768 particles), 1 on, 2 off; used
+                                 0 default (on from 655,360 particles), 1 on, 2 off; used
                                  with brick edge 4 and gather mode 2 (results are the
                                  same either way) */
 } fluid_hip_config;
@@ -228,7 +226,7 @@ int fluid_hip_get_stats(fluid_hip_ctx* ctx, int64_t* out, int32_t n);
  * the workgroup size (64..1024), the cell table's brick edge (1, 2, 4, 8),
  * the XCD-aware tile order, the LDS-tiled passes of sparse bricks (a
  * kernel-structure choice: one persistent tile kernel per pass, or every
- * particle through the per-lane kernels) and, on request, the gather mode of wavefronts
+ * particle through the passes over heads) and, on request, the gather mode of wavefronts
  * sharing a cell (wave_mode 1..3).  The gather mode is left out by default:
  * which mode is fastest depends on how far particles have piled up, which a
  * short trial at one state does not show.  Every candidate runs
@@ -313,7 +311,7 @@ int fluid_hip_step_noalloc(const fluid_hip_params* params, int64_t n, float* pos
  * "vorticity_omega", "vorticity_apply"; with LDS tiles also "tile_neighbors",
  * "tile_lambda", "tile_delta", "tile_xsph", "tile_vorticity_omega" and
  * "tile_vorticity_apply", the tile kernels alone, timed on the stream they run
- * on (a pass's own name spans its per-lane and tile kernels).  Launches of a substep that
+ * on (a pass's own name spans its kernel over heads and its tile kernel).  Launches of a substep that
  * overflowed a capacity, and of the substeps queued behind it, are not
  * counted (fluid_hip_step runs them again after growing the tables). */
 int fluid_hip_profile(fluid_hip_ctx* ctx, int32_t enable);
