@@ -98,18 +98,19 @@ constexpr int kHead = 1, kList = 2, kDense = 4, kCell = 8;
 // Heads of a dense unit, at most, and the heads of dense cells a batch has for
 // each head of a unit.  A unit's wavefront shares every ordered addition among
 // its heads, but units of more heads are fewer and longer.  Measured (ms per
-// two substeps of the piled-up million-particle block, 56,000 such heads; per
-// four substeps of the splashing 262,144-particle dam breaks, 11,700): units
-// of up to 1 / 4 / 8 heads 51 / 24.7 / 27.3 and 12.0 / 8.1 / 8.1; one more
-// head a unit for every 512 / 2,048 / 4,096 heads 26.9 / 27.3 / 27.5 and 8.8 /
-// 8.1 / 10.6 (units of up to 8).
-constexpr int kUnitHeads = 4;
+// four substeps of the splashing 262,144-particle dam breaks, 11,700 such heads):
+// units of up to 1 / 4 / 8 heads 12.0 / 8.1 / 8.1; one more head a unit for every
+// 512 / 2,048 / 4,096 heads 8.8 / 8.1 / 10.6.  Eight heads only where there are
+// several units of eight for every wavefront on the chip to balance them (ms per
+// two substeps of the piled-up million-particle block, 56,000 such heads: 12.3
+// with four, 10.8 with eight).
+constexpr int kUnitHeads = 8;
 constexpr int kHeadsPerUnitHead = 2048;
 
 // Heads per dense unit (a power of two) for `heads` heads of dense cells.
 __device__ __forceinline__ int unit_heads(int heads) {
   const int k = heads / kHeadsPerUnitHead;
-  return k >= 4 ? kUnitHeads : k >= 2 ? 2 : 1;
+  return k >= 2 * kUnitHeads ? kUnitHeads : k >= 4 ? 4 : k >= 2 ? 2 : 1;
 }
 
 // The class of slot s (0 for slots that are no head; a tile's heads are
@@ -1086,7 +1087,7 @@ __device__ __forceinline__ void pass_lists(const StepConsts& c, const GatherView
 
 // Dense units: a wavefront each, 64 runs of candidates (entries) at a time;
 // those that are neighbors of one of its heads are packed in LDS.  The lanes
-// form G-lane groups, one per head (G = 64 for a single head, 16 for four); a
+// form G-lane groups, one per head (G = 64 for a single head, 8 for eight); a
 // group's lanes compute the packed entries' terms of its head side by side, and
 // then one lane per head and accumulator adds them in order.  All heads of the
 // unit see one sequence of entries, so an entry's multiplicity is uniform: a
@@ -1100,7 +1101,7 @@ __device__ __forceinline__ void pass_lists(const StepConsts& c, const GatherView
 // its longest wavefronts (0.4 us per candidate): lambda of the splashing
 // 32,768-particle dam break took 237 us per launch and takes 28, the
 // 262,144-particle dam breaks' 725 and 96, the piled-up million-particle
-// block's 2,000 and 344 (beside its tiles).
+// block's 2,000 and 292 (beside its tiles).
 template <typename Pass>
 __device__ __forceinline__ void pass_dense(const StepConsts& c, const GatherView& gv,
                                            const Pass& pass, float* lds, float* sums, Ranges& R,
