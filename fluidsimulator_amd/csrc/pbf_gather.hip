@@ -100,9 +100,9 @@ constexpr int kHead = 1, kList = 2, kDense = 4, kCell = 8;
 // its heads, but units of more heads are fewer and longer.  Measured (ms per
 // four substeps of the splashing 262,144-particle dam breaks, 11,700 such heads):
 // units of up to 1 / 4 / 8 heads 12.0 / 8.1 / 8.1; one more head a unit for every
-// 512 / 2,048 / 4,096 heads 8.8 / 8.1 / 10.6.  Eight heads only where there are
-// several units of eight for every wavefront on the chip to balance them (ms per
-// two substeps of the piled-up million-particle block, 56,000 such heads: 12.3
+// 512 / 2,048 / 4,096 heads 8.8 / 8.1 / 10.6.  Eight heads only where that
+// leaves a unit for every wavefront the chip holds at once (4,096; ms per two
+// substeps of the piled-up million-particle block, 56,000 such heads: 12.3
 // with four, 10.8 with eight).
 constexpr int kUnitHeads = 8;
 constexpr int kHeadsPerUnitHead = 2048;
