@@ -165,6 +165,18 @@ __device__ __forceinline__ void for_each_key_group(bool want, int key, Fn&& fn) 
   }
 }
 
+// Waits until the calling wavefront's earlier atomics are done at agent scope.
+// The barrier of a workgroup waits for none of them.
+__device__ __forceinline__ void release_agent() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+}
+
+// kCounted: the caller counts the workgroup as finished after a barrier, and
+// whoever counts it reads the boxes and the flags (k_predict_setup).  A tile of
+// one scene has its box stored by the thread that counts, but the boxes of a
+// tile that straddles scenes, and the range flag, are atomics of any wavefront:
+// each releases its own.
+template <bool kCounted>
 __device__ __forceinline__ void predict_bbox(
     const StepConsts& c, const float4* __restrict__ pos, const float4* __restrict__ vel,
     const ScenePlanes* __restrict__ sp, const int* __restrict__ seg,
@@ -198,7 +210,10 @@ __device__ __forceinline__ void predict_bbox(
     mn1 = mx1 = cy;
     mn2 = mx2 = cz;
   }
-  if (bad) atomicOr(flags, kFlagRange);
+  if (bad) {
+    atomicOr(flags, kFlagRange);
+    if (kCounted) release_agent();
+  }
   const int last = min(base + static_cast<int>(blockDim.x), c.n) - 1;
   if (base > last) return;  // whole block past the end (uniform)
   const int s_first = scene_of(base, seg, c.n_scenes);
@@ -240,6 +255,7 @@ __device__ __forceinline__ void predict_bbox(
         atomicMax(b + 3, b0), atomicMax(b + 4, b1), atomicMax(b + 5, b2);
       }
     });
+    if (kCounted) release_agent();
     if (threadIdx.x == 0) {
       int* b = tile_bbox + 6 * tile;
       b[0] = b[1] = b[2] = INT_MAX;
@@ -384,7 +400,7 @@ __global__ __launch_bounds__(1024) void k_predict_bbox(
     const ScenePlanes* __restrict__ sp, const int* __restrict__ seg,
     uint64_t* __restrict__ cellc, int* __restrict__ bbox, int* __restrict__ tile_bbox,
     unsigned* __restrict__ flags) {
-  predict_bbox(c, pos, vel, sp, seg, cellc, bbox, tile_bbox, flags);
+  predict_bbox<false>(c, pos, vel, sp, seg, cellc, bbox, tile_bbox, flags);
 }
 
 __global__ __launch_bounds__(kGridSetupThreads) void k_grid_setup(GridSetup gs,
@@ -400,10 +416,10 @@ __global__ __launch_bounds__(1024) void k_predict_setup(
     const ScenePlanes* __restrict__ sp, uint64_t* __restrict__ cellc, int* bbox, int* tile_bbox,
     int* finished, unsigned* flags) {
   __shared__ int last_sh;
-  predict_bbox(c, pos, vel, sp, gs.seg, cellc, bbox, tile_bbox, flags);
+  predict_bbox<true>(c, pos, vel, sp, gs.seg, cellc, bbox, tile_bbox, flags);
   __syncthreads();
   if (threadIdx.x == 0) {
-    __threadfence();  // this workgroup's box before its count
+    __threadfence();  // this thread's box before its workgroup's count
     last_sh = atomicAdd(finished, 1) == static_cast<int>(gridDim.x) - 1;
     __threadfence();  // every workgroup's box after the last count
   }
