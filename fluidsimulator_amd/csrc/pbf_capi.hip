@@ -1273,6 +1273,9 @@ int fluid_hip_get_neighbors(fluid_hip_ctx* ctx, int32_t* out, int64_t cap, int64
     }
     HIP_TRY(hipMemcpy(nw.data(), c.nwords, sizeof(int) * n, hipMemcpyDeviceToHost),
             "read lengths");
+    for (size_t s = 0; s < n; ++s)
+      if (nw[s] == fluidhip::kLongList)  // none are built after a substep that failed
+        return fail(FLUID_HIP_ESTATE, "the last step failed: its long lists are gone");
   }
   HIP_TRY(hipMemcpy(off.data(), c.noff, sizeof(long long) * n, hipMemcpyDeviceToHost), "read offsets");
   if (any_tile || any_row) {

@@ -910,10 +910,13 @@ __device__ __forceinline__ int dense_ranges(const GatherView& gv, Ranges& R, int
   return __builtin_amdgcn_readfirstlane(total);
 }
 
-// Neighbor counts of the dense units' heads (statistics).
+// Neighbor counts of the dense units' heads (statistics).  Nothing is counted
+// after a substep that failed, whose arrays are of two substeps.
 __global__ __launch_bounds__(kBlock) void k_count_dense(StepConsts c, GatherView gv,
-                                                        int* __restrict__ ncount) {
+                                                        int* __restrict__ ncount,
+                                                        const unsigned* __restrict__ flags) {
   __shared__ Ranges rng[kWaves];
+  if (fatal(flags)) return;
   const int D = gv.info[2];
   Ranges& R = rng[threadIdx.x / kWave];
   const int nw = static_cast<int>(gridDim.x) * kWaves;
@@ -936,13 +939,15 @@ __global__ __launch_bounds__(kBlock) void k_count_dense(StepConsts c, GatherView
 }
 
 // Every slot's count from its run's head (from the tile lists for tile
-// slots), and the sum of all.
+// slots), and the sum of all (0 after a substep that failed).
 __global__ __launch_bounds__(kBlock) void k_count_slots(int n, const int* __restrict__ run_no,
                                                         const int* __restrict__ rep,
                                                         const int* __restrict__ in_tile,
                                                         const int* __restrict__ tile_cnt,
                                                         int* __restrict__ ncount,
-                                                        unsigned long long* __restrict__ total) {
+                                                        unsigned long long* __restrict__ total,
+                                                        const unsigned* __restrict__ flags) {
+  if (fatal(flags)) return;
   unsigned long long v = 0ull;
   const int stride = static_cast<int>(gridDim.x) * kBlock;
   for (int s = blockIdx.x * kBlock + threadIdx.x; s < n; s += stride) {
@@ -1673,10 +1678,10 @@ hipError_t enqueue_count_pairs(Ctx& c) {
   k_reset_total<<<1, 64, 0, c.stream>>>(c.pair_total);
   if (c.n == 0) return hipGetLastError();
   k_count_dense<<<std::min(kDenseGrid, blocks_for(c.n, kWaves)), kBlock, 0, c.stream>>>(
-      c.consts, gather_view(c, c.pred[0]), c.ncount);
+      c.consts, gather_view(c, c.pred[0]), c.ncount, c.flags);
   k_count_slots<<<std::min(1024, blocks_for(c.n, kBlock)), kBlock, 0, c.stream>>>(
       c.n, c.run_no, c.rep_list, c.consts.tiles ? c.in_tile : nullptr, c.tile_cnt, c.ncount,
-      c.pair_total);
+      c.pair_total, c.flags);
   return hipGetLastError();
 }
 

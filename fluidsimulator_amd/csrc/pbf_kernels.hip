@@ -292,7 +292,6 @@ __device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_
   GridDesc* __restrict__ grid = gs.grid;
   __shared__ long long sh[kGridSetupThreads / kWave];
   __shared__ int box[6 * kLocalBoxes];
-  long long carry = 0;
   // After a failed substep the counters keep what the host needs to size
   // the retry; only the bounding boxes are reset.
   const bool was_fatal = (*flags & kFlagFatal) != 0u;
@@ -330,67 +329,89 @@ __device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_
     }
   }
   __syncthreads();
-  for (int b0 = 0; b0 < n_scenes; b0 += blockDim.x) {
-    const int s = b0 + threadIdx.x;
-    long long nc = 0;
-    GridDesc g{};
-    if (s < n_scenes) {
-      const int* from = (local ? box : bbox) + 6 * s;
-      const long long lx = from[0], ly = from[1], lz = from[2];
-      const long long hx = from[3], hy = from[4], hz = from[5];
-      if (lx <= hx && ly <= hy && lz <= hz) {
-        const long long sx = hx - lx + 3, sy = hy - ly + 3, sz = hz - lz + 3;
-        const long long e = 1ll << bshift;
-        const long long bx = (sx + e - 1) / e, by = (sy + e - 1) / e, bz = (sz + e - 1) / e;
-        nc = (bx * by * bz) << (3 * bshift);
-        g.ox = static_cast<int>(lx - 1);
-        g.oy = static_cast<int>(ly - 1);
-        g.oz = static_cast<int>(lz - 1);
-        g.nbx = static_cast<int>(bx);
-        g.nby = static_cast<int>(by);
-        g.nbz = static_cast<int>(bz);
-      }
-      g.bshift = bshift;
-      int* bb = bbox + 6 * s;
-      bb[0] = INT_MAX, bb[1] = INT_MAX, bb[2] = INT_MAX;
-      bb[3] = INT_MIN, bb[4] = INT_MIN, bb[5] = INT_MIN;
-    }
-    // exclusive scan of nc over the workgroup
-    long long inc = nc;
+  // Cells of scene s's table, and its extents.
+  auto extents = [&](int s, GridDesc& g) {
+    const int* from = (local ? box : bbox) + 6 * s;
+    const long long lx = from[0], ly = from[1], lz = from[2];
+    const long long hx = from[3], hy = from[4], hz = from[5];
+    g = GridDesc{};
+    g.bshift = bshift;
+    if (lx > hx || ly > hy || lz > hz) return 0ll;
+    const long long sx = hx - lx + 3, sy = hy - ly + 3, sz = hz - lz + 3;
+    const long long e = 1ll << bshift;
+    const long long bx = (sx + e - 1) / e, by = (sy + e - 1) / e, bz = (sz + e - 1) / e;
+    g.ox = static_cast<int>(lx - 1);
+    g.oy = static_cast<int>(ly - 1);
+    g.oz = static_cast<int>(lz - 1);
+    g.nbx = static_cast<int>(bx);
+    g.nby = static_cast<int>(by);
+    g.nbz = static_cast<int>(bz);
+    return (bx * by * bz) << (3 * bshift);
+  };
+  // Exclusive prefix of one value per thread; `all` receives the sum.
+  auto prefix = [&](long long v, long long& all) {
+    long long inc = v;
     for (int o = 1; o < kWave; o <<= 1) {
       const long long u = __shfl_up(inc, o, kWave);
       if (lane >= o) inc += u;
     }
     if (lane == kWave - 1) sh[w] = inc;
     __syncthreads();
-    long long before = 0, all = 0;
+    long long before = 0;
+    all = 0;
     for (int u = 0; u < nw; ++u) {
       before += u < w ? sh[u] : 0;
       all += sh[u];
     }
-    const long long excl = inc - nc + before + carry;
+    __syncthreads();  // sh is reused
+    return inc - v + before;
+  };
+  // The scenes' cells in all come first: a substep that fails leaves the grid of
+  // the last good one, which belongs to the other arrays of that substep.
+  GridDesc g{};
+  long long total = 0, carry = 0;
+  long long nc = 0, excl = 0;
+  for (int b0 = 0; b0 < n_scenes; b0 += blockDim.x) {
+    const int s = b0 + threadIdx.x;
+    nc = s < n_scenes ? extents(s, g) : 0;
+    long long all;
+    excl = prefix(nc, all);
+    total += all;
+  }
+  const bool fits = total <= cell_cap;
+  for (int b0 = 0; b0 < n_scenes; b0 += blockDim.x) {
+    const int s = b0 + threadIdx.x;
+    long long all = total;
+    if (n_scenes > static_cast<int>(blockDim.x)) {  // otherwise as computed above
+      nc = s < n_scenes ? extents(s, g) : 0;
+      excl = prefix(nc, all);
+    }
     if (s < n_scenes) {
-      g.cell_off = static_cast<int>(excl < cell_cap ? excl : 0);
-      g.ncells = static_cast<int>(nc < cell_cap ? nc : 0);
-      grid[s] = g;
+      if (fits && !was_fatal) {
+        g.cell_off = static_cast<int>(excl + carry);
+        g.ncells = static_cast<int>(nc);
+        grid[s] = g;
+      }
+      int* bb = bbox + 6 * s;
+      bb[0] = INT_MAX, bb[1] = INT_MAX, bb[2] = INT_MAX;
+      bb[3] = INT_MIN, bb[4] = INT_MIN, bb[5] = INT_MIN;
     }
     carry += all;
-    __syncthreads();  // sh is reused
   }
   if (threadIdx.x == 0 && !was_fatal) {
-    *gs.nbr_total = 0ull;
-    gs.info[2] = 0;  // dense units
-    if (gs.tile_count) {
-      gs.tile_count[0] = 0;  // tiles
-      gs.tile_count[1] = 0;  // candidate bricks
-    }
-    if (carry > cell_cap) {
+    if (fits) {
+      *gs.nbr_total = 0ull;
+      gs.info[2] = 0;  // dense units
+      if (gs.tile_count) {
+        gs.tile_count[0] = 0;  // tiles
+        gs.tile_count[1] = 0;  // candidate bricks
+      }
+      *gs.total_cells = static_cast<int>(total);
+      atomicAdd(gs.steps_started, 1);
+    } else {
       atomicOr(flags, kFlagCells);
       *gs.total_cells = 0;
-      *gs.need_cells = static_cast<unsigned long long>(carry);
-    } else {
-      *gs.total_cells = static_cast<int>(carry);
-      atomicAdd(gs.steps_started, 1);
+      *gs.need_cells = static_cast<unsigned long long>(total);
     }
   }
 }
