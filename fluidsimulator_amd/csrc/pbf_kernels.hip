@@ -330,13 +330,13 @@ __device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_
   }
   __syncthreads();
   // Cells of scene s's table, and its extents.
-  auto extents = [&](int s, GridDesc& g) {
+  auto extents = [&](int s, GridDesc& g) -> long long {
     const int* from = (local ? box : bbox) + 6 * s;
     const long long lx = from[0], ly = from[1], lz = from[2];
     const long long hx = from[3], hy = from[4], hz = from[5];
     g = GridDesc{};
     g.bshift = bshift;
-    if (lx > hx || ly > hy || lz > hz) return 0ll;
+    if (lx > hx || ly > hy || lz > hz) return 0;
     const long long sx = hx - lx + 3, sy = hy - ly + 3, sz = hz - lz + 3;
     const long long e = 1ll << bshift;
     const long long bx = (sx + e - 1) / e, by = (sy + e - 1) / e, bz = (sz + e - 1) / e;
@@ -346,7 +346,10 @@ __device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_
     g.nbx = static_cast<int>(bx);
     g.nby = static_cast<int>(by);
     g.nbz = static_cast<int>(bz);
-    return (bx * by * bz) << (3 * bshift);
+    // (a table this large never fits, and neither the product nor the sum over
+    // scenes that lie in the whole coordinate range fits 64 bits)
+    const long long many = 1ll << 40;
+    return min(min(bx * by, many) * bz, many) << (3 * bshift);
   };
   // Exclusive prefix of one value per thread; `all` receives the sum.
   auto prefix = [&](long long v, long long& all) {

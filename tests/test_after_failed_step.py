@@ -96,3 +96,21 @@ def test_queries_after_a_failed_substep(kind, tiles, how):
         r = s.download()
         assert same_bits(r.pos, o["pos"]) and same_bits(r.vel, o["vel"])
         assert s.stats()["pairs"] == int(o["nbr_count"].astype(np.int64).sum())
+
+
+@pytest.mark.parametrize("edge", [1, 2, 4, 8])
+@pytest.mark.parametrize("count", [1, 2, 40])
+def test_scenes_over_the_whole_coordinate_range_do_not_fit(edge, count):
+    """Particles at opposite corners of the range of cell coordinates: the cells
+    of the table, in one scene or in all, exceed 64 bits."""
+    p = scenes.base_params((4.0, 4.0, 4.0), False)
+    p.planes = []
+    p.external_forces = (0.0, 0.0, 0.0)
+    end = 0.0999999 * (1 << 20)
+    pos = np.tile(np.array([[-end, end]] * 3, np.float32), (1, count))
+    with hip.HipSolver([p] * count, [2] * count, brick_edge=edge) as s:
+        s.upload(pos, np.zeros_like(pos))
+        with pytest.raises(hip.HipError) as e:
+            s.step(1)
+        assert e.value.code == hip.ECAPACITY
+        assert same_bits(s.download().pos, pos)
