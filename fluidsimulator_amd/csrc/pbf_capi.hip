@@ -440,7 +440,11 @@ void free_all(Ctx& c) {
   c.prof.pool.clear();
 }
 
+// The cell table, or the lists' words, in a block of `cap` entries; what the old
+// one held is gone.  A captured substep holds the old address.  After a failure
+// there is no block (ensure_tables makes one of the former capacity).
 int alloc_cells(Ctx& c, long long cap) {
+  drop_graph(c);
   give_block(c.device, c.start, c.start_bytes);
   c.start = nullptr;
   HIP_TRY(take_array(c.device, static_cast<size_t>(cap) + 1, &c.start, &c.start_bytes),
@@ -450,11 +454,20 @@ int alloc_cells(Ctx& c, long long cap) {
 }
 
 int alloc_neighbors(Ctx& c, long long cap) {
+  drop_graph(c);
   give_block(c.device, c.nbr, c.nbr_bytes);
   c.nbr = nullptr;
   HIP_TRY(take_array(c.device, static_cast<size_t>(cap), &c.nbr, &c.nbr_bytes),
           "hipMalloc(neighbor list)");
   c.nbr_cap = cap;
+  return FLUID_HIP_OK;
+}
+
+// Before any substep: a table that an earlier call could not grow.
+int ensure_tables(Ctx& c) {
+  int rc;
+  if (!c.start && (rc = alloc_cells(c, c.cell_cap))) return rc;
+  if (!c.nbr && (rc = alloc_neighbors(c, c.nbr_cap))) return rc;
   return FLUID_HIP_OK;
 }
 
@@ -479,6 +492,8 @@ int collect_profile(Ctx& c, int keep_steps = INT_MAX) {
 }
 
 int queue_steps(Ctx& c, int nsteps, bool use_graph) {
+  const int rc = ensure_tables(c);
+  if (rc) return rc;
   if (use_graph && c.n > 0) {
     if (!c.graph_exec) {
       // The graph holds every buffer address of one substep: it is dropped
@@ -561,7 +576,9 @@ int check_ctx(fluid_hip_ctx* ctx) {
 
 // After a substep that raised a capacity flag: grow the table it reported
 // (geometrically, at least to 1.5x the need) so that the substep can be
-// replayed; the committed state of a failed substep is left untouched.
+// replayed; the committed state of a failed substep is left untouched.  The last
+// good substep's cells or lists go with the old table: until a substep has run
+// there is nothing to query.
 int grow_tables(Ctx& c, const DevStatus& st) {
   int rc;
   if (st.flags & fluidhip::kFlagCells) {
@@ -569,16 +586,17 @@ int grow_tables(Ctx& c, const DevStatus& st) {
     const long long cap = std::max(need + need / 2 + 4096, 2 * c.cell_cap);
     if (need + 4096 >= INT_MAX)
       return fail(FLUID_HIP_ECAPACITY, "cell table would exceed 2^31 cells");
+    c.stepped = false;
     if ((rc = alloc_cells(c, std::min<long long>(cap, INT_MAX - 1)))) return rc;
   } else {
     const long long need = static_cast<long long>(st.nbr_total);
     const long long cap = std::max(need + need / 2 + 4096, 2 * c.nbr_cap);
+    c.stepped = false;
     if ((rc = alloc_neighbors(c, cap))) {
       g_last_error = "neighbor list of " + std::to_string(cap) + " words: " + g_last_error;
       return FLUID_HIP_ECAPACITY;
     }
   }
-  drop_graph(c);
   ++c.grow_events;
   return FLUID_HIP_OK;
 }
@@ -658,6 +676,7 @@ int record_segment(Ctx& c, AdjRecord& a, int sg, int len) {
   auto& b = a.buf;
   if (!b.tape_need) HIP_TRY(dalloc(&b.tape_need, 1), "hipMalloc(tape need)");
   int rc;
+  if ((rc = ensure_tables(c))) return rc;
   for (int attempt = 0; attempt < 16; ++attempt) {
     if (attempt > 0) {
       if ((rc = load_state(c, a.ck_pos[sg], a.ck_vel[sg]))) return rc;
@@ -1259,6 +1278,7 @@ int fluid_hip_get_neighbors(fluid_hip_ctx* ctx, int32_t* out, int64_t cap, int64
   }
   if (any_long) {
     // the words buffer holds nothing else then
+    if ((rc = ensure_tables(c))) return rc;
     for (int attempt = 0; attempt < 2; ++attempt) {
       HIP_TRY(fluidhip::enqueue_long_lists(c), "long lists");
       unsigned long long need = 0;
@@ -1266,10 +1286,10 @@ int fluid_hip_get_neighbors(fluid_hip_ctx* ctx, int32_t* out, int64_t cap, int64
               "read total");
       HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
       if (need <= static_cast<unsigned long long>(c.nbr_cap)) break;
-      drop_graph(c);
-      if ((rc = alloc_neighbors(c, static_cast<long long>(need)))) return rc;
+      // those that did fit are gone with the old buffer, also when there is no new one
       HIP_TRY(hipMemcpy(c.nwords, nw.data(), sizeof(int) * n, hipMemcpyHostToDevice),
               "restore lengths");
+      if ((rc = alloc_neighbors(c, static_cast<long long>(need)))) return rc;
     }
     HIP_TRY(hipMemcpy(nw.data(), c.nwords, sizeof(int) * n, hipMemcpyDeviceToHost),
             "read lengths");
