@@ -713,6 +713,7 @@ int record_segment(Ctx& c, AdjRecord& a, int sg, int len) {
       for (auto& t : a.tapes)
         if (t.nbr_cap < cap) {
           dfree(t.nbr);
+          t.nbr_cap = 0;
           HIP_TRY(dalloc(&t.nbr, static_cast<size_t>(cap)), "hipMalloc(tape neighbor lists)");
           t.nbr_cap = cap;
         }
@@ -1660,11 +1661,18 @@ int fluid_hip_forward_record(fluid_hip_ctx* ctx, int32_t nsteps, int32_t checkpo
     if (!c.adj) return fail(FLUID_HIP_EHIP, "out of host memory");
     auto& b = c.adj->buf;
     const size_t n = static_cast<size_t>(std::max(c.n, 1));
+    hipError_t e = hipSuccess;
     for (float4** p : {&b.GX, &b.GV, &b.U, &b.PB, &b.XB, &b.W, &b.LB})
-      HIP_TRY(dalloc(p, n), "hipMalloc(adjoint buffers)");
-    HIP_TRY(dalloc(&b.RB, n), "hipMalloc(adjoint buffers)");
-    HIP_TRY(dalloc(&b.gacc, 3 * static_cast<size_t>(c.n_scenes)), "hipMalloc(adjoint buffers)");
-    HIP_TRY(dalloc(&b.stage, 6 * n), "hipMalloc(adjoint buffers)");
+      if (e == hipSuccess) e = dalloc(p, n);
+    if (e == hipSuccess) e = dalloc(&b.RB, n);
+    if (e == hipSuccess) e = dalloc(&b.gacc, 3 * static_cast<size_t>(c.n_scenes));
+    if (e == hipSuccess) e = dalloc(&b.stage, 6 * n);
+    if (e == hipSuccess) e = dalloc(&c.adj->fin_pos, n);
+    if (e == hipSuccess) e = dalloc(&c.adj->fin_vel, n);
+    if (e != hipSuccess) {
+      free_adj(c);  // all of them or none
+      return hip_fail(e, "hipMalloc(adjoint buffers)");
+    }
   }
   AdjRecord& a = *c.adj;
   a.valid = false;
@@ -1681,8 +1689,12 @@ int fluid_hip_forward_record(fluid_hip_ctx* ctx, int32_t nsteps, int32_t checkpo
   while (static_cast<int>(a.ck_pos.size()) < nseg) {
     float4 *p = nullptr, *v = nullptr;
     HIP_TRY(dalloc(&p, n), "hipMalloc(checkpoint)");
+    const hipError_t e = dalloc(&v, n);
+    if (e != hipSuccess) {
+      dfree(p);
+      return hip_fail(e, "hipMalloc(checkpoint)");
+    }
     a.ck_pos.push_back(p);
-    HIP_TRY(dalloc(&v, n), "hipMalloc(checkpoint)");
     a.ck_vel.push_back(v);
   }
   a.ck_time.assign(nseg, 0.0f);
@@ -1696,12 +1708,9 @@ int fluid_hip_forward_record(fluid_hip_ctx* ctx, int32_t nsteps, int32_t checkpo
     a.tapes.pop_back();
   }
   while (static_cast<int>(a.tapes.size()) < ntapes) {
-    a.tapes.emplace_back();
-    if ((rc = alloc_tape(c, a.tapes.back()))) return rc;
-  }
-  if (!a.fin_pos) {
-    HIP_TRY(dalloc(&a.fin_pos, n), "hipMalloc(final state)");
-    HIP_TRY(dalloc(&a.fin_vel, n), "hipMalloc(final state)");
+    SubTape t;
+    if ((rc = alloc_tape(c, t))) return rc;
+    a.tapes.push_back(t);
   }
   for (int sg = 0; sg < nseg; ++sg) {
     const int s0 = sg * checkpoint_every;

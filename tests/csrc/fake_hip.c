@@ -249,10 +249,10 @@ int hipLaunchKernel(const void* host, dim3_t grid, dim3_t block, void** args, si
       *(unsigned long long*)ptr(args, 8) = fake_total;
     }
   } else if (strstr(name, "k_tape_copy")) {
-    need(args, 6, "k_tape_copy without a list buffer");
-    need(args, 8, "k_tape_copy without a tape");
-    need_list(args, 12, "k_tape_copy without a tape's list buffer");
-    if (fake_tape_need) *(unsigned long long*)ptr(args, 14) = fake_tape_need;
+    need(args, 7, "k_tape_copy without a list buffer");
+    need(args, 9, "k_tape_copy without a tape");
+    need_list(args, 15, "k_tape_copy without a tape's list buffer");
+    if (fake_tape_need) *(unsigned long long*)ptr(args, 17) = fake_tape_need;
     fake_tape_need = 0;
   } else if (strstr(name, "k_adj_seed")) {
     need(args, 1, "k_adj_seed without a tape");

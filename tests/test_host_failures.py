@@ -150,6 +150,40 @@ def lists_built_on_request(fake):
     s.close()
 
 
+@case
+def recording(fake):
+    from fluidsimulator_amd import hip
+
+    failed = 0
+    for at in range(100):
+        s = solver()
+        fake.fail_malloc(at=at)
+        bad = raises(hip.EHIP, s.forward_record, 6, 3)
+        fake.works()
+        failed += bad
+        if bad:
+            assert raises(hip.ESTATE, s.backward)
+        for steps, every in ((6, 3), (4, 2)):
+            s.forward_record(steps, every)
+            s.backward()
+        fake.check()
+        s.close()
+        if not bad:
+            break
+    assert failed > 10
+    # a tape whose lists outgrew it
+    s = solver()
+    s.forward_record(4, 2)
+    fake.tape_need = 12345
+    fake.fail_malloc()
+    assert raises(hip.EHIP, s.forward_record, 4, 2)
+    fake.works()
+    s.forward_record(4, 2)
+    s.backward()
+    fake.check()
+    s.close()
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_host_path(runtime, name):
     env = dict(os.environ, LD_LIBRARY_PATH=runtime, PYTHONPATH=ROOT)
