@@ -349,7 +349,9 @@ __device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_
     // (a table this large never fits, and neither the product nor the sum over
     // scenes that lie in the whole coordinate range fits 64 bits)
     const long long many = 1ll << 40;
-    return min(min(bx * by, many) * bz, many) << (3 * bshift);
+    const long long layer = bx * by < many ? bx * by : many;
+    const long long bricks = layer * bz < many ? layer * bz : many;
+    return bricks << (3 * bshift);
   };
   // Exclusive prefix of one value per thread; `all` receives the sum.
   auto prefix = [&](long long v, long long& all) {
