@@ -230,12 +230,17 @@ std::vector<fluidhip::ScenePlanes> scene_tables(const Ctx& c) {
 // context for every substep, and hipMalloc and hipFree of its buffers took 0.9
 // to 2.5 ms of each call (of the 1,728-particle call's 2.0 ms in all, and up to
 // 3.9 ms), hipFree of the two 64 MiB cell arrays alone 0.5 ms.  Bounded:
-// at most kKeepBytes over all devices (more is freed, oldest first) and
-// kKeepStreams stream sets; given back when an allocation fails.  A block is
-// kept only once the work that used it has finished, and belongs to nobody
-// until it is handed out again, so any thread may take it.
+// at most kKeepBytes in kKeepBlocks blocks over all devices (more is freed,
+// oldest first; a block that is larger alone is freed at once and drives no
+// other out) and kKeepStreams stream sets.  Given back when an allocation fails,
+// or by fluid_hip_release_kept.  A block is kept only once the work that used it
+// has finished, and belongs to nobody until it is handed out again, so any
+// thread may take it.  hipDeviceReset frees what is kept: a mark, a small
+// allocation of an unusual size, says whether that has happened to a device.
 constexpr size_t kKeepBytes = static_cast<size_t>(256) << 20;
-constexpr size_t kKeepStreams = 4;
+constexpr int kKeepBlocks = 64;
+constexpr int kKeepStreams = 4;
+constexpr size_t kMarkBytes = 4099;
 
 struct Kept {
   struct Block {
@@ -249,13 +254,50 @@ struct Kept {
     hipEvent_t fork, join;
   };
   std::mutex mu;
-  std::vector<Block> blocks;  // oldest first
+  Block blocks[kKeepBlocks];  // oldest first
+  int n_blocks = 0;
   size_t bytes = 0;
-  std::vector<Streams> streams;
+  Streams streams[kKeepStreams];
+  int n_streams = 0;
+  Block marks[kKeepBlocks];  // one per device
+  int n_marks = 0;
+
+  Block take(int i) {
+    const Block b = blocks[i];
+    bytes -= b.bytes;
+    std::copy(blocks + i + 1, blocks + n_blocks--, blocks + i);
+    return b;
+  }
+  Streams take_streams(int i) {
+    const Streams s = streams[i];
+    std::copy(streams + i + 1, streams + n_streams--, streams + i);
+    return s;
+  }
+  // What is kept of a device that was reset since is gone.
+  void forget(int device) {
+    for (int i = n_blocks - 1; i >= 0; --i)
+      if (blocks[i].device == device) (void)take(i);
+    for (int i = n_streams - 1; i >= 0; --i)
+      if (streams[i].device == device) (void)take_streams(i);
+  }
 };
 Kept& kept() {
   static Kept* k = new Kept();  // never destroyed: contexts may outlive statics
   return *k;
+}
+
+// Frees kept blocks, oldest first, until at most `bytes` in `count` are left.
+void shrink_kept(size_t bytes, int count) {
+  Kept& k = kept();
+  for (;;) {
+    Kept::Block b;
+    {
+      std::lock_guard<std::mutex> lock(k.mu);
+      if (k.bytes <= bytes && k.n_blocks <= count) return;
+      b = k.take(0);
+    }
+    (void)hipFree(b.p);
+  }
 }
 
 // hipMalloc; when memory runs out, again without the kept blocks.
@@ -263,15 +305,39 @@ hipError_t device_malloc(void** p, size_t bytes) {
   const hipError_t e = hipMalloc(p, bytes);
   if (e != hipErrorOutOfMemory) return e;
   (void)hipGetLastError();
-  Kept& k = kept();
-  std::vector<Kept::Block> out;
-  {
-    std::lock_guard<std::mutex> lock(k.mu);
-    out.swap(k.blocks);
-    k.bytes = 0;
-  }
-  for (auto& b : out) (void)hipFree(b.p);
+  shrink_kept(0, 0);
   return hipMalloc(p, bytes);
+}
+
+// Before a context takes anything kept of the current device: forgets it all
+// when the device was reset since.
+void check_kept(int device) {
+  Kept& k = kept();
+  std::lock_guard<std::mutex> lock(k.mu);
+  int i = 0;
+  while (i < k.n_marks && k.marks[i].device != device) ++i;
+  if (i < k.n_marks) {
+    hipDeviceptr_t base = nullptr;
+    size_t bytes = 0;
+    const hipError_t e = hipMemGetAddressRange(&base, &bytes, k.marks[i].p);
+    if (e == hipSuccess && base == k.marks[i].p && bytes == kMarkBytes) return;
+    (void)hipGetLastError();
+    k.marks[i] = k.marks[--k.n_marks];
+  }
+  k.forget(device);
+  if (k.n_marks == kKeepBlocks) return;  // nothing is kept without a mark
+  void* p = nullptr;
+  if (hipMalloc(&p, kMarkBytes) == hipSuccess)
+    k.marks[k.n_marks++] = {device, p, kMarkBytes};
+  else
+    (void)hipGetLastError();
+}
+
+// (under the lock)
+bool has_mark(const Kept& k, int device) {
+  for (int i = 0; i < k.n_marks; ++i)
+    if (k.marks[i].device == device) return true;
+  return false;
 }
 
 template <typename T>
@@ -292,42 +358,41 @@ void dfree(T*& p) {
 hipError_t take_block(int device, size_t bytes, void** p, size_t* got) {
   *p = nullptr;
   *got = bytes;
-  Kept& k = kept();
   {
+    Kept& k = kept();
     std::lock_guard<std::mutex> lock(k.mu);
-    size_t best = k.blocks.size();
-    for (size_t i = 0; i < k.blocks.size(); ++i) {
+    int best = -1;
+    for (int i = 0; i < k.n_blocks; ++i) {
       const Kept::Block& b = k.blocks[i];
       if (b.device == device && b.bytes >= bytes && b.bytes / 2 <= bytes &&
-          (best == k.blocks.size() || b.bytes < k.blocks[best].bytes))
+          (best < 0 || b.bytes < k.blocks[best].bytes))
         best = i;
     }
-    if (best < k.blocks.size()) {
-      *p = k.blocks[best].p;
-      *got = k.blocks[best].bytes;
-      k.bytes -= *got;
-      k.blocks.erase(k.blocks.begin() + static_cast<long>(best));
+    if (best >= 0) {
+      const Kept::Block b = k.take(best);
+      *p = b.p;
+      *got = b.bytes;
       return hipSuccess;
     }
   }
   return device_malloc(p, bytes);
 }
 
-// Gives back a block whose work has finished.
-void give_block(int device, void* p, size_t bytes) {
+// Gives back a block; `idle`: the work that used it is known to have finished
+// (hipFree waits for it otherwise).
+void give_block(int device, void* p, size_t bytes, bool idle) {
   if (!p) return;
-  Kept& k = kept();
-  std::vector<Kept::Block> out;
-  {
+  if (idle && bytes <= kKeepBytes) {
+    shrink_kept(kKeepBytes - bytes, kKeepBlocks - 1);
+    Kept& k = kept();
     std::lock_guard<std::mutex> lock(k.mu);
-    k.blocks.push_back({device, p, bytes});
-    k.bytes += bytes;
-    size_t n = 0;
-    while (k.bytes > kKeepBytes) k.bytes -= k.blocks[n++].bytes;
-    out.assign(k.blocks.begin(), k.blocks.begin() + static_cast<long>(n));
-    k.blocks.erase(k.blocks.begin(), k.blocks.begin() + static_cast<long>(n));
+    if (k.bytes + bytes <= kKeepBytes && k.n_blocks < kKeepBlocks && has_mark(k, device)) {
+      k.blocks[k.n_blocks++] = {device, p, bytes};
+      k.bytes += bytes;
+      return;
+    }
   }
-  for (auto& b : out) (void)hipFree(b.p);
+  (void)hipFree(p);
 }
 
 template <typename T>
@@ -421,12 +486,13 @@ void drop_graph(Ctx& c) {
 
 void free_adj(Ctx& c);
 
-void free_all(Ctx& c) {
+// `idle`: the context's work is known to have finished.
+void free_all(Ctx& c, bool idle) {
   drop_graph(c);
   free_adj(c);
-  give_block(c.device, c.arena, c.arena_bytes);
-  give_block(c.device, c.start, c.start_bytes);
-  give_block(c.device, c.nbr, c.nbr_bytes);
+  give_block(c.device, c.arena, c.arena_bytes, idle);
+  give_block(c.device, c.start, c.start_bytes, idle);
+  give_block(c.device, c.nbr, c.nbr_bytes, idle);
   c.arena = nullptr;
   c.start = c.nbr = nullptr;
   for (auto& q : c.prof.pending) {
@@ -441,11 +507,11 @@ void free_all(Ctx& c) {
 }
 
 // The cell table, or the lists' words, in a block of `cap` entries; what the old
-// one held is gone.  A captured substep holds the old address.  After a failure
+// one held is gone (no work that uses it is queued).  A captured substep holds the old address.  After a failure
 // there is no block (ensure_tables makes one of the former capacity).
 int alloc_cells(Ctx& c, long long cap) {
   drop_graph(c);
-  give_block(c.device, c.start, c.start_bytes);
+  give_block(c.device, c.start, c.start_bytes, true);
   c.start = nullptr;
   HIP_TRY(take_array(c.device, static_cast<size_t>(cap) + 1, &c.start, &c.start_bytes),
           "hipMalloc(cell starts)");
@@ -455,7 +521,7 @@ int alloc_cells(Ctx& c, long long cap) {
 
 int alloc_neighbors(Ctx& c, long long cap) {
   drop_graph(c);
-  give_block(c.device, c.nbr, c.nbr_bytes);
+  give_block(c.device, c.nbr, c.nbr_bytes, true);
   c.nbr = nullptr;
   HIP_TRY(take_array(c.device, static_cast<size_t>(cap), &c.nbr, &c.nbr_bytes),
           "hipMalloc(neighbor list)");
@@ -779,13 +845,13 @@ int noalloc_scratch(int dev, unsigned char** out) {
 
 // The context's streams and events: kept ones, or new ones.
 hipError_t make_streams(Ctx& c) {
-  Kept& k = kept();
+  check_kept(c.device);
   {
+    Kept& k = kept();
     std::lock_guard<std::mutex> lock(k.mu);
-    for (size_t i = 0; i < k.streams.size(); ++i)
+    for (int i = 0; i < k.n_streams; ++i)
       if (k.streams[i].device == c.device) {
-        const Kept::Streams s = k.streams[i];
-        k.streams.erase(k.streams.begin() + static_cast<long>(i));
+        const Kept::Streams s = k.take_streams(i);
         c.stream = s.main;
         c.own_stream = true;
         c.side = s.side;
@@ -804,18 +870,24 @@ hipError_t make_streams(Ctx& c) {
   return e;
 }
 
+void close_streams(Ctx& c);
+
 // Gives back the context's own streams and events (the main stream only when
-// it is not the caller's); their work has finished.
-void destroy_streams(Ctx& c) {
-  if (c.own_stream && c.stream && c.side && c.ev_fork && c.ev_join) {
+// it is not the caller's); `idle`: their work is known to have finished.
+void destroy_streams(Ctx& c, bool idle) {
+  if (idle && c.own_stream && c.stream && c.side && c.ev_fork && c.ev_join) {
     Kept& k = kept();
     std::lock_guard<std::mutex> lock(k.mu);
-    if (k.streams.size() < kKeepStreams) {
-      k.streams.push_back({c.device, c.stream, c.side, c.ev_fork, c.ev_join});
+    if (k.n_streams < kKeepStreams && has_mark(k, c.device)) {
+      k.streams[k.n_streams++] = {c.device, c.stream, c.side, c.ev_fork, c.ev_join};
       c.stream = c.side = nullptr;
       c.ev_fork = c.ev_join = nullptr;
     }
   }
+  close_streams(c);
+}
+
+void close_streams(Ctx& c) {
   if (c.ev_fork) hipEventDestroy(c.ev_fork);
   if (c.ev_join) hipEventDestroy(c.ev_join);
   if (c.side) hipStreamDestroy(c.side);
@@ -936,8 +1008,10 @@ int fluid_hip_create(fluid_hip_ctx** out, int32_t n_scenes, const int64_t* scene
   compute_consts(c);
 
   auto bail = [&](int code) {
-    free_all(c);
-    destroy_streams(c);
+    // copies and kernels may be queued already
+    const bool idle = c.stream && hipStreamSynchronize(c.stream) == hipSuccess;
+    free_all(c, idle);
+    destroy_streams(c, idle);
     delete h;
     return code;
   };
@@ -996,11 +1070,48 @@ int fluid_hip_create(fluid_hip_ctx** out, int32_t n_scenes, const int64_t* scene
 int fluid_hip_destroy(fluid_hip_ctx* ctx) {
   if (!ctx) return FLUID_HIP_OK;
   hipSetDevice(ctx->c.device);
-  if (ctx->c.stream) hipStreamSynchronize(ctx->c.stream);
-  if (ctx->c.side) hipStreamSynchronize(ctx->c.side);
-  free_all(ctx->c);
-  destroy_streams(ctx->c);
+  // what may still be in use (a caller's stream that is gone or capturing, an
+  // earlier error) is freed, not kept
+  bool idle = true;
+  if (ctx->c.stream) idle &= hipStreamSynchronize(ctx->c.stream) == hipSuccess;
+  if (ctx->c.side) idle &= hipStreamSynchronize(ctx->c.side) == hipSuccess;
+  free_all(ctx->c, idle);
+  destroy_streams(ctx->c, idle);
   delete ctx;
+  return FLUID_HIP_OK;
+}
+
+int fluid_hip_release_kept(void) {
+  shrink_kept(0, 0);
+  int dev = 0;
+  const bool restore = hipGetDevice(&dev) == hipSuccess;
+  Kept& k = kept();
+  for (;;) {
+    Kept::Streams s{};
+    Kept::Block m{};
+    {
+      std::lock_guard<std::mutex> lock(k.mu);
+      if (k.n_streams > 0)
+        s = k.take_streams(k.n_streams - 1);
+      else if (k.n_marks > 0 && k.n_blocks == 0)
+        m = k.marks[--k.n_marks];
+    }
+    if (s.main) {
+      Ctx c;
+      c.stream = s.main;
+      c.own_stream = true;
+      c.side = s.side;
+      c.ev_fork = s.fork;
+      c.ev_join = s.join;
+      hipSetDevice(s.device);
+      close_streams(c);
+    } else if (m.p) {
+      (void)hipFree(m.p);
+    } else {
+      break;
+    }
+  }
+  if (restore) hipSetDevice(dev);
   return FLUID_HIP_OK;
 }
 

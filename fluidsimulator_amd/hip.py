@@ -66,6 +66,7 @@ _SIGS = {
     "fluid_hip_create": (C.c_int, [C.POINTER(C.c_void_p), C.c_int32, C.POINTER(C.c_int64),
                                    C.POINTER(FluidHipParams), C.POINTER(FluidHipConfig)]),
     "fluid_hip_destroy": (C.c_int, [C.c_void_p]),
+    "fluid_hip_release_kept": (C.c_int, []),
     "fluid_hip_set_params": (C.c_int, [C.c_void_p, C.POINTER(FluidHipParams)]),
     "fluid_hip_set_stream": (C.c_int, [C.c_void_p, C.c_void_p]),
     "fluid_hip_upload": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_float]),
@@ -146,6 +147,12 @@ def hip_device_available():
     err = C.c_char_p()
     ok = load_library().fluid_hip_device_available(C.byref(cnt), C.byref(err))
     return bool(ok), int(cnt.value), (err.value.decode() if err.value else None)
+
+
+def release_kept() -> None:
+    """Frees the device memory (up to 256 MiB) and streams that destroyed
+    contexts left for the next ones."""
+    _check(load_library().fluid_hip_release_kept())
 
 
 def pack_params(p: Params) -> FluidHipParams:

@@ -134,7 +134,18 @@ const char* fluid_hip_last_error(void);
  */
 int fluid_hip_create(fluid_hip_ctx** out, int32_t n_scenes, const int64_t* scene_counts,
                      const fluid_hip_params* params, const fluid_hip_config* config);
+
+/* Destroys a context.  Its device memory and streams are kept for the next
+ * contexts of the process (a stateless substep creates and destroys one): at
+ * most 256 MiB in 64 blocks, and 4 sets of two streams, over all devices.  A
+ * block that may still be in use (a stream of the caller's that is gone or
+ * capturing), or that is larger than that alone, is freed.  Kept blocks are
+ * freed when one of the library's own allocations finds no memory. */
 int fluid_hip_destroy(fluid_hip_ctx* ctx);
+
+/* Frees all memory and streams kept from destroyed contexts, so that other
+ * allocators of the process can have them.  Live contexts are not affected. */
+int fluid_hip_release_kept(void);
 
 /* Replace the per-scene parameters (same validation as create). */
 int fluid_hip_set_params(fluid_hip_ctx* ctx, const fluid_hip_params* params);

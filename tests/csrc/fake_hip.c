@@ -79,6 +79,22 @@ int hipFree(void* p) {
   violation("hipFree of memory that is not allocated");
   return kUnknown;
 }
+int hipMemGetAddressRange(void** base, size_t* bytes, void* p) {
+  for (int i = 0; i < g_nmem; ++i)
+    if (p >= g_mem[i].p && (char*)p < (char*)g_mem[i].p + g_mem[i].bytes) {
+      *base = g_mem[i].p;
+      *bytes = g_mem[i].bytes;
+      return kOk;
+    }
+  return kUnknown;
+}
+// Every allocation and stream is gone (the host memory stays, so that a use of it
+// shows as a violation and not as a crash).
+int hipDeviceReset(void) {
+  g_nmem = 0;
+  memset(g_streams, 0, sizeof(g_streams));
+  return kOk;
+}
 int hipHostMalloc(void** p, size_t bytes, unsigned flags) {
   (void)flags;
   *p = calloc(bytes ? bytes : 1, 1);

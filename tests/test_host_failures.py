@@ -54,6 +54,18 @@ class Fake:
     def __setattr__(self, name, v):
         self._var(name).value = v
 
+    def live(self):
+        return self.lib.fake_live()
+
+    def live_bytes(self):
+        return self.lib.fake_live_bytes()
+
+    def pending_streams(self):
+        return self.lib.fake_pending_streams()
+
+    def all_streams(self):
+        return self.lib.fake_all_streams()
+
     def fail_malloc(self, at=0, times=2):  # the library asks once more without its kept memory
         self.malloc_at, self.malloc_times = at, times
 
@@ -182,6 +194,94 @@ def recording(fake):
     s.backward()
     fake.check()
     s.close()
+
+
+@case
+def kept_memory_is_idle(fake):
+    from fluidsimulator_amd import hip
+
+    solver().close()
+    kept, streams = fake.live(), fake.all_streams()
+    assert kept > 1 and streams == 2 and fake.pending_streams() == 0
+    before = fake.mallocs
+    s = solver()  # takes what the first one left
+    assert fake.mallocs == before and fake.all_streams() == streams
+    # a context whose work may still run leaves nothing
+    s.step(1)
+    fake.sync_fails = 1
+    s.close()
+    fake.sync_fails = 0
+    assert fake.live() == 1 and fake.all_streams() == 0  # (the mark of the device)
+    # contexts that fail on the way: nothing that is in use is kept
+    for sync_fails in (0, 1):
+        for at in range(3):
+            fake.copy_at, fake.sync_fails = at, sync_fails
+            bad = raises(hip.EHIP, solver)
+            fake.copy_at, fake.sync_fails = -1, 0
+            assert bad  # the segments, the scene tables, the upload
+            assert fake.pending_streams() == 0
+            if sync_fails:
+                assert fake.live() == 1 and fake.all_streams() == 0
+    fake.check()
+
+
+@case
+def kept_memory_is_bounded(fake):
+    from fluidsimulator_amd import hip
+
+    solver(cell_capacity=1 << 12, neighbor_capacity=1 << 12).close()
+    small = fake.live()
+    # blocks larger than all that may be kept drive nothing out
+    solver(cell_capacity=100 << 20, neighbor_capacity=100 << 20).close()
+    assert fake.live() == small
+    # ... and smaller ones the oldest only
+    for k in range(20):
+        s = solver(cell_capacity=(8 + k) << 20, neighbor_capacity=1 << 12)
+        t = solver(cell_capacity=(4 + k) << 20, neighbor_capacity=1 << 14)
+        s.close(), t.close()
+        assert fake.live_bytes() <= (256 << 20) + 4099
+    assert fake.live_bytes() > 100 << 20
+    for k in range(40):  # ... many small ones too
+        a = [solver(cell_capacity=4000 + 500 * i, neighbor_capacity=4000 + 700 * i)
+             for i in range(30)]
+        for s in a:
+            s.close()
+    assert fake.live() <= 64 + 1 and fake.all_streams() <= 8
+    s = solver()
+    hip.release_kept()
+    s.step(1)
+    assert fake.live() == 3 and fake.all_streams() == 2  # the live context's
+    s.close()
+    # an allocation that finds no memory gets the kept blocks'
+    s = solver()
+    s.close()
+    fake.fail_malloc(times=1)
+    s = solver(cell_capacity=1 << 26, neighbor_capacity=1 << 26)
+    s.close()
+    hip.release_kept()
+    assert fake.live() == 0 and fake.all_streams() == 0
+    solver().close()
+    fake.check()
+
+
+@case
+def a_reset_device(fake):
+    from fluidsimulator_amd import hip
+
+    for _ in range(3):
+        s = solver()
+        s.step(1)
+        s.close()
+        fake.lib.hipDeviceReset()
+        s = solver()
+        s.step(1)
+        s.close()
+        assert fake.live() == 4 and fake.all_streams() == 2  # three blocks and the mark
+    fake.lib.hipDeviceReset()
+    solver().close()
+    hip.release_kept()
+    assert fake.live() == 0 and fake.all_streams() == 0
+    fake.check()
 
 
 @pytest.mark.parametrize("name", sorted(CASES))
