@@ -190,7 +190,7 @@ void compute_consts_of(Ctx& c, const fluid_hip_params* params, int n_scenes) {
                 ? 1
                 : 0;
   c.consts = k;
-  c.iterations = p.solver_iterations;
+  c.iterations = c.consts.iterations = p.solver_iterations;
   c.xsph = p.enable_xsph && p.visc_c != 0.0f;           // core.cpp:423
   c.vort = p.enable_vorticity && p.vort_epsilon != 0.0f;  // core.cpp:468
   c.restitution_any = false;
@@ -464,6 +464,7 @@ void carve_arrays(Ctx& c, Carver& a, bool omega) {
   a.take(c.planes, ns);
   a.take(c.flags, 1);
   a.take(c.steps_started, 1);
+  a.take(c.last, 1);
   // brick tiles: beyond this capacity bricks take the other passes
   c.tile_cap = static_cast<long long>(n / 32 + 256);
   a.take(c.in_tile, n);
@@ -619,6 +620,25 @@ int read_status(Ctx& c, DevStatus& st) {
                          hipMemcpyDeviceToHost, c.stream),
           "read cell need");
   HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+  return FLUID_HIP_OK;
+}
+
+// The constants of the last good substep and, in its slot order, the particles'
+// ids.  (posA has the ids in that order too, but not after a restored state.)
+int read_last(Ctx& c, fluidhip::StepConsts& k, std::vector<int>* ids) {
+  const size_t n = static_cast<size_t>(c.n);
+  std::vector<float4> pos(ids ? n : 0);
+  HIP_TRY(hipMemcpyAsync(&k, c.last, sizeof(k), hipMemcpyDeviceToHost, c.stream),
+          "read constants");
+  if (!pos.empty())
+    HIP_TRY(hipMemcpyAsync(pos.data(), c.posB, sizeof(float4) * n, hipMemcpyDeviceToHost,
+                           c.stream),
+            "read ids");
+  HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+  if (ids) {
+    ids->resize(n);
+    for (size_t s = 0; s < n; ++s) std::memcpy(&(*ids)[s], &pos[s].w, sizeof(int));
+  }
   return FLUID_HIP_OK;
 }
 
@@ -1301,14 +1321,9 @@ int fluid_hip_get_diag(fluid_hip_ctx* ctx, int32_t* cell, int32_t* sorted_ids,
   if (!c.stepped) return fail(FLUID_HIP_ESTATE, "no step taken since upload");
   if (cell && !c.record_diag) return fail(FLUID_HIP_ESTATE, "cells need record_diag=1");
   const size_t n = static_cast<size_t>(c.n);
-  std::vector<float4> pos(n);
-  HIP_TRY(hipMemcpy(pos.data(), c.posA, sizeof(float4) * n, hipMemcpyDeviceToHost), "read pos");
-  std::vector<int> ids(n);
-  for (size_t s = 0; s < n; ++s) {
-    int id;
-    std::memcpy(&id, &pos[s].w, sizeof(int));
-    ids[s] = id;
-  }
+  fluidhip::StepConsts last{};
+  std::vector<int> ids;
+  if ((rc = read_last(c, last, &ids))) return rc;
   if (sorted_ids) std::copy(ids.begin(), ids.end(), sorted_ids);
   if (cell) {
     std::vector<uint64_t> dc(n);
@@ -1323,10 +1338,10 @@ int fluid_hip_get_diag(fluid_hip_ctx* ctx, int32_t* cell, int32_t* sorted_ids,
     }
   }
   if (nbr_count) {
-    if (c.lists_partial) {
+    if (!last.full_lists) {
       // dense heads and the other slots of runs kept no count: a counting
       // walk of the last grid writes every slot's
-      HIP_TRY(fluidhip::enqueue_count_pairs(c), "count pairs");
+      HIP_TRY(fluidhip::enqueue_count_pairs(c, last), "count pairs");
       HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
     }
     std::vector<int> nc(n);
@@ -1336,12 +1351,12 @@ int fluid_hip_get_diag(fluid_hip_ctx* ctx, int32_t* cell, int32_t* sorted_ids,
   if (rho) {
     std::vector<float> r(n);
     HIP_TRY(hipMemcpy(r.data(), c.rho, sizeof(float) * n, hipMemcpyDeviceToHost), "read rho");
-    for (size_t s = 0; s < n; ++s) rho[ids[s]] = c.iterations > 0 ? r[s] : 0.0f;
+    for (size_t s = 0; s < n; ++s) rho[ids[s]] = last.iterations > 0 ? r[s] : 0.0f;
   }
   if (lambda) {
-    if (c.iterations > 0) {
+    if (last.iterations > 0) {
       std::vector<float4> P(n);
-      HIP_TRY(hipMemcpy(P.data(), fluidhip::iterate_buffer(c, c.iterations - 1), sizeof(float4) * n,
+      HIP_TRY(hipMemcpy(P.data(), fluidhip::iterate_buffer(c, last.iterations - 1), sizeof(float4) * n,
                         hipMemcpyDeviceToHost),
               "read lambda");
       for (size_t s = 0; s < n; ++s) lambda[ids[s]] = P[s].w;
@@ -1358,15 +1373,16 @@ int fluid_hip_get_neighbors(fluid_hip_ctx* ctx, int32_t* out, int64_t cap, int64
   Ctx& c = ctx->c;
   if (!c.stepped) return fail(FLUID_HIP_ESTATE, "no step taken since upload");
   const size_t n = static_cast<size_t>(c.n);
-  std::vector<float4> pos(n);
   std::vector<long long> off(n);
   std::vector<int> nw(n);
-  HIP_TRY(hipMemcpy(pos.data(), c.posA, sizeof(float4) * n, hipMemcpyDeviceToHost), "read pos");
+  fluidhip::StepConsts last{};
+  std::vector<int> ids;
+  if ((rc = read_last(c, last, &ids))) return rc;
   HIP_TRY(hipMemcpy(nw.data(), c.nwords, sizeof(int) * n, hipMemcpyDeviceToHost), "read lengths");
   // particles of LDS tiles keep LDS records of the tile's halo: decode them
   // with its layout; list heads keep slots in their row, and a step that
   // stores no words leaves lists too long for a row to this call
-  const bool tiled = c.consts.tiles && c.last_runs && c.in_tile != nullptr;
+  const bool tiled = last.tiles && last.runs;
   std::vector<int> in_tile, tseg, tsrc, tcnt, ncnt;
   std::vector<uint16_t> tlist;
   if (tiled) {
@@ -1392,7 +1408,7 @@ int fluid_hip_get_neighbors(fluid_hip_ctx* ctx, int32_t* out, int64_t cap, int64
     // the words buffer holds nothing else then
     if ((rc = ensure_tables(c))) return rc;
     for (int attempt = 0; attempt < 2; ++attempt) {
-      HIP_TRY(fluidhip::enqueue_long_lists(c), "long lists");
+      HIP_TRY(fluidhip::enqueue_long_lists(c, last), "long lists");
       unsigned long long need = 0;
       HIP_TRY(hipMemcpyAsync(&need, c.nbr_total, sizeof(need), hipMemcpyDeviceToHost, c.stream),
               "read total");
@@ -1453,13 +1469,8 @@ int fluid_hip_get_neighbors(fluid_hip_ctx* ctx, int32_t* out, int64_t cap, int64
   std::vector<int> list(used);
   if (used)
     HIP_TRY(hipMemcpy(list.data(), c.nbr, sizeof(int) * used, hipMemcpyDeviceToHost), "read list");
-  std::vector<int> ids(n), slot_of(n);
-  for (size_t s = 0; s < n; ++s) {
-    int id;
-    std::memcpy(&id, &pos[s].w, sizeof(int));
-    ids[s] = id;
-    slot_of[id] = static_cast<int>(s);
-  }
+  std::vector<int> slot_of(n);
+  for (size_t s = 0; s < n; ++s) slot_of[ids[s]] = static_cast<int>(s);
   int64_t k = 0;
   std::vector<int> tn;
   for (size_t id = 0; id < n; ++id) {
@@ -1528,9 +1539,11 @@ int fluid_hip_get_stats(fluid_hip_ctx* ctx, int64_t* out, int32_t n) {
   int64_t v[10] = {0, 0, 0, c.nbr_cap, c.cell_cap, c.grow_events, tape_bytes(c),
                    c.adj ? c.adj->recomputed : 0, 0, 0};
   if (c.stepped && c.n > 0) {
-    if (c.lists_partial) {
+    fluidhip::StepConsts last{};
+    if ((rc = read_last(c, last, nullptr))) return rc;
+    if (!last.full_lists) {
       // dense heads stored no list: count their pairs again
-      HIP_TRY(fluidhip::enqueue_count_pairs(c), "count pairs");
+      HIP_TRY(fluidhip::enqueue_count_pairs(c, last), "count pairs");
       unsigned long long pairs = 0;
       HIP_TRY(hipMemcpyAsync(&pairs, c.pair_total, sizeof(pairs), hipMemcpyDeviceToHost,
                              c.stream),
@@ -1549,7 +1562,7 @@ int fluid_hip_get_stats(fluid_hip_ctx* ctx, int64_t* out, int32_t n) {
     int cells = 0;
     HIP_TRY(hipMemcpy(&cells, c.total_cells, sizeof(int), hipMemcpyDeviceToHost), "read cells");
     v[2] = cells;
-    if (c.consts.tiles && c.last_runs && c.tile_count) {
+    if (last.tiles && last.runs) {
       int tiles = 0;
       HIP_TRY(hipMemcpy(&tiles, c.tile_count, sizeof(int), hipMemcpyDeviceToHost), "read tiles");
       tiles = static_cast<int>(std::min<int64_t>(tiles, c.tile_cap));

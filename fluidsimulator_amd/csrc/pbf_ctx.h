@@ -183,6 +183,12 @@ struct Ctx {
   int* seg = nullptr;
   ScenePlanes* planes = nullptr;
 
+  // The constants of the last good substep, written with its grid: what queries
+  // of its slots and lists go by, whatever parameters or launch knobs the
+  // context has now, whether it was recorded, and whether a graph replayed it.
+  // Its ids are in posB.
+  StepConsts* last = nullptr;
+
   // status
   unsigned* flags = nullptr;
   int* steps_started = nullptr;
@@ -190,12 +196,6 @@ struct Ctx {
   bool uploaded = false;
   bool stepped = false;
   long long grow_events = 0;  // capacity growths (each replays the failed substep)
-  // the last substep stored no words of any list (counts of dense heads need
-  // a counting walk), and its p^0 is in pred[0]
-  bool lists_partial = false;
-  // the last substep computed each run of identical slots once (it was not
-  // recorded and kept no diagnostics)
-  bool last_runs = false;
 
   // staging for transfers
   float* stage = nullptr;  // 6 * n
@@ -314,12 +314,12 @@ hipError_t enqueue_xsph(Ctx& c, const StepConsts& k, const GatherView& gv, bool 
                         unsigned* rm);
 hipError_t enqueue_vort_omega(Ctx& c, const StepConsts& k, const GatherView& gv);
 hipError_t enqueue_vort_apply(Ctx& c, const StepConsts& k, const GatherView& gv, bool rest);
-// After a substep that stored no words: counts every particle's neighbors
-// into c.ncount and their sum into c.pair_total.
-hipError_t enqueue_count_pairs(Ctx& c);
+// After a substep with constants k that stored no words: counts every particle's
+// neighbors into c.ncount and their sum into c.pair_total.
+hipError_t enqueue_count_pairs(Ctx& c, const StepConsts& k);
 // ... or stores the lists too long for a row (nwords kLongList) in c.nbr;
 // *c.nbr_total is what they need, and a list that does not fit is left out.
-hipError_t enqueue_long_lists(Ctx& c);
+hipError_t enqueue_long_lists(Ctx& c, const StepConsts& k);
 
 // The tile kernels (pbf_tiles.hip).
 hipError_t enqueue_tile_classify(Ctx& c, const StepConsts& k);

@@ -65,6 +65,7 @@ struct StepConsts {
   int runs;         // 1: a run of identical consecutive slots is computed once
   int full_lists;   // 1: every particle's list is stored (diagnostics), 2: as
                     //    plain slots where it fits a row (the adjoint's)
+  int iterations;   // of the constraint loop
   int tiles;        // 1: sparse 4x4x4-cell bricks run the LDS-tiled passes
   int exact_terms;  // 1: pair terms need no range tests (tile_spiky)
 };

@@ -1665,22 +1665,22 @@ hipError_t enqueue_neighbors(Ctx& c, const StepConsts& k, const GatherView& gv) 
   return hipGetLastError();
 }
 
-hipError_t enqueue_long_lists(Ctx& c) {
+hipError_t enqueue_long_lists(Ctx& c, const StepConsts& k) {
   if (c.n == 0) return hipSuccess;
   k_reset_total<<<1, 64, 0, c.stream>>>(c.nbr_total);
   k_long_lists<<<std::min(kDenseGrid, blocks_for(c.n, kWaves)), kBlock, 0, c.stream>>>(
-      c.consts, gather_view(c, c.pred[0]), 1, c.noff, c.nwords, c.ncount,
+      k, gather_view(c, c.pred[0]), 1, c.noff, c.nwords, c.ncount,
       c.nbr, c.nbr_cap, c.nbr_total, c.flags);
   return hipGetLastError();
 }
 
-hipError_t enqueue_count_pairs(Ctx& c) {
+hipError_t enqueue_count_pairs(Ctx& c, const StepConsts& k) {
   k_reset_total<<<1, 64, 0, c.stream>>>(c.pair_total);
   if (c.n == 0) return hipGetLastError();
   k_count_dense<<<std::min(kDenseGrid, blocks_for(c.n, kWaves)), kBlock, 0, c.stream>>>(
-      c.consts, gather_view(c, c.pred[0]), c.ncount, c.flags);
+      k, gather_view(c, c.pred[0]), c.ncount, c.flags);
   k_count_slots<<<std::min(1024, blocks_for(c.n, kBlock)), kBlock, 0, c.stream>>>(
-      c.n, c.run_no, c.rep_list, c.consts.tiles ? c.in_tile : nullptr, c.tile_cnt, c.ncount,
+      c.n, c.run_no, c.rep_list, k.tiles ? c.in_tile : nullptr, c.tile_cnt, c.ncount,
       c.pair_total, c.flags);
   return hipGetLastError();
 }

@@ -278,14 +278,15 @@ struct GridSetup {
   int* __restrict__ steps_started;
   int* __restrict__ tile_count;  // null without tiles
   int* __restrict__ info;
+  StepConsts* __restrict__ last;  // the constants of the last good substep
 };
 
 // One workgroup: per-scene table extents and key offsets; resets the per-step
 // counters.
 constexpr int kGridSetupThreads = 1024;
 constexpr int kLocalBoxes = 64;  // scenes whose boxes are folded in LDS
-__device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_bbox, int* bbox,
-                                           unsigned* flags) {
+__device__ __forceinline__ void grid_setup(const StepConsts& c, const GridSetup& gs,
+                                           const int* tile_bbox, int* bbox, unsigned* flags) {
   const int n_scenes = gs.n_scenes, tile_size = gs.tile_size, bshift = gs.bshift;
   const long long cell_cap = gs.cell_cap;
   const int* __restrict__ seg = gs.seg;
@@ -405,6 +406,7 @@ __device__ __forceinline__ void grid_setup(const GridSetup& gs, const int* tile_
   }
   if (threadIdx.x == 0 && !was_fatal) {
     if (fits) {
+      *gs.last = c;
       *gs.nbr_total = 0ull;
       gs.info[2] = 0;  // dense units
       if (gs.tile_count) {
@@ -429,10 +431,10 @@ __global__ __launch_bounds__(1024) void k_predict_bbox(
   predict_bbox<false>(c, pos, vel, sp, seg, cellc, bbox, tile_bbox, flags);
 }
 
-__global__ __launch_bounds__(kGridSetupThreads) void k_grid_setup(GridSetup gs,
+__global__ __launch_bounds__(kGridSetupThreads) void k_grid_setup(StepConsts c, GridSetup gs,
                                                                   const int* tile_bbox, int* bbox,
                                                                   unsigned* flags) {
-  grid_setup(gs, tile_bbox, bbox, flags);
+  grid_setup(c, gs, tile_bbox, bbox, flags);
 }
 
 // Both in one launch: the workgroup that finishes last (a device counter,
@@ -452,7 +454,7 @@ __global__ __launch_bounds__(1024) void k_predict_setup(
   __syncthreads();
   if (!last_sh) return;
   if (threadIdx.x == 0) *finished = 0;
-  grid_setup(gs, tile_bbox, bbox, flags);
+  grid_setup(c, gs, tile_bbox, bbox, flags);
 }
 
 // The cell key of slot p of the previous substep's order.
@@ -979,8 +981,6 @@ hipError_t enqueue_substep(Ctx& c, const SubstepRec* rec) {
   const TileArgs ta{c.slot_cell, c.tile_count, static_cast<int>(c.tile_cap), c.tile_rec,
                     c.tile_seg,  c.tile_src,   c.tile_list, c.tile_list_cap, c.tile_cnt};
   const GatherView gv = gather_view(c, PK(0));
-  c.lists_partial = !k.full_lists;
-  c.last_runs = k.runs != 0;
   const int bs = c.block;
   const int nb = blocks_for(c.n, bs);
   hipStream_t st = c.stream;
@@ -994,7 +994,8 @@ hipError_t enqueue_substep(Ctx& c, const SubstepRec* rec) {
 
   const GridSetup gs{c.n_scenes,    c.seg,        bs,           c.grid,
                      c.total_cells, c.cell_cap,   c.brick_shift, c.nbr_total,
-                     c.need_cells,  c.steps_started, tiles ? c.tile_count : nullptr, c.info};
+                     c.need_cells,  c.steps_started, tiles ? c.tile_count : nullptr, c.info,
+                     c.last};
   // A small batch's launches take about 4 us each, whatever they do: one less.
   // (In a large one the workgroups' fences cost more, and many scenes' boxes
   // are folded by 1,024 threads.)
@@ -1010,7 +1011,7 @@ hipError_t enqueue_substep(Ctx& c, const SubstepRec* rec) {
                                         c.tile_bbox, c.flags);
     }));
     FH_TRY(L("grid_setup", [&] {
-      k_grid_setup<<<1, kGridSetupThreads, 0, st>>>(gs, c.tile_bbox, c.bbox, c.flags);
+      k_grid_setup<<<1, kGridSetupThreads, 0, st>>>(k, gs, c.tile_bbox, c.bbox, c.flags);
     }));
   }
   // keys lie below the cell table's capacity: 8 bits per pass
