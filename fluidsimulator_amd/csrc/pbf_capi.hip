@@ -1623,7 +1623,11 @@ int fluid_hip_autotune(fluid_hip_ctx* ctx, int32_t trial_steps, int32_t knobs,
   struct Knobs {
     int block, remap, wave, bshift, tiles;
   };
-  const Knobs start{c.block, c.xcd_remap, c.wave_mode, c.brick_shift, c.tile_gather == 2 ? 2 : 1};
+  // the default tile mode by its name (1 on, 2 off) only where it is compared
+  const int tiles_set =
+      c.tile_gather ? c.tile_gather : c.n >= fluidhip::kTileAutoMinParticles ? 1 : 2;
+  const Knobs start{c.block, c.xcd_remap, c.wave_mode, c.brick_shift,
+                    (knobs & FLUID_HIP_TUNE_TILES) ? tiles_set : c.tile_gather};
   const size_t n = static_cast<size_t>(c.n);
   const size_t soa = 3 * n;
   invalidate_record(c);

@@ -244,7 +244,8 @@ int fluid_hip_get_stats(fluid_hip_ctx* ctx, int64_t* out, int32_t n);
  * `trial_steps` substeps from the current state between two events; its
  * final state must equal the starting configuration's bit for bit, or it is
  * rejected.  The fastest candidate (by at least 3%) is kept; the state and
- * time are restored.  `best` receives the chosen configuration, report[0..3]
+ * time are restored.  `best` receives the chosen configuration (tile_gather as
+ * the context had it unless FLUID_HIP_TUNE_TILES is given), report[0..3]
  * the starting and chosen ms per substep, the candidates timed and the
  * candidates rejected (either may be NULL).  A recorded rollout is
  * discarded. */

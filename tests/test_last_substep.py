@@ -107,3 +107,20 @@ def test_recorded_substeps_and_replays(block, tiles):
         s.step(1)
         # (the first cells of 32 particles or more, which keep no lists)
         check(s, want(p, pos, vel, 10), neighbors=False)
+
+
+@pytest.mark.parametrize("tiles", [0, 1, 2])
+@pytest.mark.parametrize("knobs", [hip.TUNE_BLOCK, hip.TUNE_BLOCK | hip.TUNE_TILES])
+def test_the_tuner_leaves_the_tile_mode_unless_asked(tiles, knobs):
+    sc = scenes.dam_break(seed=91, dims=(38, 34, 31), flags=True)  # 40,052 particles: none by default
+    with hip.HipSolver(sc.params, [sc.state.n], tile_gather=tiles) as s:
+        s.upload(sc.state.pos, sc.state.vel)
+        rep = s.autotune(trial_steps=1, knobs=knobs)
+        s.step(1)
+        st = s.stats()
+    assert rep["candidates_rejected"] == 0
+    assert (st["tiles"] > 0) == (rep["tile_gather"] == 1)
+    if knobs == hip.TUNE_BLOCK:
+        assert rep["tile_gather"] == tiles
+    else:
+        assert rep["tile_gather"] in (1, 2)
