@@ -33,9 +33,13 @@ constexpr unsigned kFlagFatal = kFlagRange | kFlagCells | kFlagNeighbors;
 constexpr int kRadixTile = 1024;
 
 // The heads of batches of up to this many particles are listed by one workgroup
-// instead of in two launches.  Measured, both ways, us per 8 substeps: 4,199
-// particles 916 / 935, 7,429 particles 1,170 / 1,153.
-constexpr int kSmallHeads = 8192;
+// instead of in two launches: its rounds over 1,024 slots each are in series.
+// Measured, one / two launches, us per 8 substeps of a block just released and
+// after 24 substeps, with a workgroup for 8,192: 1,728 particles 724 / 755 and
+// 714 / 743; 4,199: 852 / 864 and 919 / 932; 4,896: 895 / 898 and 940 / 942;
+// 5,760: 961 / 961 and 1,069 / 1,062; 6,800: 947 / 935 and 998 / 983; 8,000:
+// 1,142 / 1,117 and 1,167 / 1,141.
+constexpr int kSmallHeads = 5120;
 
 struct StepConsts {
   int n;            // particles, all scenes

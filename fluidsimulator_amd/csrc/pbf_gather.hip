@@ -297,13 +297,16 @@ __global__ __launch_bounds__(1024) void k_heads_small(
     long long* __restrict__ noff, int* __restrict__ nwords, int* __restrict__ ncount,
     const unsigned* __restrict__ flags) {
   constexpr int kT = 1024, kW = kT / kWave, kR = kSmallHeads / kT;
-  static_assert(kR * kT == kSmallHeads && kR * kW % kWave == 0, "whole rounds of the scan");
-  __shared__ int runs[kR * kW], lists[kR * kW];
+  static_assert(kR * kT == kSmallHeads, "whole rounds");
+  // (round, wavefront) counts, padded to whole rounds of their scan
+  constexpr int kCounts = kR * kW, kScan = (kCounts + kWave - 1) / kWave * kWave;
+  __shared__ int runs[kScan], lists[kScan];
   __shared__ int nd_sh, ndense;
   if (fatal(flags)) return;
   const int n = c.n, tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
   const unsigned long long below = (1ull << lane) - 1ull;
   if (tid == 0) nd_sh = ndense = 0;
+  if (tid < kScan - kCounts) runs[kCounts + tid] = lists[kCounts + tid] = 0;
   int cls[kR];
 #pragma unroll
   for (int r = 0; r < kR; ++r) {
@@ -328,7 +331,7 @@ __global__ __launch_bounds__(1024) void k_heads_small(
     int* a = w == 0 ? runs : lists;
     int carry = 0;
 #pragma unroll
-    for (int i = 0; i < kR * kW; i += kWave) {
+    for (int i = 0; i < kScan; i += kWave) {
       const int v = a[i + lane];
       const int inc = incl_scan<kWave>(v);
       a[i + lane] = carry + inc - v;
