@@ -281,10 +281,12 @@ struct GridSetup {
   StepConsts* __restrict__ last;  // the constants of the last good substep
 };
 
-// One workgroup: per-scene table extents and key offsets; resets the per-step
-// counters.
 constexpr int kGridSetupThreads = 1024;
 constexpr int kLocalBoxes = 64;  // scenes whose boxes are folded in LDS
+
+// One workgroup: per-scene table extents and key offsets; resets the per-step
+// counters (kFew: no more scenes than threads).
+template <bool kFew>
 __device__ __forceinline__ void grid_setup(const StepConsts& c, const GridSetup& gs,
                                            const int* tile_bbox, int* bbox, unsigned* flags) {
   const int n_scenes = gs.n_scenes, tile_size = gs.tile_size, bshift = gs.bshift;
@@ -330,17 +332,18 @@ __device__ __forceinline__ void grid_setup(const StepConsts& c, const GridSetup&
     }
   }
   __syncthreads();
-  // Cells of scene s's table, and its extents.
+  // Scene s's extents and the cells of its table.
   auto extents = [&](int s, GridDesc& g) -> long long {
+    if (s >= n_scenes) return 0;
     const int* from = (local ? box : bbox) + 6 * s;
     const long long lx = from[0], ly = from[1], lz = from[2];
     const long long hx = from[3], hy = from[4], hz = from[5];
-    g = GridDesc{};
     g.bshift = bshift;
     if (lx > hx || ly > hy || lz > hz) return 0;
-    const long long sx = hx - lx + 3, sy = hy - ly + 3, sz = hz - lz + 3;
-    const long long e = 1ll << bshift;
-    const long long bx = (sx + e - 1) / e, by = (sy + e - 1) / e, bz = (sz + e - 1) / e;
+    // (cells of a margin of one on each side, in whole bricks)
+    const int up = (1 << bshift) + 2;
+    const long long bx = (hx - lx + up) >> bshift, by = (hy - ly + up) >> bshift,
+                    bz = (hz - lz + up) >> bshift;
     g.ox = static_cast<int>(lx - 1);
     g.oy = static_cast<int>(ly - 1);
     g.oz = static_cast<int>(lz - 1);
@@ -372,29 +375,28 @@ __device__ __forceinline__ void grid_setup(const StepConsts& c, const GridSetup&
     __syncthreads();  // sh is reused
     return inc - v + before;
   };
-  // The scenes' cells in all come first: a substep that fails leaves the grid of
-  // the last good one, which belongs to the other arrays of that substep.
-  GridDesc g{};
+  // A substep that fails leaves the grid of the last good one, which belongs to
+  // the other arrays of that substep: the scenes' cells in all are known before
+  // any scene's grid is written.
+  const bool few = kFew || n_scenes <= static_cast<int>(blockDim.x);
   long long total = 0, carry = 0;
-  long long nc = 0, excl = 0;
-  for (int b0 = 0; b0 < n_scenes; b0 += blockDim.x) {
-    const int s = b0 + threadIdx.x;
-    nc = s < n_scenes ? extents(s, g) : 0;
-    long long all;
-    excl = prefix(nc, all);
-    total += all;
-  }
-  const bool fits = total <= cell_cap;
-  for (int b0 = 0; b0 < n_scenes; b0 += blockDim.x) {
-    const int s = b0 + threadIdx.x;
-    long long all = total;
-    if (n_scenes > static_cast<int>(blockDim.x)) {  // otherwise as computed above
-      nc = s < n_scenes ? extents(s, g) : 0;
-      excl = prefix(nc, all);
+  if (!few)
+    for (int b0 = 0; b0 < n_scenes; b0 += blockDim.x) {
+      GridDesc g{};
+      long long all;
+      (void)prefix(extents(b0 + threadIdx.x, g), all);
+      total += all;
     }
+  for (int b0 = 0; b0 < (kFew ? 1 : n_scenes); b0 += blockDim.x) {
+    const int s = b0 + threadIdx.x;
+    GridDesc g{};
+    const long long nc = extents(s, g);
+    long long all;
+    const long long excl = prefix(nc, all) + carry;
+    if (few) total = all;
     if (s < n_scenes) {
-      if (fits && !was_fatal) {
-        g.cell_off = static_cast<int>(excl + carry);
+      if (total <= cell_cap && !was_fatal) {
+        g.cell_off = static_cast<int>(excl);
         g.ncells = static_cast<int>(nc);
         grid[s] = g;
       }
@@ -405,8 +407,14 @@ __device__ __forceinline__ void grid_setup(const StepConsts& c, const GridSetup&
     carry += all;
   }
   if (threadIdx.x == 0 && !was_fatal) {
-    if (fits) {
-      *gs.last = c;
+    if (total <= cell_cap) {
+      // word by word: as a struct it goes through scratch memory, which costs
+      // every wavefront of the launch
+      static_assert(sizeof(StepConsts) % sizeof(int) == 0, "whole words");
+      const int* from = reinterpret_cast<const int*>(&c);
+      int* to = reinterpret_cast<int*>(gs.last);
+#pragma unroll
+      for (size_t i = 0; i < sizeof(StepConsts) / sizeof(int); ++i) to[i] = from[i];
       *gs.nbr_total = 0ull;
       gs.info[2] = 0;  // dense units
       if (gs.tile_count) {
@@ -434,7 +442,7 @@ __global__ __launch_bounds__(1024) void k_predict_bbox(
 __global__ __launch_bounds__(kGridSetupThreads) void k_grid_setup(StepConsts c, GridSetup gs,
                                                                   const int* tile_bbox, int* bbox,
                                                                   unsigned* flags) {
-  grid_setup(c, gs, tile_bbox, bbox, flags);
+  grid_setup<false>(c, gs, tile_bbox, bbox, flags);
 }
 
 // Both in one launch: the workgroup that finishes last (a device counter,
@@ -454,7 +462,7 @@ __global__ __launch_bounds__(1024) void k_predict_setup(
   __syncthreads();
   if (!last_sh) return;
   if (threadIdx.x == 0) *finished = 0;
-  grid_setup(c, gs, tile_bbox, bbox, flags);
+  grid_setup<true>(c, gs, tile_bbox, bbox, flags);
 }
 
 // The cell key of slot p of the previous substep's order.

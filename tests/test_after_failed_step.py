@@ -114,3 +114,45 @@ def test_scenes_over_the_whole_coordinate_range_do_not_fit(edge, count):
             s.step(1)
         assert e.value.code == hip.ECAPACITY
         assert same_bits(s.download().pos, pos)
+
+
+@pytest.mark.parametrize("count", [17, 65, 1024, 1025, 2100])
+def test_grids_of_many_scenes(count):
+    """Scenes beyond the threads of the grid setup, some of them empty: bitwise,
+    also after a substep whose table did not fit and after one that had a
+    particle out of range."""
+    p = scenes.base_params((4.0, 4.0, 4.0), True)
+    p.planes = []
+    rng = np.random.default_rng(count)
+    counts = [0 if k % 7 == 3 else int(rng.integers(1, 9)) for k in range(count)]
+    n = sum(counts)
+    pos = (0.2 + 0.3 * rng.random((3, n))).astype(np.float32)
+    vel = rng.standard_normal((3, n)).astype(np.float32)
+    want, at = [], 0
+    for c in counts:
+        if c:
+            o = oracle.step(p, pos[:, at:at + c], vel[:, at:at + c], nsteps=2)
+            want.append(np.concatenate([o["pos"], o["vel"]]))
+        at += c
+    want = np.concatenate(want, 1)
+    with hip.HipSolver([p] * count, counts, cell_capacity=1000) as s:
+        s.upload(pos, vel)
+        s.step(1)
+        _, grid = s.grid()
+        assert (grid[:, 7] > 0).sum() == sum(c > 0 for c in counts)
+        assert np.array_equal(grid[:, 6], np.concatenate([[0], np.cumsum(grid[:-1, 7])]))
+        s.step(1)
+        r = s.download()
+        assert same_bits(np.concatenate([r.pos, r.vel]), want)
+        _, grid = s.grid()
+        q = scenes.base_params((4.0, 4.0, 4.0), True)
+        q.planes, q.external_forces = [], (0.0, 0.0, 3e38)
+        s.set_params(q)
+        with pytest.raises(hip.HipError):
+            s.step(1)
+        assert np.array_equal(s.grid()[1], grid)
+        s.set_params(p)
+        s.upload(pos, vel)
+        s.step(2)
+        r = s.download()
+        assert same_bits(np.concatenate([r.pos, r.vel]), want)
