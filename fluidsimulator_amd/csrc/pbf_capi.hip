@@ -178,7 +178,6 @@ void compute_consts_of(Ctx& c, const fluid_hip_params* params, int n_scenes) {
   k.visc_c = p.visc_c;
   k.vort_eps = p.vort_epsilon;
   k.vort_norm_eps = p.vort_norm_eps;
-  k.record_diag = c.record_diag ? 1 : 0;
   k.xcd_remap = c.xcd_remap;
   k.runs = (c.wave_mode == 2 && !c.record_diag) ? 1 : 0;
   k.full_lists = (c.record_diag || c.wave_mode == 1) ? 1 : 0;
@@ -923,7 +922,6 @@ void close_streams(Ctx& c) {
 // when they do not fit.
 bool noalloc_layout(Ctx& c, unsigned char* base, size_t bytes) {
   Carver a{base, bytes};
-  c.lane_cap = 3ll * c.n + 64;
   carve_arrays(c, a, c.vort);
   if (!a.ok) return false;
   a.off = (a.off + 255) & ~static_cast<size_t>(255);
@@ -1041,9 +1039,7 @@ int fluid_hip_create(fluid_hip_ctx** out, int32_t n_scenes, const int64_t* scene
   if (e != hipSuccess) return bail(hip_fail(e, "hipStreamCreate"));
 
   const size_t n = static_cast<size_t>(c.n);
-  c.lane_cap = 3ll * n + 64;
-  if (cfg.lane_capacity > 0)
-    c.lane_cap = std::min<long long>(c.lane_cap, std::max<long long>(cfg.lane_capacity, n));
+  c.lane_capacity = cfg.lane_capacity;
   {
     // one block for all fixed arrays (omega too: set_params may turn
     // vorticity on)
@@ -1745,7 +1741,9 @@ int fluid_hip_autotune(fluid_hip_ctx* ctx, int32_t trial_steps, int32_t knobs,
       best->tile_gather = cur.tiles;
       best->cell_capacity = c.cell_cap;
       best->neighbor_capacity = c.nbr_cap;
-      best->lane_capacity = c.lane_cap;
+      const long long lanes = 3ll * c.n + 64;
+      best->lane_capacity =
+          c.lane_capacity > 0 ? std::min(lanes, std::max<long long>(c.lane_capacity, c.n)) : lanes;
       best->device = c.device;
       best->record_diag = c.record_diag ? 1 : 0;
     }

@@ -67,7 +67,6 @@ struct GatherView {
   const int* slot_key;
   const GridDesc* grid;
   const int* start;
-  const int* seg;
   const float4* p0;        // predicted positions p^0 (xyz) of the lists
   int dense_blocks;        // workgroups of a pass that take the dense units
 };
@@ -155,7 +154,7 @@ struct Ctx {
   int4* units = nullptr;       // per list head: {slot, neighbors or -1, slots of its run, scene}
   int2* dense = nullptr;       // groups of heads without a row: {first slot, scene | kSingle}
   int* info = nullptr;         // 5: runs, list heads, dense units, heads per unit, workgroups done
-  long long lane_cap = 0;      // reported by the tuner; no layout depends on it
+  long long lane_capacity = 0;  // as configured: ignored, reported by the tuner
 
   // brick tiles (sparse bricks whose passes run through LDS)
   int* in_tile = nullptr;      // per slot: 1 + its tile's index this substep, 0 outside tiles

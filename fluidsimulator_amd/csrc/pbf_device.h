@@ -64,7 +64,6 @@ struct StepConsts {
   float visc_c;
   float vort_eps;
   float vort_norm_eps;
-  int record_diag;
   int xcd_remap;
   int runs;         // 1: a run of identical consecutive slots is computed once
   int full_lists;   // 1: every particle's list is stored (diagnostics), 2: as

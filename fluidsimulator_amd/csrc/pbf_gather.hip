@@ -1627,7 +1627,7 @@ int list_blocks(const Ctx& c) {
 GatherView gather_view(const Ctx& c, const float4* p0) {
   return GatherView{c.info,   c.units, c.dense, c.run_no, c.rep_list,
                     reinterpret_cast<const int4*>(c.tile_list), row_capacity(c),
-                    c.slot_cell, c.slot_key, c.grid, c.start, c.seg, p0, dense_blocks(c)};
+                    c.slot_cell, c.slot_key, c.grid, c.start, p0, dense_blocks(c)};
 }
 
 hipError_t enqueue_heads(Ctx& c, const StepConsts& k) {

@@ -97,9 +97,9 @@ typedef struct fluid_hip_config {
                                  once, 3 every particle computed (same results) */
   int32_t brick_edge;         /* cells per brick edge of the cell table's Z-order:
                                  0 default (4), 1, 2, 4 or 8 */
-  int64_t lane_capacity;      /* 0 default (3n + 64), otherwise clamped to
-                                 [n, 3n + 64]; reported back, no layout
-                                 depends on it any more */
+  int64_t lane_capacity;      /* deprecated and ignored; the tuner reports it back
+                                 (3n + 64 for 0, otherwise clamped to
+                                 [n, 3n + 64]) */
   int32_t tile_gather;        /* passes of sparse 4x4x4-cell bricks through LDS tiles:
                                  0 default (on from 655,360 particles), 1 on, 2 off; used
                                  with brick edge 4 and gather mode 2 (results are the
