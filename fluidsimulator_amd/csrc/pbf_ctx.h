@@ -31,12 +31,18 @@ static_assert(kTileList >= kTileMaxCand - 1, "large-batch tiles must never overf
 // side stream (at 65,536 particles overlapping the two kernels of a pass
 // saves about what the fork and join cost)
 constexpr int kForkMinParticles = 1 << 18;
-// Default tile mode: tiles from this size on.  Below it the passes over the
-// heads are faster, above the tiles are while a scene is still spread out.
-// Measured, us per substep with tiles / without, all flags, released and after
-// 16 substeps: 32,768 particles 339 / 199 and 1,050 / 352; 131,072 460 / 384 and
-// 1,488 / 696; 262,144 774 / 599 and 1,906 / 1,192; 524,288 994 / 1,014 and
-// 2,330 / 1,922; 1,048,576 1,427 / 1,891 and 6,253 / 7,069.
+// Default tile mode: tiles from this size on.  A scene just released gains from
+// them from about 524,288 particles up, one that has piled up or sprayed loses
+// a little up to about 1,048,576; the line lies where the gain is a fifth and
+// the loss a few percent.  Measured, us per substep with tiles / without, all
+// flags, released, after 16 and after 32 substeps: 32,768 particles 314 / 196,
+// 884 / 381, 909 / 467; 131,072 415 / 374, 1,359 / 708, 1,160 / 652; 262,144
+// 708 / 562, 1,414 / 1,125, 1,158 / 951; 524,288 891 / 933, 1,833 / 1,798,
+// 2,299 / 2,174; 655,360 975 / 1,197, 2,196 / 2,181, 2,939 / 2,805; 802,816
+// 1,087 / 1,432, 2,924 / 2,859, 3,212 / 2,996; 1,048,576 1,265 / 1,745,
+// 4,065 / 4,464, 9,000 / 9,083.  256 scenes of 2,059,640 particles in all,
+// released, after 4 and after 24 substeps: 2,342 / 3,315, 3,248 / 3,080,
+// 3,139 / 2,925.
 constexpr int kTileAutoMinParticles = 5 << 17;
 constexpr int kTileGrid = 2048;     // workgroups of the persistent tile kernels
 

@@ -923,11 +923,9 @@ __global__ __launch_bounds__(kPass, kWavesPerSimd) void k_tile_vort_apply(
 // ------------------------------------------------------------ launching
 
 hipError_t enqueue_tile_classify(Ctx& c, const StepConsts& k) {
-  // small batches tile every brick they can (coincident particles
-  // included): the passes over heads then have no heads, whose latency
-  // costs each pass about 20 us for any number of them, and a few small
-  // tiles cost little; large ones leave bricks of sparse spray and runs of
-  // coincident particles to the passes over heads
+  // small batches, tiled only on request, tile every brick they can
+  // (coincident particles included); large ones leave bricks of sparse spray
+  // and runs of coincident particles to the passes over heads
   const bool large = c.n >= kForkMinParticles;
   const int min_particles = large ? kTileMinParticles : 1;
   k_tile_bricks<<<1024, kThreads, 0, c.stream>>>(c.start, c.total_cells, c.in_tile, c.tile_count,
