@@ -1153,14 +1153,12 @@ int fluid_hip_set_stream(fluid_hip_ctx* ctx, void* stream) {
   if (rc) return rc;
   Ctx& c = ctx->c;
   HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+  // the new one first: a call that fails leaves the old one in place
+  hipStream_t next = static_cast<hipStream_t>(stream);
+  if (!stream) HIP_TRY(hipStreamCreateWithFlags(&next, hipStreamNonBlocking), "hipStreamCreate");
   if (c.own_stream) hipStreamDestroy(c.stream);
-  if (stream) {
-    c.stream = static_cast<hipStream_t>(stream);
-    c.own_stream = false;
-  } else {
-    HIP_TRY(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking), "hipStreamCreate");
-    c.own_stream = true;
-  }
+  c.stream = next;
+  c.own_stream = !stream;
   drop_graph(c);
   return FLUID_HIP_OK;
 }

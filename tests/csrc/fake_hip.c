@@ -17,6 +17,7 @@ enum { kOk = 0, kOutOfMemory = 2, kUnknown = 999 };
 // ---- what the test sets and reads
 int fake_malloc_at = -1, fake_malloc_times = 0;  // the next mallocs but `at` fail, `times` of them
 int fake_copy_at = -1;                           // the asynchronous copy that fails
+int fake_stream_fails = 0;                       // streams cannot be created
 int fake_sync_fails = 0;                         // stream synchronizations fail
 unsigned fake_flags = 0;                         // status flags after the next reset
 int fake_flags_times = 0;
@@ -144,6 +145,8 @@ int hipGetLastError(void) { return kOk; }
 const char* hipGetErrorString(int e) { return e == kOutOfMemory ? "out of memory" : "error"; }
 int hipStreamCreateWithFlags(stream_t** s, unsigned flags) {
   (void)flags;
+  *s = NULL;
+  if (fake_stream_fails) return kUnknown;
   *s = calloc(1, sizeof(stream_t));
   ++fake_streams;
   for (int i = 0; i < 256; ++i)
@@ -163,8 +166,17 @@ int hipStreamDestroy(stream_t* s) {
   violation("hipStreamDestroy of no stream");
   return kUnknown;
 }
+static int known(stream_t* s) {
+  for (int i = 0; i < 256; ++i)
+    if (g_streams[i] == s) return 1;
+  return s == NULL;
+}
 int hipStreamSynchronize(stream_t* s) {
   ++fake_syncs;
+  if (!known(s)) {
+    violation("hipStreamSynchronize of no stream");
+    return kUnknown;
+  }
   if (fake_sync_fails) return kUnknown;
   if (s) s->pending = 0;
   return kOk;

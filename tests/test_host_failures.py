@@ -284,6 +284,30 @@ def a_reset_device(fake):
     fake.check()
 
 
+@case
+def a_stream_that_cannot_be_made(fake):
+    from fluidsimulator_amd import hip
+
+    fake.stream_fails = 1
+    assert raises(hip.EHIP, solver)
+    fake.stream_fails = 0
+    s = solver()
+    mine = C.c_void_p()
+    assert fake.lib.hipStreamCreateWithFlags(C.byref(mine), 0) == 0
+    for first in (None, mine):
+        assert s.lib.fluid_hip_set_stream(s.h, first) == 0
+        fake.stream_fails = 1
+        assert s.lib.fluid_hip_set_stream(s.h, None) == hip.EHIP
+        fake.stream_fails = 0
+        s.step(1)
+        s.download()
+    assert s.lib.fluid_hip_set_stream(s.h, None) == 0
+    s.step(1)
+    s.close()
+    assert fake.lib.hipStreamDestroy(mine) == 0
+    fake.check()
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_host_path(runtime, name):
     env = dict(os.environ, LD_LIBRARY_PATH=runtime, PYTHONPATH=ROOT)
