@@ -145,8 +145,7 @@ int hipGetLastError(void) { return kOk; }
 const char* hipGetErrorString(int e) { return e == kOutOfMemory ? "out of memory" : "error"; }
 int hipStreamCreateWithFlags(stream_t** s, unsigned flags) {
   (void)flags;
-  *s = NULL;
-  if (fake_stream_fails) return kUnknown;
+  if (fake_stream_fails) return kUnknown;  // (*s is not promised to be written)
   *s = calloc(1, sizeof(stream_t));
   ++fake_streams;
   for (int i = 0; i < 256; ++i)
