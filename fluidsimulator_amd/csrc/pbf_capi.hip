@@ -179,12 +179,12 @@ void compute_consts_of(Ctx& c, const fluid_hip_params* params, int n_scenes) {
   k.vort_eps = p.vort_epsilon;
   k.vort_norm_eps = p.vort_norm_eps;
   k.xcd_remap = c.xcd_remap;
-  k.runs = (c.wave_mode == 2 && !c.record_diag) ? 1 : 0;
+  k.runs = c.wave_mode == 2 ? 1 : 0;
   k.full_lists = (c.record_diag || c.wave_mode == 1) ? 1 : 0;
   // tile mode 0 (default) tiles from kTileAutoMinParticles particles on
   const bool tile_mode = c.tile_gather == 1 || (c.tile_gather == 0 && c.n >= fluidhip::kTileAutoMinParticles);
   k.exact_terms = tile_terms_exact(h, h2, k.min_r2) ? 1 : 0;
-  k.tiles = (k.runs && c.brick_shift == 2 && tile_mode && p.solver_iterations > 0 &&
+  k.tiles = (k.runs && !c.record_diag && c.brick_shift == 2 && tile_mode && p.solver_iterations > 0 &&
              k.exact_terms)
                 ? 1
                 : 0;
@@ -1376,7 +1376,7 @@ int fluid_hip_get_neighbors(fluid_hip_ctx* ctx, int32_t* out, int64_t cap, int64
   // particles of LDS tiles keep LDS records of the tile's halo: decode them
   // with its layout; list heads keep slots in their row, and a step that
   // stores no words leaves lists too long for a row to this call
-  const bool tiled = last.tiles && last.runs;
+  const bool tiled = last.tiles && !last.full_lists;
   std::vector<int> in_tile, tseg, tsrc, tcnt, ncnt;
   std::vector<uint16_t> tlist;
   if (tiled) {
@@ -1556,7 +1556,7 @@ int fluid_hip_get_stats(fluid_hip_ctx* ctx, int64_t* out, int32_t n) {
     int cells = 0;
     HIP_TRY(hipMemcpy(&cells, c.total_cells, sizeof(int), hipMemcpyDeviceToHost), "read cells");
     v[2] = cells;
-    if (last.tiles && last.runs) {
+    if (last.tiles && !last.full_lists) {
       int tiles = 0;
       HIP_TRY(hipMemcpy(&tiles, c.tile_count, sizeof(int), hipMemcpyDeviceToHost), "read tiles");
       tiles = static_cast<int>(std::min<int64_t>(tiles, c.tile_cap));

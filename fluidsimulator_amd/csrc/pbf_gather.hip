@@ -14,8 +14,9 @@
 //                position and one velocity (bit for bit, after gravity):
 //                their lists hold the same values in the same order, so the
 //                first slot (the head) stands for all and writes every
-//                slot's outputs.  Without runs (recorded substeps,
-//                diagnostics) every slot is a head.
+//                slot's outputs.  Without runs (gather modes 1 and 3) every
+//                slot is a head.  Recorded substeps and diagnostics store
+//                the list of every slot of a run.
 //   list heads   heads of cells of fewer than kDenseCell particles, with at
 //                most row_cap neighbors: their neighbors' slots are stored
 //                in a row; kListLanes lanes work on one head.
@@ -711,17 +712,18 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
   }
 }
 
-// The rows of a recorded substep's list heads as plain words: a workgroup
-// takes consecutive units, whose lists it allocates with one atomic (atomics on
-// one address take about 10 ns each: one for every 8 heads made the neighbor
-// kernel take 107 us at 65,536 particles; without them it takes 27, and this
-// one 21).
+// The rows of a recorded substep's list heads as plain words, one list for every
+// slot of the head's run (the run's slots but the list's own are one stretch of
+// it): a workgroup takes consecutive units, whose lists it
+// allocates with one atomic (atomics on one address take about 10 ns each: one
+// for every 8 heads made the neighbor kernel take 107 us at 65,536 particles;
+// without them it takes 27, and this one 21).
 __global__ __launch_bounds__(kBlock) void k_store_rows(
     StepConsts c, GatherView gv, long long* __restrict__ noff, int* __restrict__ nwords,
-    int* __restrict__ nbr, long long nbr_cap, unsigned long long* __restrict__ nbr_total,
-    unsigned* __restrict__ flags) {
+    int* __restrict__ ncount, int* __restrict__ nbr, long long nbr_cap,
+    unsigned long long* __restrict__ nbr_total, unsigned* __restrict__ flags) {
   constexpr int kLanes = 8, kUnits = kBlock / kLanes;
-  __shared__ int wsum[kWaves];
+  __shared__ long long wsum[kWaves];
   __shared__ long long base_sh;
   __shared__ int abort_sh;
   if (threadIdx.x == 0) abort_sh = fatal(flags) ? 1 : 0;
@@ -731,14 +733,16 @@ __global__ __launch_bounds__(kBlock) void k_store_rows(
   const int per = (L + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
   const int u0 = blockIdx.x * per, u1 = min(L, u0 + per);
   if (u0 >= u1) return;  // uniform
-  int sum = 0;
-  for (int u = u0 + static_cast<int>(threadIdx.x); u < u1; u += kBlock)
-    sum += max(gv.units[u].y, 0);
+  long long sum = 0;
+  for (int u = u0 + static_cast<int>(threadIdx.x); u < u1; u += kBlock) {
+    const int4 unit = gv.units[u];
+    sum += static_cast<long long>(max(unit.y, 0)) * unit.z;
+  }
   for (int o = kWave / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
   if (lane_id() == 0) wsum[threadIdx.x / kWave] = sum;
   __syncthreads();
   if (threadIdx.x == 0) {
-    int total = 0;
+    long long total = 0;
     for (int w = 0; w < kWaves; ++w) total += wsum[w];
     const long long at =
         static_cast<long long>(atomicAdd(nbr_total, static_cast<unsigned long long>(total)));
@@ -753,28 +757,42 @@ __global__ __launch_bounds__(kBlock) void k_store_rows(
   for (int b = u0; b < u1; b += kUnits) {
     const int u = b + g;
     const int4 unit = u < u1 ? gv.units[u] : make_int4(0, -1, 0, 0);
-    const int cnt = max(unit.y, 0);
-    // the lists before this one: within the wavefront (its groups' first
+    const int s = unit.x, cnt = max(unit.y, 0), len = unit.z;
+    const long long mine = static_cast<long long>(cnt) * len;
+    // the lists before this unit's: within the wavefront (its groups' first
     // lanes), then the wavefronts before
-    int inc = cnt;
+    long long inc = mine;
     for (int o = kLanes; o < kWave; o <<= 1) {
-      const int v = __shfl_up(inc, o);
+      const long long v = __shfl_up(inc, o);
       if (lane_id() >= o) inc += v;
     }
     __syncthreads();  // wsum is reused
     if (lane_id() == kWave - 1) wsum[threadIdx.x / kWave] = inc;
     __syncthreads();
-    long long off = at + inc - cnt;
+    long long off = at + inc - mine;
     for (int w = 0; w < kWaves; ++w) {
       off += w < static_cast<int>(threadIdx.x) / kWave ? wsum[w] : 0;
       at += wsum[w];
     }
-    for (int k = q; k < cnt; k += kLanes)
-      nbr[off + k] = rows[(static_cast<size_t>(k >> 2) * c.n + unit.x) * 4 + (k & 3)];
-    if (q == 0 && unit.y >= 0) {
-      noff[unit.x] = off;
-      nwords[unit.x] = cnt;
+    auto row = [&](int k) { return rows[(static_cast<size_t>(k >> 2) * c.n + s) * 4 + (k & 3)]; };
+    // the run's other slots: entries [own, own + len - 1) of the row
+    int own = cnt;
+    if (len > 1)
+      for (int k = q; k < cnt; k += kLanes)
+        if (row(k) == s + 1) own = k;
+    for (int o = kLanes / 2; o > 0; o >>= 1) own = min(own, __shfl_xor(own, o));
+    for (int k = q; k < cnt; k += kLanes) {
+      const int v = row(k), i = k - own;
+      const bool in_run = i >= 0 && i < len - 1;
+      for (int j = 0; j < len; ++j)
+        nbr[off + static_cast<long long>(j) * cnt + k] = in_run ? s + i + (i >= j ? 1 : 0) : v;
     }
+    if (unit.y >= 0)
+      for (int j = q; j < len; j += kLanes) {
+        noff[s + j] = off + static_cast<long long>(j) * cnt;
+        nwords[s + j] = cnt;
+        ncount[s + j] = cnt;
+      }
   }
 }
 
@@ -800,65 +818,6 @@ __device__ __forceinline__ DenseUnit dense_unit(const GatherView& gv, int u, int
     d.heads = min(left, unit - (d.r0 & (unit - 1)));
   }
   return d;
-}
-
-// The lists of the dense units' heads as run-length words, one wavefront per
-// unit, each cell's slots 64 at a time: counted, allocated (one atomic per
-// list) and filled.  With `only_long` the heads of dense cells are left out,
-// and no flag is raised when the lists do not fit (*nbr_total says what they
-// need).
-__global__ __launch_bounds__(kBlock) void k_long_lists(
-    StepConsts c, GatherView gv, int only_long, long long* __restrict__ noff,
-    int* __restrict__ nwords, int* __restrict__ ncount, int* __restrict__ nbr, long long nbr_cap,
-    unsigned long long* __restrict__ nbr_total, unsigned* __restrict__ flags) {
-  if (fatal(flags)) return;
-  const int D = gv.info[2];
-  const int lane = lane_id();
-  const int nw = static_cast<int>(gridDim.x) * kWaves;
-  for (int u = blockIdx.x * kWaves + threadIdx.x / kWave; u < D; u += nw) {
-    const DenseUnit d = dense_unit(gv, u, gv.info[3]);
-    if (only_long && !d.single) continue;
-    int a, b;
-    if (!cell_range(gv, d.s, d.sc, lane, a, b)) continue;
-    for (int h = 0; h < d.heads; ++h) {
-      const int s = __builtin_amdgcn_readfirstlane(gv.rep[d.r0 + h]);
-      const float3 me = ld3(gv.p0, s);
-      auto walk = [&](auto fill, RunWriter& w) {
-        for (int ci = 0; ci < 27; ++ci) {
-          const int ca = __builtin_amdgcn_readlane(a, ci), cb = __builtin_amdgcn_readlane(b, ci);
-          for (int t0 = ca; t0 < cb; t0 += kWave) {
-            const int t = min(t0 + lane, cb - 1);
-            unsigned long long m =
-                __ballot(t0 + lane < cb && t != s && near0(me, ld3(gv.p0, t), c));
-            while (m != 0ull) {
-              const int j = __builtin_ctzll(m);
-              const unsigned long long rest = ~(m >> j);
-              const int len = rest != 0ull ? __builtin_ctzll(rest) : kWave - j;
-              w.template add_range<decltype(fill)::value>(t0 + j, t0 + j + len);
-              m = (j + len >= kWave) ? 0ull : (m & (~0ull << (j + len)));
-            }
-          }
-        }
-        w.template flush<decltype(fill)::value>();
-      };
-      RunWriter w{nullptr, false};
-      walk(std::false_type{}, w);
-      unsigned long long at = 0;
-      if (lane == 0) at = atomicAdd(nbr_total, static_cast<unsigned long long>(w.words));
-      const long long off = static_cast<long long>(__shfl(at, 0));
-      if (off + w.words > nbr_cap) {
-        if (!only_long && lane == 0) atomicOr(flags, kFlagNeighbors);
-        continue;
-      }
-      RunWriter f{nbr + off, lane == 0};
-      walk(std::true_type{}, f);
-      if (lane == 0) {
-        noff[s] = off;
-        nwords[s] = static_cast<int>(w.words);
-        ncount[s] = w.count;
-      }
-    }
-  }
 }
 
 // ------------------------------------------------------------ dense walk
@@ -911,6 +870,113 @@ __device__ __forceinline__ int dense_ranges(const GatherView& gv, Ranges& R, int
   const int total = pack_ranges<kWave>(R, ra, rb);
   wave_sync();
   return __builtin_amdgcn_readfirstlane(total);
+}
+
+// ------------------------------------------------------------ lists of dense units
+
+// Builds the list of slot s, at me, in w: the runs of the 27 cells (entries of R)
+// 64 at a time; a run's slots are neighbors together.
+template <bool kFill>
+__device__ __forceinline__ void list_walk(const StepConsts& c, const GatherView& gv,
+                                          const Ranges& R, int total, int s, const float3& me,
+                                          RunWriter& w) {
+  walk_runs(gv, R, total, [](int t) { return t; },
+            [&](int, int, int k, const float3& p, int t) {
+              const int to = t + k;
+              unsigned long long m = __ballot(k > 0 && near0(me, p, c));
+              // entries whose slots follow the entry's before (lane 0's comes with w)
+              const unsigned long long follow = __ballot(t == __shfl_up(to, 1)) & ~1ull;
+              while (m != 0ull) {
+                const int j = __builtin_ctzll(m);
+                const int len = 1 + __builtin_ctzll(~((m & follow) >> j >> 1));
+                const int t0 = __builtin_amdgcn_readlane(t, j);
+                const int t1 = __builtin_amdgcn_readlane(to, j + len - 1);
+                if (t0 <= s && s < t1) {  // every slot but s itself
+                  w.template add_range<kFill>(t0, s);
+                  w.template add_range<kFill>(s + 1, t1);
+                } else {
+                  w.template add_range<kFill>(t0, t1);
+                }
+                m = (j + len >= kWave) ? 0ull : (m & (~0ull << (j + len)));
+              }
+            });
+  w.template flush<kFill>();
+}
+
+// Counts, allocates (one atomic) and fills the list of slot s of scene sc, by a
+// whole wavefront; false when it does not fit.
+__device__ __forceinline__ bool store_list(const StepConsts& c, const GatherView& gv, Ranges& R,
+                                           int s, int sc, long long* __restrict__ noff,
+                                           int* __restrict__ nwords, int* __restrict__ ncount,
+                                           int* __restrict__ nbr, long long nbr_cap,
+                                           unsigned long long* __restrict__ nbr_total) {
+  const int lane = lane_id();
+  wave_sync();  // R is reused
+  const int total = dense_ranges(gv, R, s, sc);
+  const float3 me = ld3(gv.p0, s);
+  RunWriter w{nullptr, false};
+  list_walk<false>(c, gv, R, total, s, me, w);
+  unsigned long long at = 0;
+  if (lane == 0) at = atomicAdd(nbr_total, static_cast<unsigned long long>(w.words));
+  const long long off = static_cast<long long>(__shfl(at, 0));
+  if (off + w.words > nbr_cap) return false;
+  RunWriter f{nbr + off, lane == 0};
+  list_walk<true>(c, gv, R, total, s, me, f);
+  if (lane == 0) {
+    noff[s] = off;
+    nwords[s] = static_cast<int>(w.words);
+    ncount[s] = w.count;
+  }
+  return true;
+}
+
+// On request: the lists of the heads too long for a row.  No flag is raised when
+// they do not fit (*nbr_total says what they need).
+__global__ __launch_bounds__(kBlock) void k_long_lists(
+    StepConsts c, GatherView gv, long long* __restrict__ noff, int* __restrict__ nwords,
+    int* __restrict__ ncount, int* __restrict__ nbr, long long nbr_cap,
+    unsigned long long* __restrict__ nbr_total, const unsigned* __restrict__ flags) {
+  __shared__ Ranges rng[kWaves];
+  if (fatal(flags)) return;
+  const int D = gv.info[2];
+  const int nw = static_cast<int>(gridDim.x) * kWaves;
+  for (int u = blockIdx.x * kWaves + threadIdx.x / kWave; u < D; u += nw) {
+    const DenseUnit d = dense_unit(gv, u, gv.info[3]);
+    if (d.single)
+      (void)store_list(c, gv, rng[threadIdx.x / kWave], d.s, d.sc, noff, nwords, ncount, nbr,
+                       nbr_cap, nbr_total);
+  }
+}
+
+// After the list heads' lists are stored: the lists of all other slots (nwords <
+// 0), those of dense units and of runs.  Wavefront w of W takes slots w, w + W,
+// ...: the slots of a pile, whose lists are the longest, lie side by side.
+// (velB.w: scenes.)  Bound by the loads and serial bits of two walks per list.
+// With one wavefront per unit, walking slots instead of runs, and every slot a
+// head, the recorded substep of the million-particle block after 100 substeps took
+// 377 ms, and takes 10 (diagnostics 442 and 11); after 40 substeps of the
+// 32,768-particle dam break this kernel 137 us, and takes 124.
+__global__ __launch_bounds__(kBlock) void k_dense_lists(
+    StepConsts c, GatherView gv, const float4* __restrict__ velB, long long* __restrict__ noff,
+    int* __restrict__ nwords, int* __restrict__ ncount, int* __restrict__ nbr, long long nbr_cap,
+    unsigned long long* __restrict__ nbr_total, unsigned* __restrict__ flags) {
+  __shared__ Ranges rng[kWaves];
+  if (fatal(flags) || (gv.info[2] == 0 && gv.info[0] == c.n)) return;
+  const int lane = lane_id();
+  const long long W = static_cast<long long>(gridDim.x) * kWaves;
+  for (long long s0 = blockIdx.x * kWaves + threadIdx.x / kWave; s0 < c.n; s0 += kWave * W) {
+    const long long mine = s0 + lane * W;
+    unsigned long long todo = __ballot(mine < c.n && nwords[mine < c.n ? mine : 0] < 0);
+    while (todo != 0ull) {
+      const int s = __builtin_amdgcn_readfirstlane(
+          static_cast<int>(s0 + __builtin_ctzll(todo) * W));
+      todo &= todo - 1ull;
+      const int sc = __builtin_amdgcn_readfirstlane(__float_as_int(velB[s].w));
+      const bool fits = store_list(c, gv, rng[threadIdx.x / kWave], s, sc, noff, nwords, ncount,
+                                   nbr, nbr_cap, nbr_total);
+      if (!fits && lane == 0) atomicOr(flags, kFlagNeighbors);
+    }
+  }
 }
 
 // Neighbor counts of the dense units' heads (statistics).  Nothing is counted
@@ -1661,10 +1727,9 @@ hipError_t enqueue_neighbors(Ctx& c, const StepConsts& k, const GatherView& gv) 
   if (!k.full_lists) return hipGetLastError();
   if (k.full_lists == 2)
     k_store_rows<<<std::min(kDenseGrid, blocks_for(c.n, 32)), kBlock, 0, c.stream>>>(
-        k, gv, c.noff, c.nwords, c.nbr, c.nbr_cap, c.nbr_total, c.flags);
-  k_long_lists<<<std::min(kDenseGrid, blocks_for(c.n, kWaves)), kBlock, 0, c.stream>>>(
-      k, gv, 0, c.noff, c.nwords, c.ncount, c.nbr, c.nbr_cap, c.nbr_total,
-      c.flags);
+        k, gv, c.noff, c.nwords, c.ncount, c.nbr, c.nbr_cap, c.nbr_total, c.flags);
+  k_dense_lists<<<std::min(kDenseGrid, blocks_for(c.n, kWaves)), kBlock, 0, c.stream>>>(
+      k, gv, c.velB, c.noff, c.nwords, c.ncount, c.nbr, c.nbr_cap, c.nbr_total, c.flags);
   return hipGetLastError();
 }
 
@@ -1672,8 +1737,8 @@ hipError_t enqueue_long_lists(Ctx& c, const StepConsts& k) {
   if (c.n == 0) return hipSuccess;
   k_reset_total<<<1, 64, 0, c.stream>>>(c.nbr_total);
   k_long_lists<<<std::min(kDenseGrid, blocks_for(c.n, kWaves)), kBlock, 0, c.stream>>>(
-      k, gather_view(c, c.pred[0]), 1, c.noff, c.nwords, c.ncount,
-      c.nbr, c.nbr_cap, c.nbr_total, c.flags);
+      k, gather_view(c, c.pred[0]), c.noff, c.nwords, c.ncount, c.nbr, c.nbr_cap, c.nbr_total,
+      c.flags);
   return hipGetLastError();
 }
 

@@ -978,10 +978,7 @@ hipError_t enqueue_substep(Ctx& c, const SubstepRec* rec) {
   Launcher L{c};
   StepConsts k = c.consts;
   // a recorded substep keeps every particle's own list (the adjoint reads them)
-  if (rec) {
-    k.runs = 0;
-    k.full_lists = 2;
-  }
+  if (rec) k.full_lists = 2;
   // sparse bricks through the LDS-tiled passes: their slots are no heads of
   // the other passes
   const bool tiles = k.tiles != 0 && c.tile_list != nullptr;

@@ -267,14 +267,14 @@ int hipLaunchKernel(const void* host, dim3_t grid, dim3_t block, void** args, si
     for (int i = 0; i < n; ++i) ((int*)ptr(args, 7))[i] = fake_nwords;
     need_list(args, 9, "k_neighbors without a list buffer");
   } else if (strstr(name, "k_store_rows")) {
-    need_list(args, 4, "k_store_rows without a list buffer");
+    need_list(args, 5, "k_store_rows without a list buffer");
+  } else if (strstr(name, "k_dense_lists")) {
+    need_list(args, 6, "k_dense_lists without a list buffer");
   } else if (strstr(name, "k_long_lists")) {
     ++fake_long_lists;
-    need_list(args, 6, "k_long_lists without a list buffer");
-    if (*(int*)args[2]) {  // on request: some lists are stored before one does not fit
-      ((int*)ptr(args, 4))[0] = 1;
-      *(unsigned long long*)ptr(args, 8) = fake_total;
-    }
+    need_list(args, 5, "k_long_lists without a list buffer");
+    ((int*)ptr(args, 3))[0] = 1;  // some lists are stored before one does not fit
+    *(unsigned long long*)ptr(args, 7) = fake_total;
   } else if (strstr(name, "k_tape_copy")) {
     need(args, 7, "k_tape_copy without a list buffer");
     need(args, 9, "k_tape_copy without a tape");
