@@ -454,16 +454,19 @@ void carve_arrays(Ctx& c, Carver& a, bool omega) {
   a.take(c.dense, n);
   a.take(c.info, 5);
   a.take(c.grid, ns);
-  a.take(c.total_cells, 1);
   a.take(c.scan_partial, 3 * static_cast<size_t>(c.scan_blocks) + 2);
-  a.take(c.nbr_total, 1);
   a.take(c.need_cells, 1);
-  a.take(c.pair_total, 1);
   a.take(c.seg, ns + 1);
   a.take(c.planes, ns);
   a.take(c.flags, 1);
   a.take(c.steps_started, 1);
-  a.take(c.last, 1);
+  a.take(c.query, 1);
+  if (c.query) {
+    c.last = &c.query->last;
+    c.pair_total = &c.query->pair_total;
+    c.nbr_total = &c.query->nbr_total;
+    c.total_cells = &c.query->total_cells;
+  }
   // brick tiles: beyond this capacity bricks take the other passes
   c.tile_cap = static_cast<long long>(n / 32 + 256);
   a.take(c.in_tile, n);
@@ -624,20 +627,18 @@ int read_status(Ctx& c, DevStatus& st) {
 
 // The constants of the last good substep and, in its slot order, the particles'
 // ids.  (posA has the ids in that order too, but not after a restored state.)
-int read_last(Ctx& c, fluidhip::StepConsts& k, std::vector<int>* ids) {
+int read_last(Ctx& c, fluidhip::StepConsts& k, std::vector<int>& ids) {
   const size_t n = static_cast<size_t>(c.n);
-  std::vector<float4> pos(ids ? n : 0);
+  std::vector<float4> pos(n);
   HIP_TRY(hipMemcpyAsync(&k, c.last, sizeof(k), hipMemcpyDeviceToHost, c.stream),
           "read constants");
-  if (!pos.empty())
+  if (n > 0)
     HIP_TRY(hipMemcpyAsync(pos.data(), c.posB, sizeof(float4) * n, hipMemcpyDeviceToHost,
                            c.stream),
             "read ids");
   HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
-  if (ids) {
-    ids->resize(n);
-    for (size_t s = 0; s < n; ++s) std::memcpy(&(*ids)[s], &pos[s].w, sizeof(int));
-  }
+  ids.resize(n);
+  for (size_t s = 0; s < n; ++s) std::memcpy(&ids[s], &pos[s].w, sizeof(int));
   return FLUID_HIP_OK;
 }
 
@@ -1317,7 +1318,10 @@ int fluid_hip_get_diag(fluid_hip_ctx* ctx, int32_t* cell, int32_t* sorted_ids,
   const size_t n = static_cast<size_t>(c.n);
   fluidhip::StepConsts last{};
   std::vector<int> ids;
-  if ((rc = read_last(c, last, &ids))) return rc;
+  // dense heads and the other slots of runs may have kept no count: a counting
+  // walk of the last grid writes every slot's
+  if (nbr_count) HIP_TRY(fluidhip::enqueue_count_pairs(c), "count pairs");
+  if ((rc = read_last(c, last, ids))) return rc;
   if (sorted_ids) std::copy(ids.begin(), ids.end(), sorted_ids);
   if (cell) {
     std::vector<uint64_t> dc(n);
@@ -1332,12 +1336,6 @@ int fluid_hip_get_diag(fluid_hip_ctx* ctx, int32_t* cell, int32_t* sorted_ids,
     }
   }
   if (nbr_count) {
-    if (!last.full_lists) {
-      // dense heads and the other slots of runs kept no count: a counting
-      // walk of the last grid writes every slot's
-      HIP_TRY(fluidhip::enqueue_count_pairs(c, last), "count pairs");
-      HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
-    }
     std::vector<int> nc(n);
     HIP_TRY(hipMemcpy(nc.data(), c.ncount, sizeof(int) * n, hipMemcpyDeviceToHost), "read counts");
     for (size_t s = 0; s < n; ++s) nbr_count[ids[s]] = nc[s];
@@ -1371,7 +1369,7 @@ int fluid_hip_get_neighbors(fluid_hip_ctx* ctx, int32_t* out, int64_t cap, int64
   std::vector<int> nw(n);
   fluidhip::StepConsts last{};
   std::vector<int> ids;
-  if ((rc = read_last(c, last, &ids))) return rc;
+  if ((rc = read_last(c, last, ids))) return rc;
   HIP_TRY(hipMemcpy(nw.data(), c.nwords, sizeof(int) * n, hipMemcpyDeviceToHost), "read lengths");
   // particles of LDS tiles keep LDS records of the tile's halo: decode them
   // with its layout; list heads keep slots in their row, and a step that
@@ -1533,29 +1531,23 @@ int fluid_hip_get_stats(fluid_hip_ctx* ctx, int64_t* out, int32_t n) {
   int64_t v[10] = {0, 0, 0, c.nbr_cap, c.cell_cap, c.grow_events, tape_bytes(c),
                    c.adj ? c.adj->recomputed : 0, 0, 0};
   if (c.stepped && c.n > 0) {
-    fluidhip::StepConsts last{};
-    if ((rc = read_last(c, last, nullptr))) return rc;
+    // dense heads may have stored no list: their pairs are counted again
+    HIP_TRY(fluidhip::enqueue_count_pairs(c), "count pairs");
+    fluidhip::QueryWords q{};
+    HIP_TRY(hipMemcpyAsync(&q, c.query, sizeof(q), hipMemcpyDeviceToHost, c.stream),
+            "read statistics");
+    HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+    const fluidhip::StepConsts& last = q.last;
     if (!last.full_lists) {
-      // dense heads stored no list: count their pairs again
-      HIP_TRY(fluidhip::enqueue_count_pairs(c, last), "count pairs");
-      unsigned long long pairs = 0;
-      HIP_TRY(hipMemcpyAsync(&pairs, c.pair_total, sizeof(pairs), hipMemcpyDeviceToHost,
-                             c.stream),
-              "read pairs");
-      HIP_TRY(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
-      v[0] = static_cast<int64_t>(pairs);
+      v[0] = static_cast<int64_t>(q.pair_total);
     } else {
       std::vector<int> cnt(c.n);
       HIP_TRY(hipMemcpy(cnt.data(), c.ncount, sizeof(int) * c.n, hipMemcpyDeviceToHost),
               "read counts");
       for (int x : cnt) v[0] += x;
     }
-    unsigned long long words = 0;
-    HIP_TRY(hipMemcpy(&words, c.nbr_total, sizeof(words), hipMemcpyDeviceToHost), "read words");
-    v[1] = static_cast<int64_t>(words);
-    int cells = 0;
-    HIP_TRY(hipMemcpy(&cells, c.total_cells, sizeof(int), hipMemcpyDeviceToHost), "read cells");
-    v[2] = cells;
+    v[1] = static_cast<int64_t>(q.nbr_total);
+    v[2] = q.total_cells;
     if (last.tiles && !last.full_lists) {
       int tiles = 0;
       HIP_TRY(hipMemcpy(&tiles, c.tile_count, sizeof(int), hipMemcpyDeviceToHost), "read tiles");

@@ -90,6 +90,14 @@ struct Prof {
   std::unordered_map<std::string, std::pair<double, long long>> acc;
 };
 
+// Device words that statistics read, side by side for one copy.
+struct QueryWords {
+  StepConsts last;                // constants of the last good substep
+  unsigned long long pair_total;  // neighbor pairs, counted on request
+  unsigned long long nbr_total;   // words of the stored lists
+  int total_cells;                // of the cell table
+};
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -150,7 +158,6 @@ struct Ctx {
   int* bbox = nullptr;   // n_scenes * 6
   int* tile_bbox = nullptr;  // 6 per particle tile (workgroup)
   GridDesc* grid = nullptr;
-  int* total_cells = nullptr;
   int* scan_partial = nullptr;  // 3 scan_blocks + 2: range sums of up to three scanned arrays
   uint64_t* slot_cell = nullptr;  // packed cell of pred0 per sorted slot
   int* slot_key = nullptr;  // table key of each sorted slot's cell
@@ -180,19 +187,20 @@ struct Ctx {
   int* ncount = nullptr;      // neighbors (decoded length)
   int* nbr = nullptr;         // run-length-encoded lists, nbr_cap words
   long long nbr_cap = 0;
-  unsigned long long* nbr_total = nullptr;
   unsigned long long* need_cells = nullptr;  // cells a failed substep needed
-  unsigned long long* pair_total = nullptr;  // neighbor pairs, counted on request
 
   // scenes
   int* seg = nullptr;
   ScenePlanes* planes = nullptr;
 
-  // The constants of the last good substep, written with its grid: what queries
-  // of its slots and lists go by, whatever parameters or launch knobs the
-  // context has now, whether it was recorded, and whether a graph replayed it.
-  // Its ids are in posB.
-  StepConsts* last = nullptr;
+  // `last` is written with a substep's grid: what queries of its slots and lists
+  // go by, whatever parameters or launch knobs the context has now, whether the
+  // substep was recorded, and whether a graph replayed it.  Its ids are in posB.
+  QueryWords* query = nullptr;
+  StepConsts* last = nullptr;  // parts of *query
+  unsigned long long* pair_total = nullptr;
+  unsigned long long* nbr_total = nullptr;
+  int* total_cells = nullptr;
 
   // status
   unsigned* flags = nullptr;
@@ -319,10 +327,10 @@ hipError_t enqueue_xsph(Ctx& c, const StepConsts& k, const GatherView& gv, bool 
                         unsigned* rm);
 hipError_t enqueue_vort_omega(Ctx& c, const StepConsts& k, const GatherView& gv);
 hipError_t enqueue_vort_apply(Ctx& c, const StepConsts& k, const GatherView& gv, bool rest);
-// After a substep with constants k that stored no words: counts every particle's
+// After a substep that did not store every list: counts every particle's
 // neighbors into c.ncount and their sum into c.pair_total.
-hipError_t enqueue_count_pairs(Ctx& c, const StepConsts& k);
-// ... or stores the lists too long for a row (nwords kLongList) in c.nbr;
+hipError_t enqueue_count_pairs(Ctx& c);
+// ... or, its constants being k, stores the lists too long for a row (nwords kLongList) in c.nbr;
 // *c.nbr_total is what they need, and a list that does not fit is left out.
 hipError_t enqueue_long_lists(Ctx& c, const StepConsts& k);
 

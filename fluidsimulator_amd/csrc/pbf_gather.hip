@@ -981,11 +981,13 @@ __global__ __launch_bounds__(kBlock) void k_dense_lists(
 
 // Neighbor counts of the dense units' heads (statistics).  Nothing is counted
 // after a substep that failed, whose arrays are of two substeps.
-__global__ __launch_bounds__(kBlock) void k_count_dense(StepConsts c, GatherView gv,
+__global__ __launch_bounds__(kBlock) void k_count_dense(const StepConsts* __restrict__ last,
+                                                        GatherView gv,
                                                         int* __restrict__ ncount,
                                                         const unsigned* __restrict__ flags) {
   __shared__ Ranges rng[kWaves];
-  if (fatal(flags)) return;
+  if (fatal(flags) || last->full_lists) return;
+  const StepConsts c = *last;
   const int D = gv.info[2];
   Ranges& R = rng[threadIdx.x / kWave];
   const int nw = static_cast<int>(gridDim.x) * kWaves;
@@ -1008,15 +1010,18 @@ __global__ __launch_bounds__(kBlock) void k_count_dense(StepConsts c, GatherView
 }
 
 // Every slot's count from its run's head (from the tile lists for tile
-// slots), and the sum of all (0 after a substep that failed).
+// slots), and the sum of all (0 after a substep that failed, or that stored every
+// list and with it every count).
 __global__ __launch_bounds__(kBlock) void k_count_slots(int n, const int* __restrict__ run_no,
                                                         const int* __restrict__ rep,
+                                                        const StepConsts* __restrict__ last,
                                                         const int* __restrict__ in_tile,
                                                         const int* __restrict__ tile_cnt,
                                                         int* __restrict__ ncount,
                                                         unsigned long long* __restrict__ total,
                                                         const unsigned* __restrict__ flags) {
-  if (fatal(flags)) return;
+  if (fatal(flags) || last->full_lists) return;
+  if (!last->tiles) in_tile = nullptr;
   unsigned long long v = 0ull;
   const int stride = static_cast<int>(gridDim.x) * kBlock;
   for (int s = blockIdx.x * kBlock + threadIdx.x; s < n; s += stride) {
@@ -1742,13 +1747,13 @@ hipError_t enqueue_long_lists(Ctx& c, const StepConsts& k) {
   return hipGetLastError();
 }
 
-hipError_t enqueue_count_pairs(Ctx& c, const StepConsts& k) {
+hipError_t enqueue_count_pairs(Ctx& c) {
   k_reset_total<<<1, 64, 0, c.stream>>>(c.pair_total);
   if (c.n == 0) return hipGetLastError();
   k_count_dense<<<std::min(kDenseGrid, blocks_for(c.n, kWaves)), kBlock, 0, c.stream>>>(
-      k, gather_view(c, c.pred[0]), c.ncount, c.flags);
+      c.last, gather_view(c, c.pred[0]), c.ncount, c.flags);
   k_count_slots<<<std::min(1024, blocks_for(c.n, kBlock)), kBlock, 0, c.stream>>>(
-      c.n, c.run_no, c.rep_list, k.tiles ? c.in_tile : nullptr, c.tile_cnt, c.ncount,
+      c.n, c.run_no, c.rep_list, c.last, c.in_tile, c.tile_cnt, c.ncount,
       c.pair_total, c.flags);
   return hipGetLastError();
 }
