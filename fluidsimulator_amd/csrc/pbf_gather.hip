@@ -724,6 +724,7 @@ __global__ __launch_bounds__(kBlock) void k_store_rows(
     unsigned long long* __restrict__ nbr_total, unsigned* __restrict__ flags) {
   constexpr int kLanes = 8, kUnits = kBlock / kLanes;
   __shared__ long long wsum[kWaves];
+  __shared__ int round[kWaves];
   __shared__ long long base_sh;
   __shared__ int abort_sh;
   if (threadIdx.x == 0) abort_sh = fatal(flags) ? 1 : 0;
@@ -758,23 +759,31 @@ __global__ __launch_bounds__(kBlock) void k_store_rows(
     const int u = b + g;
     const int4 unit = u < u1 ? gv.units[u] : make_int4(0, -1, 0, 0);
     const int s = unit.x, cnt = max(unit.y, 0), len = unit.z;
-    const long long mine = static_cast<long long>(cnt) * len;
+    const int mine = cnt * len;  // (a row's entries times a sparse cell's slots)
     // the lists before this unit's: within the wavefront (its groups' first
     // lanes), then the wavefronts before
-    long long inc = mine;
+    int inc = mine;
     for (int o = kLanes; o < kWave; o <<= 1) {
-      const long long v = __shfl_up(inc, o);
+      const int v = __shfl_up(inc, o);
       if (lane_id() >= o) inc += v;
     }
-    __syncthreads();  // wsum is reused
-    if (lane_id() == kWave - 1) wsum[threadIdx.x / kWave] = inc;
+    __syncthreads();  // round is reused
+    if (lane_id() == kWave - 1) round[threadIdx.x / kWave] = inc;
     __syncthreads();
     long long off = at + inc - mine;
     for (int w = 0; w < kWaves; ++w) {
-      off += w < static_cast<int>(threadIdx.x) / kWave ? wsum[w] : 0;
-      at += wsum[w];
+      off += w < static_cast<int>(threadIdx.x) / kWave ? round[w] : 0;
+      at += round[w];
     }
     auto row = [&](int k) { return rows[(static_cast<size_t>(k >> 2) * c.n + s) * 4 + (k & 3)]; };
+    if (!__any(len > 1)) {  // no run among the wavefront's heads
+      for (int k = q; k < cnt; k += kLanes) nbr[off + k] = row(k);
+      if (q == 0 && unit.y >= 0) {
+        noff[s] = off;
+        nwords[s] = cnt;
+      }
+      continue;
+    }
     // the run's other slots: entries [own, own + len - 1) of the row
     int own = cnt;
     if (len > 1)
@@ -784,12 +793,11 @@ __global__ __launch_bounds__(kBlock) void k_store_rows(
     for (int k = q; k < cnt; k += kLanes) {
       const int v = row(k), i = k - own;
       const bool in_run = i >= 0 && i < len - 1;
-      for (int j = 0; j < len; ++j)
-        nbr[off + static_cast<long long>(j) * cnt + k] = in_run ? s + i + (i >= j ? 1 : 0) : v;
+      for (int j = 0; j < len; ++j) nbr[off + j * cnt + k] = in_run ? s + i + (i >= j ? 1 : 0) : v;
     }
     if (unit.y >= 0)
       for (int j = q; j < len; j += kLanes) {
-        noff[s + j] = off + static_cast<long long>(j) * cnt;
+        noff[s + j] = off + j * cnt;
         nwords[s + j] = cnt;
         ncount[s + j] = cnt;
       }
