@@ -170,9 +170,9 @@ ROCPROF_NAME = {"predict_bbox": "k_predict_bbox", "lambda": "k_lambda", "delta":
 
 def window_bounds(pos: list, take: int) -> tuple:
     """Bounds of the timed window on the ascending dispatch positions (start
-    times or dispatch ids) of a per-lane pass kernel: halfway to its launch
+    times or dispatch ids) of a head pass kernel: halfway to its launch
     before the window and halfway past its last.  The pass's tile kernel is
-    launched next to each per-lane launch, so exactly its launches of the
+    launched next to each head launch, so exactly its launches of the
     window fall inside; those of another context (the early-regime record)
     or of the warm-up fall outside."""
     w = pos[-take:]
@@ -246,7 +246,7 @@ def summarize_traffic(outdir: str, json_path: str | None = None, steps: int | No
     km = per_dispatch("pmc_l2", "TCC_MISS_sum", required=False)
 
     def window(d, key, per_step):
-        """Per-launch values of pass `key` over the timed window: the per-lane
+        """Per-launch values of pass `key` over the timed window: the head
         kernel and, when the window's launches have one, its LDS-tile kernel,
         summed launch by launch."""
         if d is None:
@@ -260,7 +260,7 @@ def summarize_traffic(outdir: str, json_path: str | None = None, steps: int | No
         if tile:
             if len(tile) != len(out):
                 raise SystemExit(f"{key}: {len(tile)} tile launches against {len(out)} "
-                                 "per-lane launches in the timed window")
+                                 "head launches in the timed window")
             out = [a + v for a, (_, v) in zip(out, tile)]
         return out
 
@@ -327,9 +327,9 @@ def summarize_rocprof(outdir: str, steps: int, launches_per_step: dict,
               "(dispatches that returned at once, under 1% of the kernel's median, are",
               "left out: after a capacity overflow the substeps queued behind the failed",
               "one do no work, and the failed one runs again):"]
-    # a tile kernel counts only inside its per-lane pass kernel's window (the
+    # a tile kernel counts only inside its head pass kernel's window (the
     # tile lists and classification inside predict_bbox's, one per substep);
-    # per-lane keys come first
+    # head keys come first
     bounds = {}
     for key, per_step in launches_per_step.items():
         rows = cur.execute("select start, duration from kernels where name like ? order by start",
@@ -384,8 +384,8 @@ def bench_ensemble(args) -> dict:
     vel = np.concatenate([st.vel for st in ens.states], axis=1)
 
     # the ensemble's default is tiles off: its scenes turn to sparse spray and
-    # wall piles within a few substeps, where the per-lane passes are faster
-    # (240 substeps: 5.50 ms per substep batched, against 6.07 with tiles)
+    # wall piles within a few substeps, where the passes over heads are faster
+    # (240 substeps: 3.40 ms per substep batched, against 4.26 with tiles)
     tiles = "off" if args.tiles == "default" else args.tiles
     tg = {"auto": 0, "on": 1, "off": 2}[tiles]
 
