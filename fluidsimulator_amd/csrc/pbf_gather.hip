@@ -717,7 +717,7 @@ __global__ __launch_bounds__(kBlock) void k_neighbors(
 // it): a workgroup takes consecutive units, whose lists it
 // allocates with one atomic (atomics on one address take about 10 ns each: one
 // for every 8 heads made the neighbor kernel take 107 us at 65,536 particles;
-// without them it takes 27, and this one 21).
+// without them it takes 27, and this one 24).
 __global__ __launch_bounds__(kBlock) void k_store_rows(
     StepConsts c, GatherView gv, long long* __restrict__ noff, int* __restrict__ nwords,
     int* __restrict__ ncount, int* __restrict__ nbr, long long nbr_cap,
